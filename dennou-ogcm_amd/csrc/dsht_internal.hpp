@@ -248,6 +248,12 @@ int reg_fft_inv(const GT* G, const FftArgs& a, XT* xy, hipStream_t s);
 // legendre_f64d.hip: FP64 contractions as per-wave fragment streams (DSHT_TUNE_LEG = 2)
 int launch_leg_inv_direct(const dsht_plan* p, int op, const LegInvArgs& a, hipStream_t s);
 int launch_leg_fwd_direct(const dsht_plan* p, int op, const LegFwdArgs& a, hipStream_t s);
+// legendre_f64w.hip: FP64 contractions with the whole K extent in LDS (the default where a
+// block's data fit: *_ok)
+bool leg_inv_staged_ok(const dsht_plan* p, int op);
+bool leg_fwd_staged_ok(const dsht_plan* p, int op);
+int launch_leg_inv_staged(const dsht_plan* p, int op, const LegInvArgs& a, hipStream_t s);
+int launch_leg_fwd_staged(const dsht_plan* p, int op, const LegFwdArgs& a, hipStream_t s);
 int launch_fft_fwd32(const dsht_plan* p, const double* xy, long ldg, int ncols, float2* G, long gld,
                      unsigned* colmax, hipStream_t s);
 int launch_fft_inv32(const dsht_plan* p, const float2* G, long gld, int ncols, double* xy, long ldg,

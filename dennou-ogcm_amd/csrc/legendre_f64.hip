@@ -578,6 +578,7 @@ int launch_leg_fwd(const dsht_plan* p, int op, const LegFwdArgs& a, hipStream_t 
   ProfScope ps("leg_fwd", s, by, fl);
   // forward: the per-wave fragment-stream kernel by default (measured 165 against 174 us at
   // T170 x 360); DSHT_TUNE_LEG = 1 or 3 selects the LDS-staged kernel
+  if (p->leg_kind == 0 && leg_fwd_staged_ok(p, op)) return launch_leg_fwd_staged(p, op, a, s);
   if (p->leg_kind == 0 || p->leg_kind == 2) return launch_leg_fwd_direct(p, op, a, s);
   switch (op) {
     case F_VAL: return wide ? fwd_pick<F_VAL, 32>(p, a, s) : fwd_pick<F_VAL, 16>(p, a, s);
@@ -603,6 +604,7 @@ int launch_leg_inv(const dsht_plan* p, int op, const LegInvArgs& a, hipStream_t 
   leg_work(p, nin[op], nw, nt[op], ntab[op], false, a.ncols, &by, &fl);
   ProfScope ps("leg_inv", s, by, fl);
   if (p->leg_kind == 2) return launch_leg_inv_direct(p, op, a, s);
+  if (p->leg_kind == 0 && leg_inv_staged_ok(p, op)) return launch_leg_inv_staged(p, op, a, s);
   switch (op) {
     case I_VAL: return wide ? inv_pick<I_VAL, 32>(p, a, s) : inv_pick<I_VAL, 16>(p, a, s);
     case I_GRADLAMBDA: return wide ? inv_pick<I_GRADLAMBDA, 32>(p, a, s) : inv_pick<I_GRADLAMBDA, 16>(p, a, s);
