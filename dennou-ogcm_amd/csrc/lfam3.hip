@@ -75,68 +75,129 @@ __global__ void k_lf_fill(double* __restrict__ x, double v, long n) {
   LF_LOOP(n) x[g] = v;
 }
 
-// EOS_Linear_Eval(theta, S, p = -RefDens GeoPot) for every layer of every run
+// Column walks: one thread per grid point of a run (grid y) goes through the layers, LG of them
+// per round with their loads issued together.  The layers' running sums (pressure from the
+// top, omega from the bottom) stay in registers, so a field that is only a step between two
+// others (omega, the vertical fluxes) is never written.  Bound by HBM: every layer field in
+// and out is touched once.
+constexpr int LG = 4;
+
+__device__ __forceinline__ double lf_ld(const double* x) { return __builtin_nontemporal_load(x); }
+
+inline dim3 lf_gridc(long npts, int nr, int threads) { return dim3((unsigned)((npts + threads - 1) / threads), (unsigned)nr); }
+// small grids take small blocks, so that the columns spread over the chip
+inline int lf_threads(long npts, int nr) { return npts * nr >= 65536 ? 256 : 64; }
+
+// EOS_Linear_Eval(theta, S, p = -RefDens GeoPot) and the hydrostatic pressure of its density
+// (HBEDiagnose_HydPres, HBEDiagnose_hspm_vfvm_mod.f90:315-321) for every layer of every run
 struct EosArgs {
   double ref_dens, ptemp_dep, press_dep, salt_dep, ref_temp, ref_salt, depth, grav;
 };
-__global__ void k_lf_eos(const double* __restrict__ ts, long npts, int K, const double* __restrict__ zck, EosArgs e,
-                         long ncols, double* __restrict__ dens) {
-  LF_CP(ncols, npts) {
-    const long g = c * npts + p;
-    const int k = (int)(c % K);
-    const long r = c / K;
-    const double t = ts[((2 * r) * K + k) * npts + p];
-    const double s = ts[((2 * r + 1) * K + k) * npts + p];
-    const double geo = e.grav * (e.depth * zck[k]);
-    const double pr = -e.ref_dens * geo;
-    dens[g] = e.ref_dens * (e.ptemp_dep * (t - e.ref_temp) + e.press_dep * pr + e.salt_dep * (s - e.ref_salt));
+__global__ __launch_bounds__(256) void k_lf_eos_hyd(const double* __restrict__ ts, long npts, int K,
+                                                    const double* __restrict__ zck, const double* __restrict__ cdk,
+                                                    EosArgs e, double* __restrict__ dens, double* __restrict__ hyd) {
+#pragma clang fp contract(off)
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= npts) return;
+  const long r = blockIdx.y;
+  const double* tp = ts + 2 * r * K * npts + p;
+  const double* sp = tp + (long)K * npts;
+  const long o = r * K * npts + p;
+  const double gh = e.grav * e.depth;
+  double sum = 0.0;
+  for (int k0 = 0; k0 < K; k0 += 2 * LG) {
+    double t[2 * LG], s[2 * LG];
+#pragma unroll
+    for (int u = 0; u < 2 * LG; u++) {
+      const long k = k0 + u < K ? k0 + u : K - 1;
+      t[u] = lf_ld(tp + k * npts);
+      s[u] = lf_ld(sp + k * npts);
+    }
+#pragma unroll
+    for (int u = 0; u < 2 * LG; u++) {
+      const int k = k0 + u;
+      if (k >= K) break;
+      const double geo = e.grav * (e.depth * zck[k]);
+      const double pr = -e.ref_dens * geo;
+      const double d = e.ref_dens *
+                       (e.ptemp_dep * (t[u] - e.ref_temp) + e.press_dep * pr + e.salt_dep * (s[u] - e.ref_salt));
+      const double next = sum + (gh * d) * cdk[k];
+      dens[o + k * npts] = d;
+      hyd[o + k * npts] = 0.5 * (sum + next);
+      sum = next;
+    }
   }
 }
 
 // The grid-space part of HBEBaroc_MOMRHS_VorDivForm (HBEBaroc_hspm_vfvm_mod.f90:366-420):
-// the vertical advection of momentum at the half levels, the absolute-vorticity fluxes A
-// and B (times cos phi) and the Bernoulli function C.  Writes -A (so that one
-// calc_UVCosLat2VorDiv call with (U cos, V cos) = (B, -A) gives -H(A, B) and H(B, -A)), B
-// and C.  The Coriolis terms are f (cn x_N + cb x_B) (:474-481, 565-570).
+// omega from the divergence (HBEDiagnose_OMG, HBEDiagnose_hspm_vfvm_mod.f90:123-131), the
+// vertical advection of momentum at the half levels, the absolute-vorticity fluxes A and B
+// (times cos phi) and the Bernoulli function C, from the bottom layer up.  Writes -A (so that
+// one calc_UVCosLat2VorDiv call with (U cos, V cos) = (B, -A) gives -H(A, B) and H(B, -A)), B
+// and C.  The Coriolis terms (:474-481, 565-570): PRED f (cn x + cb xb) of the advected winds
+// and (xa, xb) of the time level before; else f times the winds (xa, xb) of the present level.
 struct MomArgs {
-  const double *u, *v, *omg, *vor, *h, *hyd, *sp, *dens, *glon, *glat, *un, *ub, *vn, *vb;
-  const double *two_omega, *mu, *cs, *rfdk;
-  double ref_dens, radius, cn, cb;
+  double ref_dens, radius, depth, cn, cb;
   long npts;
   int I, K;
-  double *am, *bg, *cg;
 };
-__global__ void k_lf_mom(MomArgs a, long ncols) {
-  LF_CP(ncols, a.npts) {
-    const long g = c * a.npts + p;
-    const int k = (int)(c % a.K);
-    const long r = c / a.K;
-    const int j = LF_ROW(p, a.I);
-    const long np = a.npts;
-    const double u = a.u[g], v = a.v[g];
-    const double* om = a.omg + r * (a.K + 1) * np + p;  // half level h at om[h*np]
-    double vau_a = 0.0, vav_a = 0.0, vau_b = 0.0, vav_b = 0.0;
-    if (k > 0) {  // half level k, between layers k-1 and k
-      vau_a = om[(long)k * np] * (a.u[g - np] - u) * a.rfdk[k];
-      vav_a = om[(long)k * np] * (a.v[g - np] - v) * a.rfdk[k];
+template <bool PRED>
+__global__ __launch_bounds__(256) void k_lf_mom(
+    MomArgs a, const double* __restrict__ u, const double* __restrict__ v, const double* __restrict__ xa,
+    const double* __restrict__ xb, const double* __restrict__ div, const double* __restrict__ vor,
+    const double* __restrict__ hyd, const double* __restrict__ dens, const double* __restrict__ glon,
+    const double* __restrict__ glat, const double* __restrict__ sp, const double* __restrict__ two_omega,
+    const double* __restrict__ mu, const double* __restrict__ cosj, const double* __restrict__ cdk,
+    const double* __restrict__ rfdk, double* __restrict__ am, double* __restrict__ bg, double* __restrict__ cg) {
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x, np = a.npts;
+  if (p >= np) return;
+  const long r = blockIdx.y, o = r * a.K * np + p;
+  const int j = LF_ROW(p, a.I);
+  const double f = two_omega[r] * mu[j], cs = cosj[j], rr = a.ref_dens * a.radius;
+  const double sfc = sp[r * np + p];
+  double om = 0.0, vau_b = 0.0, vav_b = 0.0;  // omega and vertical advection at the layer's lower half level
+  double uk = lf_ld(u + o + (a.K - 1) * np), vk = lf_ld(v + o + (a.K - 1) * np);
+  for (int k0 = a.K - 1; k0 >= 0; k0 -= LG) {
+    double un[LG], vn[LG], x[LG], y[LG], dv[LG], vo[LG], hy[LG], de[LG], gx[LG], gy[LG];
+#pragma unroll
+    for (int q = 0; q < LG; q++) {
+      const long g = o + (k0 - q > 0 ? k0 - q : 0) * np, gn = o + (k0 - q > 1 ? k0 - q - 1 : 0) * np;
+      un[q] = lf_ld(u + gn);
+      vn[q] = lf_ld(v + gn);
+      x[q] = lf_ld(xa + g);
+      y[q] = lf_ld(xb + g);
+      dv[q] = lf_ld(div + g);
+      vo[q] = lf_ld(vor + g);
+      hy[q] = lf_ld(hyd + g);
+      de[q] = lf_ld(dens + g);
+      gx[q] = lf_ld(glon + g);
+      gy[q] = lf_ld(glat + g);
     }
-    if (k < a.K - 1) {  // half level k+1, between layers k and k+1
-      vau_b = om[(long)(k + 1) * np] * (u - a.u[g + np]) * a.rfdk[k + 1];
-      vav_b = om[(long)(k + 1) * np] * (v - a.v[g + np]) * a.rfdk[k + 1];
+#pragma unroll
+    for (int q = 0; q < LG; q++) {
+      const int k = k0 - q;
+      if (k < 0) break;
+      const long g = o + k * np;
+      om = om - dv[q] * (a.depth * cdk[k]);
+      double vau_a = 0.0, vav_a = 0.0;
+      if (k > 0) {
+        vau_a = om * (un[q] - uk) * rfdk[k];
+        vav_a = om * (vn[q] - vk) * rfdk[k];
+      }
+      const double coru = PRED ? f * (a.cn * uk + a.cb * x[q]) : f * x[q];
+      const double corv = PRED ? f * (a.cn * vk + a.cb * y[q]) : f * y[q];
+      double A = vo[q] * uk + coru + 0.5 * (vav_b + vav_a) / a.depth;
+      A = cs * (A + de[q] * gy[q] / rr);
+      double B = vo[q] * vk + corv - 0.5 * (vau_b + vau_a) / a.depth;
+      B = cs * (B + de[q] * gx[q] / rr);
+      am[g] = -A;
+      bg[g] = B;
+      cg[g] = (0.5 * (uk * uk + vk * vk) + (hy[q] + sfc) / a.ref_dens) / (a.radius * a.radius);
+      vau_b = vau_a;
+      vav_b = vav_a;
+      uk = un[q];
+      vk = vn[q];
     }
-    const double f = a.two_omega[r] * a.mu[j];
-    const double coru = f * (a.cn * a.un[g] + a.cb * a.ub[g]);
-    const double corv = f * (a.cn * a.vn[g] + a.cb * a.vb[g]);
-    const double h = a.h[g], vor = a.vor[g], dens = a.dens[g], cs = a.cs[j];
-    const double rr = a.ref_dens * a.radius;
-    double A = vor * u + coru + 0.5 * (vav_b + vav_a) / h;
-    A = cs * (A + dens * a.glat[g] / rr);
-    double B = vor * v + corv - 0.5 * (vau_b + vau_a) / h;
-    B = cs * (B + dens * a.glon[g] / rr);
-    const double pres = a.hyd[g] + a.sp[r * np + p];
-    a.am[g] = -A;
-    a.bg[g] = B;
-    a.cg[g] = (0.5 * (u * u + v * v) + pres / a.ref_dens) / (a.radius * a.radius);
   }
 }
 
@@ -185,26 +246,79 @@ __global__ void k_lf_barot_shift(double* __restrict__ u, double* __restrict__ v,
   }
 }
 
-// The grid-space part of HBEBaroc_HTRCRHS (HBEBaroc_hspm_vfvm_mod.f90:162-172): the
+// The grid-space part of HBEBaroc_HTRCRHS (HBEBaroc_hspm_vfvm_mod.f90:162-172) for both tracers
+// of every run, from the bottom layer up: omega from the divergence (HBEDiagnose_OMG), the QUICK
+// flux at the half levels (calc_ADVFlxZ_QUICK, :233-317: 0 at the surface and the bottom,
+// centred at half levels 1 and K-1, else with the curvature terms D of the two layers), the
 // horizontal flux (U, V) H cos(phi) T and the vertical flux divergence
-// -(F(k-1) - F(k)) / z_CDK(k), for both tracers of every run
-__global__ void k_lf_htrc_grid(const double* __restrict__ ts, const double* __restrict__ u,
-                               const double* __restrict__ v, const double* __restrict__ h,
-                               const double* __restrict__ cs, const double* __restrict__ flx,
-                               const double* __restrict__ rcdk, long npts, int I, int K, long ncols,
-                               double* __restrict__ fu, double* __restrict__ fv, double* __restrict__ vf) {
-  LF_CP(ncols, npts) {
-    const long g = c * npts + p;
-    const int k = (int)(c % K);
-    const long rt = c / K;  // 2 r + t
-    const long r = rt / 2;
-    const long q = (r * K + k) * npts + p;
-    const int j = LF_ROW(p, I);
-    const double tmp = h[q] * cs[j] * ts[g];
-    fu[g] = u[q] * tmp;
-    fv[g] = v[q] * tmp;
-    const double* fl = flx + rt * (K + 1) * npts + p;
-    vf[g] = -(fl[(long)k * npts] - fl[(long)(k + 1) * npts]) * rcdk[k];
+// -(F(k) - F(k+1)) / z_CDK(k).  m1, m2, dfac: the interpolation weights per half level.
+__device__ __forceinline__ double lf_curvature(double ta, double tb, double tc, double ra, double rb) {
+#pragma clang fp contract(off)
+  const double x = (ta - tb) * ra;
+  const double y = (tb - tc) * rb;
+  return (x - y) * (ra + rb);
+}
+__global__ __launch_bounds__(256) void k_lf_htrc(const double* __restrict__ ts, const double* __restrict__ u,
+                                                 const double* __restrict__ v, const double* __restrict__ div,
+                                                 double depth, double h, const double* __restrict__ cosj,
+                                                 const double* __restrict__ cdk, const double* __restrict__ rcdk,
+                                                 const double* __restrict__ rfdk, const double* __restrict__ m1,
+                                                 const double* __restrict__ m2, const double* __restrict__ dfac,
+                                                 long npts, int I, int K, double* __restrict__ fu,
+                                                 double* __restrict__ fv, double* __restrict__ vf) {
+#pragma clang fp contract(off)
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= npts) return;
+  const long r = blockIdx.y, o = r * K * npts + p, ot = 2 * r * K * npts + p, sec = (long)K * npts;
+  const double hc = h * cosj[LF_ROW(p, I)];
+  auto T = [&](int tr, int k) { return lf_ld(ts + ot + tr * sec + (long)(k > 0 ? k : 0) * npts); };
+  double om = 0.0;
+  double t0[2], t1[2], fb[2] = {0.0, 0.0}, db[2] = {0.0, 0.0};  // T[k], T[k-1], F(k+1), D[k]
+#pragma unroll
+  for (int tr = 0; tr < 2; tr++) {
+    t0[tr] = T(tr, K - 1);
+    t1[tr] = T(tr, K - 2);
+  }
+  for (int k0 = K - 1; k0 >= 0; k0 -= LG) {
+    double tn[2][LG], uu[LG], vv[LG], dv[LG];
+#pragma unroll
+    for (int q = 0; q < LG; q++) {
+      const long g = o + (long)(k0 - q > 0 ? k0 - q : 0) * npts;
+      tn[0][q] = T(0, k0 - q - 2);
+      tn[1][q] = T(1, k0 - q - 2);
+      uu[q] = lf_ld(u + g);
+      vv[q] = lf_ld(v + g);
+      dv[q] = lf_ld(div + g);
+    }
+#pragma unroll
+    for (int q = 0; q < LG; q++) {
+      const int k = k0 - q;
+      if (k < 0) break;
+      const double dz = depth * cdk[k];
+      om = om - dv[q] * dz;
+#pragma unroll
+      for (int tr = 0; tr < 2; tr++) {
+        const double t2 = tn[tr][q];  // T[k-2]
+        double da = 0.0, fl = 0.0;
+        if (k > 0) {
+          const double mid = m1[k] * t1[tr] + m2[k] * t0[tr];
+          if (k >= 2) da = lf_curvature(t2, t1[tr], t0[tr], rfdk[k - 1], rfdk[k]);
+          if (k >= 2 && k <= K - 2)
+            fl = om * (mid - dfac[k] * (da + db[tr])) + (fabs(om) * dfac[k]) * (da - db[tr]);
+          else
+            fl = om * mid;
+        }
+        const double tmp = hc * t0[tr];
+        const long g = ot + tr * sec + k * npts;
+        fu[g] = uu[q] * tmp;
+        fv[g] = vv[q] * tmp;
+        vf[g] = -(fl - fb[tr]) * rcdk[k];
+        fb[tr] = fl;
+        db[tr] = da;
+        t0[tr] = t1[tr];
+        t1[tr] = t2;
+      }
+    }
   }
 }
 
@@ -321,13 +435,13 @@ __global__ void k_lf_add2(const double* __restrict__ a, const double* __restrict
 }
 
 // full velocity and the time-centred fields of the tracer update (:783-795):
-// U_A = U_A - UBarot + UBarot_A; U = (5 U_A + 8 U_N - U_B)/12; H likewise
+// U_A = U_A - UBarot + UBarot_A; U = (5 U_A + 8 U_N - U_B)/12
 __global__ void k_lf_final_uv(double* __restrict__ ua, double* __restrict__ va, const double* __restrict__ ubt,
                               const double* __restrict__ vbt, const double* __restrict__ uba,
                               const double* __restrict__ vba, const double* __restrict__ un,
                               const double* __restrict__ ub, const double* __restrict__ vn,
-                              const double* __restrict__ vb, const double* __restrict__ h, long npts, int K, long ncols,
-                              double* __restrict__ uo, double* __restrict__ vo, double* __restrict__ hm) {
+                              const double* __restrict__ vb, long npts, int K, long ncols,
+                              double* __restrict__ uo, double* __restrict__ vo) {
   LF_CP(ncols, npts) {
     const long g = c * npts + p;
     const long q = (c / K) * npts + p;
@@ -337,8 +451,6 @@ __global__ void k_lf_final_uv(double* __restrict__ ua, double* __restrict__ va, 
     va[g] = b;
     uo[g] = (5.0 * a + 8.0 * un[g] - ub[g]) / 12.0;
     vo[g] = (5.0 * b + 8.0 * vn[g] - vb[g]) / 12.0;
-    const double hh = h[g];
-    hm[g] = (5.0 * hh + 8.0 * hh - hh) / 12.0;
   }
 }
 
@@ -374,16 +486,17 @@ struct dsht_lfam3 {
   // constants
   double *d_cdk = nullptr, *d_fdk = nullptr, *d_rcdk = nullptr, *d_rfdk = nullptr, *d_zck = nullptr;
   double *d_mu = nullptr, *d_cs = nullptr, *d_two_omega = nullptr;
+  double *d_m1 = nullptr, *d_m2 = nullptr, *d_dfac = nullptr;  // QUICK weights per half level
   double *d_dmom = nullptr, *d_dtrc = nullptr, *d_advf = nullptr, *d_nn1 = nullptr, *d_hcoef = nullptr,
          *d_e = nullptr;
   double *H = nullptr, *KV = nullptr, *KD = nullptr, *BF = nullptr;
   // state: levels B (0), N (1), A (2)
   double *U[3] = {}, *V[3] = {}, *TS[3] = {}, *SP[3] = {};
   // work
-  double *ucos = nullptr, *vcos = nullptr, *VD = nullptr, *OMG = nullptr, *Dens = nullptr, *Hyd = nullptr;
+  double *ucos = nullptr, *vcos = nullptr, *VD = nullptr, *Dens = nullptr, *Hyd = nullptr;
   double *Geo = nullptr, *GLon = nullptr, *GLat = nullptr, *Am = nullptr, *Bg = nullptr, *Cg = nullptr;
-  double *URHS = nullptr, *VRHS = nullptr, *Upr = nullptr, *Vpr = nullptr, *Hm = nullptr;
-  double *TSpr = nullptr, *HT = nullptr, *FLX = nullptr, *FU = nullptr, *FV = nullptr, *VF = nullptr;
+  double *URHS = nullptr, *VRHS = nullptr, *Upr = nullptr, *Vpr = nullptr;
+  double *TSpr = nullptr, *HT = nullptr, *FU = nullptr, *FV = nullptr, *VF = nullptr;
   double *b2[20] = {};  // 2-D barotropic work, one grid per run each
   double *wVD = nullptr, *wGeo = nullptr, *wC = nullptr, *w1 = nullptr, *w2 = nullptr;
   double *wB = nullptr, *wC2 = nullptr, *wDSP = nullptr, *wDDiv = nullptr, *wZero = nullptr;
@@ -430,30 +543,20 @@ void lf_free(dsht_lfam3* s) {
     DSHT_HIP(hipGetLastError());                                                         \
   } while (0)
 
+// column walks over the points of nr runs
+#define LF_LAUNCHC(kernel, npts, nr, s, ...)                                                  \
+  do {                                                                                        \
+    const int th_ = lf_threads(npts, nr);                                                     \
+    hipLaunchKernelGGL(kernel, lf_gridc(npts, nr, th_), dim3(th_), 0, s, __VA_ARGS__);        \
+    DSHT_HIP(hipGetLastError());                                                              \
+  } while (0)
+
 // ---- the reference's diagnostics on every active run (column kernels)
 int lf_uvbarot(dsht_lfam3* s, const double* u, const double* v, double* ub, double* vb, int nr, hipStream_t st) {
   const long np = s->np, K = s->K;
   for (int r = 0; r < nr; r++)
     if (int rc = launch_col_uvbarot(u + r * K * np, v + r * K * np, s->H + r * K * np, np, s->K, s->d_cdk,
                                     ub + r * np, vb + r * np, (int)np, st))
-      return rc;
-  return 0;
-}
-
-int lf_omega(dsht_lfam3* s, const double* div, int nr, hipStream_t st) {
-  const long np = s->np, K = s->K;
-  for (int r = 0; r < nr; r++)
-    if (int rc = launch_col_omega(div + r * K * np, s->H + r * K * np, np, s->K, s->d_cdk, s->OMG + r * (K + 1) * np,
-                                  np, (int)np, st))
-      return rc;
-  return 0;
-}
-
-int lf_hydpres(dsht_lfam3* s, int nr, hipStream_t st) {
-  const long np = s->np, K = s->K;
-  for (int r = 0; r < nr; r++)
-    if (int rc = launch_col_hydpres(s->Dens + r * K * np, s->H + r * K * np, np, s->K, s->d_cdk, s->cfg.grav,
-                                    s->Hyd + r * K * np, np, (int)np, st))
       return rc;
   return 0;
 }
@@ -468,45 +571,20 @@ int lf_vordiv(dsht_lfam3* s, const double* u, const double* v, int nc, hipStream
   return dsht_inv_d(p, DSHT_VAL, s->wVD, 2l * nc, 1, s->VD, s->np, 2 * nc, nullptr, st);
 }
 
-// HBEBaroc_MOMRHS_VorDivForm (HBEBaroc_hspm_vfvm_mod.f90:321-443) -> URHS, VRHS
-int lf_mom_rhs(dsht_lfam3* s, const double* u, const double* v, const double* cor_un, const double* cor_ub,
-               const double* cor_vn, const double* cor_vb, double cn, double cb, const double* sp, int nc,
-               hipStream_t st) {
+// HBEBaroc_MOMRHS_VorDivForm (HBEBaroc_hspm_vfvm_mod.f90:321-443) -> URHS, VRHS, with the vorticity
+// and divergence of (u, v) in VD.  pred: the Coriolis terms f (cn (u, v) + cb (xa, xb)), else
+// f (xa, xb)
+int lf_mom_rhs(dsht_lfam3* s, const double* u, const double* v, const double* xa, const double* xb, bool pred, double cn,
+               double cb, const double* sp, int nr, hipStream_t st) {
   dsht_plan* p = s->p;
-  const long n = (long)nc * s->np;
+  const int nc = nr * s->K;
   // w_GeoPot = w_xy(GeoPot); xy_GradLat_w, xy_GradLon_w of it
   if (int rc = dsht_fwd_d(p, DSHT_VAL, s->Geo, s->np, s->wGeo, nc, 1, nc, nullptr, st)) return rc;
   if (int rc = dsht_inv_vgrad_d(p, s->wGeo, nc, 1, nullptr, s->GLon, s->GLat, s->np, nc, nullptr, st)) return rc;
-  MomArgs a;
-  a.u = u;
-  a.v = v;
-  a.omg = s->OMG;
-  a.vor = s->VD;
-  a.h = s->H;
-  a.hyd = s->Hyd;
-  a.sp = sp;
-  a.dens = s->Dens;
-  a.glon = s->GLon;
-  a.glat = s->GLat;
-  a.un = cor_un;
-  a.ub = cor_ub;
-  a.vn = cor_vn;
-  a.vb = cor_vb;
-  a.two_omega = s->d_two_omega;
-  a.mu = s->d_mu;
-  a.cs = s->d_cs;
-  a.rfdk = s->d_rfdk;
-  a.ref_dens = s->cfg.ref_dens;
-  a.radius = p->R;
-  a.cn = cn;
-  a.cb = cb;
-  a.npts = s->np;
-  a.I = s->I;
-  a.K = s->K;
-  a.am = s->Am;
-  a.bg = s->Bg;
-  a.cg = s->Cg;
-  LF_LAUNCH2(k_lf_mom, nc, s->np, st, a, (long)nc);
+  const MomArgs a{s->cfg.ref_dens, p->R, s->cfg.depth, cn, cb, s->np, s->I, s->K};
+  auto k = pred ? k_lf_mom<true> : k_lf_mom<false>;
+  LF_LAUNCHC(k, s->np, nr, st, a, u, v, xa, xb, s->VD + (long)nc * s->np, s->VD, s->Hyd, s->Dens, s->GLon, s->GLat, sp,
+             s->d_two_omega, s->d_mu, s->d_cs, s->d_cdk, s->d_rfdk, s->Am, s->Bg, s->Cg);
   // (w_Vor_RHS, w_Div_RHS) = (-H(A, B), H(B, -A)) = calc_UVCosLat2VorDiv(B, -A); then
   // w_Div_RHS - w_Lapla_w(w_xy(C)) = + n(n+1) w_xy(C)
   if (int rc = dsht_uv2vordiv_d(p, s->Bg, s->Am, s->np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, nullptr, st)) return rc;
@@ -515,20 +593,14 @@ int lf_mom_rhs(dsht_lfam3* s, const double* u, const double* v, const double* co
   return dsht_vordiv2uv_d(p, s->wVD, s->wVD + nc, 2l * nc, 1, s->URHS, s->VRHS, s->np, nc, st);
 }
 
-// HBEBaroc_HTRCRHS (HBEBaroc_hspm_vfvm_mod.f90:119-202) for both tracers of the active runs
-int lf_htrc(dsht_lfam3* s, const double* ts, const double* u, const double* v, const double* h, int nr,
-            hipStream_t st) {
+// HBEBaroc_HTRCRHS (HBEBaroc_hspm_vfvm_mod.f90:119-202) for both tracers of the active runs, with
+// the divergence of (u, v) in VD and the thickness factor h
+int lf_htrc(dsht_lfam3* s, const double* ts, const double* u, const double* v, double h, int nr, hipStream_t st) {
   dsht_plan* p = s->p;
-  const long np = s->np, K = s->K;
-  const int nt = 2 * nr * s->K;
-  for (int rt = 0; rt < 2 * nr; rt++) {
-    const int r = rt / 2;
-    if (int rc = launch_col_quick(s->OMG + r * (K + 1) * np, np, ts + rt * K * np, np, s->K, s->d_cdk, s->d_rfdk, 0,
-                                  s->FLX + rt * (K + 1) * np, np, (int)np, st))
-      return rc;
-  }
-  LF_LAUNCH2(k_lf_htrc_grid, nt, np, st, ts, u, v, h, s->d_cs, s->FLX, s->d_rcdk, np, s->I, s->K, (long)nt, s->FU, s->FV,
-             s->VF);
+  const long np = s->np;
+  const int nc = nr * s->K, nt = 2 * nc;
+  LF_LAUNCHC(k_lf_htrc, np, nr, st, ts, u, v, s->VD + (long)nc * np, s->cfg.depth, h, s->d_cs, s->d_cdk, s->d_rcdk,
+             s->d_rfdk, s->d_m1, s->d_m2, s->d_dfac, np, s->I, s->K, s->FU, s->FV, s->VF);
   if (int rc = dsht_alpha_fwd_d(p, s->FU, s->FV, np, s->w1, nt, 1, nt, nullptr, st)) return rc;
   if (int rc = dsht_fwd_d(p, DSHT_VAL, s->VF, np, s->w2, nt, 1, nt, nullptr, st)) return rc;
   LF_LAUNCH2(k_lf_htrc_spec, s->L, nt, st, s->w1, s->w2, s->d_advf, s->L, nt);
@@ -621,6 +693,13 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
     s->zck[k] = ck[k + 1];
     s->rcdk[k] = 1.0 / s->cdk[k];
   }
+  std::vector<double> m1(K + 1, 0.0), m2(K + 1, 0.0), dfac(K + 1, 0.0);  // HBEBaroc_hspm_vfvm_mod.f90:264-266
+  for (int h = 1; h < K; h++) {
+    const double sum = s->cdk[h - 1] + s->cdk[h];
+    m1[h] = s->cdk[h] / sum;
+    m2[h] = s->cdk[h - 1] / sum;
+    dfac[h] = (0.125 * s->cdk[h]) * s->cdk[h - 1];
+  }
   std::vector<double> cs(J), nn1(L), e(L), hcoef(L);
   for (int j = 0; j < J; j++) cs[j] = std::sqrt((1.0 - p->mu[j]) * (1.0 + p->mu[j]));
   for (int n = 0; n <= p->N; n++)
@@ -642,6 +721,9 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
   U(&s->d_rcdk, s->rcdk);
   U(&s->d_rfdk, s->rfdk);
   U(&s->d_zck, s->zck);
+  U(&s->d_m1, m1);
+  U(&s->d_m2, m2);
+  U(&s->d_dfac, dfac);
   U(&s->d_mu, p->mu);
   U(&s->d_cs, cs);
   U(&s->d_nn1, nn1);
@@ -664,7 +746,6 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
   A(&s->ucos, NC * np);
   A(&s->vcos, NC * np);
   A(&s->VD, 2 * NC * np);
-  A(&s->OMG, R * (K + 1) * np);
   A(&s->Dens, NC * np);
   A(&s->Hyd, NC * np);
   A(&s->Geo, NC * np);
@@ -677,10 +758,8 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
   A(&s->VRHS, NC * np);
   A(&s->Upr, NC * np);
   A(&s->Vpr, NC * np);
-  A(&s->Hm, NC * np);
   A(&s->TSpr, 2 * NC * np);
   A(&s->HT, 2 * NC * np);
-  A(&s->FLX, 2 * R * (K + 1) * np);
   A(&s->FU, 2 * NC * np);
   A(&s->FV, 2 * NC * np);
   A(&s->VF, 2 * NC * np);
@@ -827,7 +906,6 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   if ((rc = lf_uvbarot(s, UB, VB, b2[UBB], b2[VBB], nr, st))) return rc;
   // ---- predictor
   if ((rc = lf_vordiv(s, UN, VN, nc, st))) return rc;
-  if ((rc = lf_omega(s, s->VD + (long)nc * np, nr, st))) return rc;  // H_A = H_B: omega from H_B
   EosArgs ea;
   ea.ref_dens = c.ref_dens;
   ea.ptemp_dep = -c.beta_t;
@@ -837,23 +915,20 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   ea.ref_salt = c.ref_salt;
   ea.depth = c.depth;
   ea.grav = c.grav;
-  LF_LAUNCH2(k_lf_eos, nc, np, st, TN, np, K, s->d_zck, ea, (long)nc, s->Dens);
-  if ((rc = lf_hydpres(s, nr, st))) return rc;
-  if ((rc = lf_mom_rhs(s, UN, VN, UN, UB, VN, VB, gamma, 1.0 - gamma, PN, nc, st))) return rc;
+  LF_LAUNCHC(k_lf_eos_hyd, np, nr, st, TN, np, K, s->d_zck, s->d_cdk, ea, s->Dens, s->Hyd);
+  if ((rc = lf_mom_rhs(s, UN, VN, UB, VB, true, gamma, 1.0 - gamma, PN, nr, st))) return rc;
   LF_LAUNCH2(k_lf_pred_uv, nc, np, st, s->URHS, s->VRHS, UN, UB, VN, VB, s->d_two_omega, s->d_mu, np, I, K,
              0.5 * (2.0 * dt), c56dt, c.alpha > 0.0 ? 1 : 0, (long)nc, s->Upr, s->Vpr);
   if ((rc = lf_uvbarot(s, s->Upr, s->Vpr, b2[UBT], b2[VBT], nr, st))) return rc;
   LF_LAUNCH2(k_lf_barot_shift, nc, np, st, s->Upr, s->Vpr, b2[UBT], b2[VBT], b2[UBN], b2[VBN], np, K, (long)nc);
-  if ((rc = lf_htrc(s, TN, UN, VN, s->H, nr, st))) return rc;
+  if ((rc = lf_htrc(s, TN, UN, VN, c.depth, nr, st))) return rc;
   LF_LAUNCH2(k_lf_pred_trc, nt, np, st, TN, TB, s->HT, s->H, np, K, c56dt, (long)nt, s->TSpr);
   // ---- corrector
   if ((rc = lf_vordiv(s, s->Upr, s->Vpr, nc, st))) return rc;
-  if ((rc = lf_omega(s, s->VD + (long)nc * np, nr, st))) return rc;
-  LF_LAUNCH2(k_lf_eos, nc, np, st, s->TSpr, np, K, s->d_zck, ea, (long)nc, s->Dens);
-  if ((rc = lf_hydpres(s, nr, st))) return rc;
+  LF_LAUNCHC(k_lf_eos_hyd, np, nr, st, s->TSpr, np, K, s->d_zck, s->d_cdk, ea, s->Dens, s->Hyd);
   const double alpha_ = 0.5, gamma_ = 0.5;
-  const double cn = gamma_ + alpha_, cb = 1.0 - alpha_ - gamma_;
-  if ((rc = lf_mom_rhs(s, s->Upr, s->Vpr, UN, UB, VN, VB, cn, cb, PN, nc, st))) return rc;
+  const double cn = gamma_ + alpha_, cb = 1.0 - alpha_ - gamma_;  // 1 and 0: the present level alone
+  if ((rc = lf_mom_rhs(s, s->Upr, s->Vpr, UN, VN, false, cn, cb, PN, nr, st))) return rc;
   // ImplUV (DOGCM_Phys_hspm_vfvm_mod.f90:666-748): implicit vertical viscosity, then
   // backward-Euler lateral viscosity on vorticity and divergence
   for (int r = 0; r < nr; r++) {
@@ -896,11 +971,11 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   LF_LAUNCH(k_lf_add2, n2, st, b2[UBAR], b2[DU], b2[VBAR], b2[DV], PN, b2[DSP], n2, b2[UBA], b2[VBA], PA);
   // ---- full velocity, time-centred fields, tracers
   if ((rc = lf_uvbarot(s, UA, VA, b2[UBT], b2[VBT], nr, st))) return rc;
-  LF_LAUNCH2(k_lf_final_uv, nc, np, st, UA, VA, b2[UBT], b2[VBT], b2[UBA], b2[VBA], UN, UB, VN, VB, s->H, np, K, (long)nc,
-             s->Upr, s->Vpr, s->Hm);
+  LF_LAUNCH2(k_lf_final_uv, nc, np, st, UA, VA, b2[UBT], b2[VBT], b2[UBA], b2[VBA], UN, UB, VN, VB, np, K, (long)nc,
+             s->Upr, s->Vpr);
   if ((rc = lf_vordiv(s, s->Upr, s->Vpr, nc, st))) return rc;
-  if ((rc = lf_omega(s, s->VD + (long)nc * np, nr, st))) return rc;  // from H_N
-  if ((rc = lf_htrc(s, s->TSpr, s->Upr, s->Vpr, s->Hm, nr, st))) return rc;
+  const double hm = (5.0 * c.depth + 8.0 * c.depth - c.depth) / 12.0;  // the time-centred thickness factor
+  if ((rc = lf_htrc(s, s->TSpr, s->Upr, s->Vpr, hm, nr, st))) return rc;
   // ImplTRC (DOGCM_Phys_hspm_vfvm_mod.f90:544-662)
   for (int rt = 0; rt < 2 * nr; rt++) {
     const long o = (long)rt * K * np, ol = (long)(rt / 2) * K * np;
