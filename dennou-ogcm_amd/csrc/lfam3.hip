@@ -454,6 +454,97 @@ __global__ void k_lf_final_uv(double* __restrict__ ua, double* __restrict__ va, 
   }
 }
 
+// The implicit vertical diffusion of a tracer (calc_VDiffTRCEq, DOGCM_Phys_hspm_vfvm_mod.f90:
+// 752-861) or of momentum (MOM; calc_VDiffMOMEq, :865-975) with the pool's constant
+// viscosities, thickness factor and bottom friction: every grid point has the same matrix, so
+// its DGTSV elimination (factors, interchanges, finished rows) is done once on the host
+// (lf_vfactor) and a thread only carries its column's right-hand side through it, in DGTSV's
+// order of operations: qa = q0 + x.  The right-hand side waits for the backward sweep in
+// registers (K <= KM), or in qa (KM = 0).  Bound by HBM: three layer fields, against the five
+// and a workspace of the general k_col_vdiff: at T170L60 two fields take 67 us (5.6 TB/s), there
+// 163; loading each group only when it is worked on took 111.  Grid y: sections of K layers,
+// grid z: field pairs.
+struct VSolve {
+  const double *q0[2], *rhs[2];
+  double* qa[2];
+};
+constexpr int VL = 8;  // layers whose loads are in flight together
+template <int KM, bool MOM>
+__global__ __launch_bounds__(256) void k_lf_vsolve(VSolve a, const double* __restrict__ fact,
+                                                   const double* __restrict__ dd, const double* __restrict__ du,
+                                                   const double* __restrict__ du2, const int* __restrict__ swapped,
+                                                   double dt, double e3, long npts, int K) {
+#pragma clang fp contract(off)
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= npts) return;
+  const long o = (long)blockIdx.y * K * npts + p;
+  const double* __restrict__ q0 = a.q0[blockIdx.z] + o;
+  const double* __restrict__ rhs = a.rhs[blockIdx.z] + o;
+  double* __restrict__ qa = a.qa[blockIdx.z] + o;
+  double xa = 0.0, xb = 0.0;  // x[k+1], x[k+2]
+  auto right = [&](double x) {
+    const double bt = dt * x;
+    return MOM ? bt : bt / e3;
+  };
+  auto back = [&](int k, double b, double q) {
+    const double t = b - du[k] * xa;
+    const double x = (t - du2[k] * xb) / dd[k];
+    __builtin_nontemporal_store(q + x, qa + (long)k * npts);
+    xb = xa;
+    xa = x;
+  };
+  // rows k-1 and k after elimination step k-1
+  auto step = [&](int k, double& up, double& lo) {
+    if (swapped[k - 1]) {
+      const double t = up;
+      up = lo;
+      lo = t - fact[k - 1] * lo;
+    } else {
+      lo = lo - fact[k - 1] * up;
+    }
+  };
+  if constexpr (KM > 0) {
+    // the next group's loads go out before this group is worked on
+    double b[KM], x[2][VL];
+    auto load = [&](const double* __restrict__ f, int k0, double (&to)[VL]) {
+#pragma unroll
+      for (int u = 0; u < VL; u++) to[u] = lf_ld(f + (long)(k0 + u < K ? k0 + u : K - 1) * npts);
+    };
+    load(rhs, 0, x[0]);
+#pragma unroll
+    for (int k0 = 0; k0 < KM; k0 += VL) {
+      if (k0 >= K) break;
+      if (k0 + VL < KM && k0 + VL < K) load(rhs, k0 + VL, x[(k0 / VL + 1) & 1]);
+#pragma unroll
+      for (int u = 0; u < VL; u++) {
+        const int k = k0 + u;
+        if (k >= K) break;
+        b[k] = right(x[(k0 / VL) & 1][u]);
+        if (k > 0) step(k, b[k > 0 ? k - 1 : 0], b[k]);
+      }
+    }
+    const int last = (K - 1) / VL * VL;
+#pragma unroll
+    for (int k0 = KM - VL; k0 >= 0; k0 -= VL) {
+      if (k0 > last) continue;
+      if (k0 == last) load(q0, k0, x[(k0 / VL) & 1]);
+      if (k0 > 0) load(q0, k0 - VL, x[(k0 / VL + 1) & 1]);
+#pragma unroll
+      for (int u = VL - 1; u >= 0; u--)
+        if (k0 + u < K) back(k0 + u, b[k0 + u], x[(k0 / VL) & 1][u]);
+    }
+  } else {
+    double up = right(lf_ld(rhs));
+    for (int k = 1; k < K; k++) {
+      double lo = right(lf_ld(rhs + (long)k * npts));
+      step(k, up, lo);
+      qa[(long)(k - 1) * npts] = up;
+      up = lo;
+    }
+    for (int k = K - 1; k >= 0; k--) back(k, k == K - 1 ? up : qa[(long)k * npts], lf_ld(q0 + (long)k * npts));
+  }
+}
+
 // T_A = H_0 T_A / H_A (DOGCM_Phys_hspm_vfvm_mod.f90:641)
 __global__ void k_lf_trc_final(double* __restrict__ ta, const double* __restrict__ h, long npts, int K, long ncols) {
   LF_CP(ncols, npts) {
@@ -489,7 +580,7 @@ struct dsht_lfam3 {
   double *d_m1 = nullptr, *d_m2 = nullptr, *d_dfac = nullptr;  // QUICK weights per half level
   double *d_dmom = nullptr, *d_dtrc = nullptr, *d_advf = nullptr, *d_nn1 = nullptr, *d_hcoef = nullptr,
          *d_e = nullptr;
-  double *H = nullptr, *KV = nullptr, *KD = nullptr, *BF = nullptr;
+  double* H = nullptr;
   // state: levels B (0), N (1), A (2)
   double *U[3] = {}, *V[3] = {}, *TS[3] = {}, *SP[3] = {};
   // work
@@ -500,8 +591,10 @@ struct dsht_lfam3 {
   double *b2[20] = {};  // 2-D barotropic work, one grid per run each
   double *wVD = nullptr, *wGeo = nullptr, *wC = nullptr, *w1 = nullptr, *w2 = nullptr;
   double *wB = nullptr, *wC2 = nullptr, *wDSP = nullptr, *wDDiv = nullptr, *wZero = nullptr;
-  double* vwork = nullptr;
-  long lvwork = 0;
+  // the elimination of the constant vertical systems (momentum, tracers): fact, d, du, du2 and
+  // the interchanges, K each
+  double* d_vf[2] = {};
+  int* d_vs[2] = {};
 };
 
 namespace {
@@ -558,6 +651,72 @@ int lf_uvbarot(dsht_lfam3* s, const double* u, const double* v, double* ub, doub
     if (int rc = launch_col_uvbarot(u + r * K * np, v + r * K * np, s->H + r * K * np, np, s->K, s->d_cdk,
                                     ub + r * np, vb + r * np, (int)np, st))
       return rc;
+  return 0;
+}
+
+// DGTSV's elimination (LAPACK 3.x SRC/dgtsv.f, partial pivoting by row interchange) of the
+// constant vertical system of momentum or of the tracers (rows as k_col_vdiff builds them):
+// fac = fact, d, du, du2 (K each), swapped = 1 where a step interchanged its rows
+void lf_vfactor(const dsht_lfam3* s, bool mom, std::vector<double>& fac, std::vector<int>& swapped) {
+#pragma clang fp contract(off)
+  const dsht_lfam3_config& c = s->cfg;
+  const int K = s->K;
+  const double kv = mom ? c.vvisc : c.vdiff, e3 = c.depth, alpha = c.lambda;
+  const bool sfc = (mom ? c.mom_sfc_bc : c.trc_sfc_bc) == 'D', btm = (mom ? c.mom_btm_bc : c.trc_btm_bc) == 'D';
+  std::vector<double> r(K + 1), al(K, 0.0), ad(K), au(K, 0.0);
+  r[0] = kv / (s->fdk[0] * e3);
+  r[K] = kv / (s->fdk[K] * e3);
+  for (int h = 1; h < K; h++) {
+    const double sum = s->cdk[h - 1] + s->cdk[h];
+    const double m1 = s->cdk[h] / sum, m2 = s->cdk[h - 1] / sum;
+    r[h] = (m1 * kv + m2 * kv) / (s->fdk[h] * (m1 * e3 + m2 * e3));
+  }
+  for (int k = 0; k < K; k++) {
+    const double ac = alpha * (c.dt / (e3 * s->cdk[k]));
+    if (k > 0) al[k] = -(ac * r[k]);
+    if (k < K - 1) au[k] = -(ac * r[k + 1]);
+    if (k == 0)
+      ad[k] = sfc ? 1.0 + ac * (r[1] + 2.0 * r[0]) : 1.0 + ac * r[1];
+    else if (k == K - 1)
+      ad[k] = !btm ? 1.0 + ac * r[k] : mom ? 1.0 + ac * (c.btm_frict + r[k]) : 1.0 + ac * (2.0 * r[K] + r[k]);
+    else
+      ad[k] = 1.0 + ac * (r[k] + r[k + 1]);
+  }
+  fac.assign(4 * (size_t)K, 0.0);
+  swapped.assign(K, 0);
+  double *fact = fac.data(), *d = fact + K, *du = d + K, *du2 = du + K;
+  for (int k = 0; k < K; k++) d[k] = ad[k], du[k] = au[k];
+  for (int j = 0; j < K - 1; j++) {
+    const double dl = al[j + 1];
+    if (std::fabs(d[j]) >= std::fabs(dl)) {
+      fact[j] = dl / d[j];
+      d[j + 1] = d[j + 1] - fact[j] * du[j];
+    } else {
+      swapped[j] = 1;
+      fact[j] = d[j] / dl;
+      d[j] = dl;
+      const double temp = d[j + 1];
+      d[j + 1] = du[j] - fact[j] * temp;
+      if (j < K - 2) {
+        du2[j] = du[j + 1];
+        du[j + 1] = -fact[j] * du2[j];
+      }
+      du[j] = temp;
+    }
+  }
+}
+
+// one or two fields (z) of ny sections through the constant solve
+int lf_vsolve(dsht_lfam3* s, bool mom, const VSolve& a, int ny, int nz, hipStream_t st) {
+  const int K = s->K, w = mom ? 0 : 1, th = lf_threads(s->np, ny * nz);
+  auto k = mom ? (K <= 32 ? k_lf_vsolve<32, true> : K <= 64 ? k_lf_vsolve<64, true> : k_lf_vsolve<0, true>)
+               : (K <= 32 ? k_lf_vsolve<32, false> : K <= 64 ? k_lf_vsolve<64, false> : k_lf_vsolve<0, false>);
+  dim3 grid = lf_gridc(s->np, ny, th);
+  grid.z = nz;
+  const double* f = s->d_vf[w];
+  hipLaunchKernelGGL(k, grid, dim3(th), 0, st, a, f, f + K, f + 2 * K, f + 3 * K, s->d_vs[w], s->cfg.dt, s->cfg.depth,
+                     s->np, K);
+  DSHT_HIP(hipGetLastError());
   return 0;
 }
 
@@ -734,9 +893,6 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
   A(&s->d_dtrc, L);
   A(&s->d_advf, L);
   A(&s->H, NC * np);
-  A(&s->KV, NC * np);
-  A(&s->KD, NC * np);
-  A(&s->BF, R * np);
   for (int lv = 0; lv < 3; lv++) {
     A(&s->U[lv], NC * np);
     A(&s->V[lv], NC * np);
@@ -774,8 +930,17 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
   A(&s->wDSP, (size_t)L * R);
   A(&s->wDDiv, (size_t)L * R);
   A(&s->wZero, (size_t)L * R);
-  s->lvwork = 3l * K * np;
-  A(&s->vwork, s->lvwork);
+  for (int w = 0; w < 2; w++) {
+    std::vector<double> vf;
+    std::vector<int> vs;
+    lf_vfactor(s, w == 0, vf, vs);
+    U(&s->d_vf[w], vf);
+    double* d = nullptr;
+    A(&d, (K + 1) / 2);
+    s->d_vs[w] = (int*)d;
+    if (!rc && hipMemcpy(d, vs.data(), sizeof(int) * K, hipMemcpyHostToDevice) != hipSuccess)
+      rc = fail(DSHT_EDEVICE, "LF-AM3 pool: upload failed");
+  }
   if (rc) {
     lf_free(s);
     delete s;
@@ -787,12 +952,8 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
     DSHT_HIP(hipGetLastError());
     return 0;
   };
-  // constant fields: xyz_H = D, the vertical viscosity/diffusivity, bottom friction; the
-  // state and every work array start at zero
+  // xyz_H = D; the state starts at zero
   if (!rc) rc = fill(s->H, c.depth, NC * np);
-  if (!rc) rc = fill(s->KV, c.vvisc, NC * np);
-  if (!rc) rc = fill(s->KD, c.vdiff, NC * np);
-  if (!rc) rc = fill(s->BF, c.btm_frict, R * np);
   if (!rc) rc = fill(s->wZero, 0.0, (long)L * R);
   for (int lv = 0; lv < 3 && !rc; lv++) {
     rc = fill(s->U[lv], 0.0, NC * np);
@@ -931,17 +1092,7 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   if ((rc = lf_mom_rhs(s, s->Upr, s->Vpr, UN, VN, false, cn, cb, PN, nr, st))) return rc;
   // ImplUV (DOGCM_Phys_hspm_vfvm_mod.f90:666-748): implicit vertical viscosity, then
   // backward-Euler lateral viscosity on vorticity and divergence
-  for (int r = 0; r < nr; r++) {
-    const long o = (long)r * K * np;
-    if ((rc = launch_col_vdiff(UN + o, s->URHS + o, s->KV + o, s->H + o, np, K, s->d_cdk, s->d_fdk, dt, c.lambda,
-                               c.mom_sfc_bc == 'D', c.mom_btm_bc == 'D', s->BF + r * np, UA + o, np, s->vwork,
-                               (int)np, st)))
-      return rc;
-    if ((rc = launch_col_vdiff(VN + o, s->VRHS + o, s->KV + o, s->H + o, np, K, s->d_cdk, s->d_fdk, dt, c.lambda,
-                               c.mom_sfc_bc == 'D', c.mom_btm_bc == 'D', s->BF + r * np, VA + o, np, s->vwork,
-                               (int)np, st)))
-      return rc;
-  }
+  if ((rc = lf_vsolve(s, true, VSolve{{UN, VN}, {s->URHS, s->VRHS}, {UA, VA}}, nr, 2, st))) return rc;
   LF_LAUNCH2(k_lf_uvcos, nc, np, st, UA, VA, s->d_cs, np, I, (long)nc, s->ucos, s->vcos);
   if ((rc = dsht_uv2vordiv_d(p, s->ucos, s->vcos, np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, s->d_dmom, st))) return rc;
   if ((rc = dsht_vordiv2uv_d(p, s->wVD, s->wVD + nc, 2l * nc, 1, UA, VA, np, nc, st))) return rc;
@@ -977,12 +1128,7 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   const double hm = (5.0 * c.depth + 8.0 * c.depth - c.depth) / 12.0;  // the time-centred thickness factor
   if ((rc = lf_htrc(s, s->TSpr, s->Upr, s->Vpr, hm, nr, st))) return rc;
   // ImplTRC (DOGCM_Phys_hspm_vfvm_mod.f90:544-662)
-  for (int rt = 0; rt < 2 * nr; rt++) {
-    const long o = (long)rt * K * np, ol = (long)(rt / 2) * K * np;
-    if ((rc = launch_col_vdiff(TN + o, s->HT + o, s->KD + ol, s->H + ol, np, K, s->d_cdk, s->d_fdk, dt, c.lambda,
-                               c.trc_sfc_bc == 'D', c.trc_btm_bc == 'D', nullptr, TA + o, np, s->vwork, (int)np, st)))
-      return rc;
-  }
+  if ((rc = lf_vsolve(s, false, VSolve{{TN, nullptr}, {s->HT, nullptr}, {TA, nullptr}}, 2 * nr, 1, st))) return rc;
   if ((rc = dsht_fwd_d(p, DSHT_VAL, TA, np, s->w1, nt, 1, nt, s->d_dtrc, st))) return rc;
   if ((rc = dsht_inv_d(p, DSHT_VAL, s->w1, nt, 1, TA, np, nt, nullptr, st))) return rc;
   LF_LAUNCH2(k_lf_trc_final, nt, np, st, TA, s->H, np, K, (long)nt);

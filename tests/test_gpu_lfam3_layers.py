@@ -1,0 +1,55 @@
+"""The LF-AM3 step's column walks and constant vertical solve (csrc/lfam3.hip) against the CPU
+restatement at the layer counts where their code changes: the smallest (2 layers: no interior
+QUICK half level; 4: one), partly filled rounds of layers, and the solve's register forms
+(up to 32 and 64 layers) and memory form (more).  One step each; boundary conditions of either
+kind; a large viscosity on the thin bottom layers makes the solve interchange rows.
+
+Tolerance: a wrong factor, layer or boundary row changes a field by 1e-6 or more of its size
+in one step.  Rounding: the horizontal gradient of the constant geopotential (5e4 m2/s2) is
+rounding noise of the transforms, about n eps geo, times the density over the winds' forcing:
+below 1e-11 of the winds at T21; the surface pressure cancels one more digit.  1e-9.
+"""
+import pytest
+
+from test_gpu_lfam3 import OMEGA, _load, _pool, _read
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-9
+
+
+@pytest.mark.parametrize("km,cfg", [
+    (2, {}), (4, {"trc_sfc_bc": "D"}), (10, {"mom_sfc_bc": "D", "mom_btm_bc": "N"}), (32, {"btm_frict": 1e-4}),
+    (34, {"trc_btm_bc": "D"}), (64, {}), (66, {}),
+    (20, {"vvisc": 50.0, "vdiff": 20.0}), (40, {"vvisc": 50.0, "vdiff": 20.0, "lam": 1.0}), (68, {"vvisc": 50.0})])
+def test_layers_match_oracle(gpu, km, cfg):
+    import numpy as np
+    import torch
+    import lfam3
+    import oracle
+    from conftest import rel_l2
+    N, I, J = 21, 64, 32
+    _, pool = _pool(N, I, J, km, 2, dt=1800.0, **cfg)
+    o = oracle.Oracle(N, I, J, 6.371e6)
+    ocfg = lfam3.Config(dt=1800.0, **cfg)
+    states, steppers = [], []
+    for r in range(2):
+        st = lfam3.initial_state(o, km, seed=km + r)
+        states.append(st)
+        steppers.append(lfam3.Step(o, km, ocfg, (r + 1) * OMEGA))
+        _load(pool, r, st)
+        pool.set_rotation(r, (r + 1) * OMEGA)
+    if cfg.get("vvisc", 0.0) > 1.0:  # the system of these cases does interchange rows
+        s = steppers[0]
+        one = np.ones((km, 1, 1))
+        _, swaps = oracle.col_vdiff(one, one, cfg["vvisc"] * one, ocfg.depth * one, s.cdk, s.fdk, ocfg.dt, ocfg.lam,
+                                    "N", "D", btm_frict=np.zeros((1, 1)))
+        assert swaps > 0
+    torch.cuda.synchronize()
+    pool.step(2)
+    torch.cuda.synchronize()
+    for r in range(2):
+        ref = steppers[r].advance(states[r])
+        got = _read(pool, r)
+        for f in ("U", "V", "T", "S", "P"):
+            assert rel_l2(got[f], ref[f + "N"]) < TOL, (r, f)
+        assert np.array_equal(got["UB"], ref["UB"])
