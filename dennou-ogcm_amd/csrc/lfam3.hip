@@ -75,18 +75,52 @@ __global__ void k_lf_fill(double* __restrict__ x, double v, long n) {
   LF_LOOP(n) x[g] = v;
 }
 
-// Column walks: one thread per grid point of a run (grid y) goes through the layers, LG of them
+// Column walks: one thread per grid point of a run (grid y) goes through the layers, G of them
 // per round with their loads issued together.  The layers' running sums (pressure from the
 // top, omega from the bottom) stay in registers, so a field that is only a step between two
-// others (omega, the vertical fluxes) is never written.  Bound by HBM: every layer field in
-// and out is touched once.
-constexpr int LG = 4;
+// others (omega, the vertical fluxes) is never written.  The next round's loads go out before
+// this round is worked on and stored, so that a round waits neither for its own loads nor for
+// the stores before it.  Bound by HBM on large grids: every layer field in and out is touched
+// once.
 
 __device__ __forceinline__ double lf_ld(const double* x) { return __builtin_nontemporal_load(x); }
 
 inline dim3 lf_gridc(long npts, int nr, int threads) { return dim3((unsigned)((npts + threads - 1) / threads), (unsigned)nr); }
-// small grids take small blocks, so that the columns spread over the chip
+// blocks of 64 where there are fewer waves than SIMDs, to spread the columns over the chip
 inline int lf_threads(long npts, int nr) { return npts * nr >= 65536 ? 256 : 64; }
+
+constexpr int LF_NONE[16] = {};
+// layers k = first, first + dir, ... (K of them): body(k, values) with the values of NF fields
+// (above: layers nearer the end of the walk, clamped to it), G layers a round
+template <int NF, int G, bool NT = true, typename Body>
+__device__ __forceinline__ void lf_walk(const double* const (&f)[NF], long npts, int K, int first, int dir, Body body,
+                                        const int* above = LF_NONE) {
+  double cur[G][NF], nxt[G][NF];
+  auto load = [&](double (&x)[G][NF], int n0) {
+#pragma unroll
+    for (int q = 0; q < G; q++)
+#pragma unroll
+      for (int i = 0; i < NF; i++) {
+        const int n = n0 + q + above[i] < K ? n0 + q + above[i] : K - 1;
+        const double* at = f[i] + (long)(first + dir * n) * npts;
+        x[q][i] = NT ? lf_ld(at) : *at;
+      }
+  };
+  load(cur, 0);
+  int n0 = 0;
+  for (; n0 + G <= K; n0 += G) {
+    load(nxt, n0 + G);
+#pragma unroll
+    for (int q = 0; q < G; q++) body(first + dir * (n0 + q), cur[q]);
+#pragma unroll
+    for (int q = 0; q < G; q++)
+#pragma unroll
+      for (int i = 0; i < NF; i++) cur[q][i] = nxt[q][i];
+  }
+#pragma unroll
+  for (int q = 0; q < G; q++)
+    if (n0 + q < K) body(first + dir * (n0 + q), cur[q]);
+}
 
 // EOS_Linear_Eval(theta, S, p = -RefDens GeoPot) and the hydrostatic pressure of its density
 // (HBEDiagnose_HydPres, HBEDiagnose_hspm_vfvm_mod.f90:315-321) for every layer of every run
@@ -105,28 +139,17 @@ __global__ __launch_bounds__(256) void k_lf_eos_hyd(const double* __restrict__ t
   const long o = r * K * npts + p;
   const double gh = e.grav * e.depth;
   double sum = 0.0;
-  for (int k0 = 0; k0 < K; k0 += 2 * LG) {
-    double t[2 * LG], s[2 * LG];
-#pragma unroll
-    for (int u = 0; u < 2 * LG; u++) {
-      const long k = k0 + u < K ? k0 + u : K - 1;
-      t[u] = lf_ld(tp + k * npts);
-      s[u] = lf_ld(sp + k * npts);
-    }
-#pragma unroll
-    for (int u = 0; u < 2 * LG; u++) {
-      const int k = k0 + u;
-      if (k >= K) break;
-      const double geo = e.grav * (e.depth * zck[k]);
-      const double pr = -e.ref_dens * geo;
-      const double d = e.ref_dens *
-                       (e.ptemp_dep * (t[u] - e.ref_temp) + e.press_dep * pr + e.salt_dep * (s[u] - e.ref_salt));
-      const double next = sum + (gh * d) * cdk[k];
-      dens[o + k * npts] = d;
-      hyd[o + k * npts] = 0.5 * (sum + next);
-      sum = next;
-    }
-  }
+  auto layer = [&](int k, double t, double s) {
+    const double geo = e.grav * (e.depth * zck[k]);
+    const double pr = -e.ref_dens * geo;
+    const double d = e.ref_dens * (e.ptemp_dep * (t - e.ref_temp) + e.press_dep * pr + e.salt_dep * (s - e.ref_salt));
+    const double next = sum + (gh * d) * cdk[k];
+    dens[o + k * npts] = d;
+    hyd[o + k * npts] = 0.5 * (sum + next);
+    sum = next;
+  };
+  const double* f[2] = {tp, sp};
+  lf_walk<2, 8>(f, npts, K, 0, 1, [&](int k, const double (&x)[2]) { layer(k, x[0], x[1]); });
 }
 
 // The grid-space part of HBEBaroc_MOMRHS_VorDivForm (HBEBaroc_hspm_vfvm_mod.f90:366-420):
@@ -157,48 +180,31 @@ __global__ __launch_bounds__(256) void k_lf_mom(
   const double sfc = sp[r * np + p];
   double om = 0.0, vau_b = 0.0, vav_b = 0.0;  // omega and vertical advection at the layer's lower half level
   double uk = lf_ld(u + o + (a.K - 1) * np), vk = lf_ld(v + o + (a.K - 1) * np);
-  for (int k0 = a.K - 1; k0 >= 0; k0 -= LG) {
-    double un[LG], vn[LG], x[LG], y[LG], dv[LG], vo[LG], hy[LG], de[LG], gx[LG], gy[LG];
-#pragma unroll
-    for (int q = 0; q < LG; q++) {
-      const long g = o + (k0 - q > 0 ? k0 - q : 0) * np, gn = o + (k0 - q > 1 ? k0 - q - 1 : 0) * np;
-      un[q] = lf_ld(u + gn);
-      vn[q] = lf_ld(v + gn);
-      x[q] = lf_ld(xa + g);
-      y[q] = lf_ld(xb + g);
-      dv[q] = lf_ld(div + g);
-      vo[q] = lf_ld(vor + g);
-      hy[q] = lf_ld(hyd + g);
-      de[q] = lf_ld(dens + g);
-      gx[q] = lf_ld(glon + g);
-      gy[q] = lf_ld(glat + g);
+  // the winds one layer ahead (above); the top layer's are not used
+  const double* fld[10] = {u + o, v + o, xa + o, xb + o, div + o, vor + o, hyd + o, dens + o, glon + o, glat + o};
+  const int above[10] = {1, 1, 0, 0, 0, 0, 0, 0, 0, 0};
+  lf_walk<10, 4>(fld, np, a.K, a.K - 1, -1, [&](int k, const double (&x)[10]) {
+    const long g = o + k * np;
+    om = om - x[4] * (a.depth * cdk[k]);
+    double vau_a = 0.0, vav_a = 0.0;
+    if (k > 0) {
+      vau_a = om * (x[0] - uk) * rfdk[k];
+      vav_a = om * (x[1] - vk) * rfdk[k];
     }
-#pragma unroll
-    for (int q = 0; q < LG; q++) {
-      const int k = k0 - q;
-      if (k < 0) break;
-      const long g = o + k * np;
-      om = om - dv[q] * (a.depth * cdk[k]);
-      double vau_a = 0.0, vav_a = 0.0;
-      if (k > 0) {
-        vau_a = om * (un[q] - uk) * rfdk[k];
-        vav_a = om * (vn[q] - vk) * rfdk[k];
-      }
-      const double coru = PRED ? f * (a.cn * uk + a.cb * x[q]) : f * x[q];
-      const double corv = PRED ? f * (a.cn * vk + a.cb * y[q]) : f * y[q];
-      double A = vo[q] * uk + coru + 0.5 * (vav_b + vav_a) / a.depth;
-      A = cs * (A + de[q] * gy[q] / rr);
-      double B = vo[q] * vk + corv - 0.5 * (vau_b + vau_a) / a.depth;
-      B = cs * (B + de[q] * gx[q] / rr);
-      am[g] = -A;
-      bg[g] = B;
-      cg[g] = (0.5 * (uk * uk + vk * vk) + (hy[q] + sfc) / a.ref_dens) / (a.radius * a.radius);
-      vau_b = vau_a;
-      vav_b = vav_a;
-      uk = un[q];
-      vk = vn[q];
-    }
-  }
+    const double coru = PRED ? f * (a.cn * uk + a.cb * x[2]) : f * x[2];
+    const double corv = PRED ? f * (a.cn * vk + a.cb * x[3]) : f * x[3];
+    double A = x[5] * uk + coru + 0.5 * (vav_b + vav_a) / a.depth;
+    A = cs * (A + x[7] * x[9] / rr);
+    double B = x[5] * vk + corv - 0.5 * (vau_b + vau_a) / a.depth;
+    B = cs * (B + x[7] * x[8] / rr);
+    am[g] = -A;
+    bg[g] = B;
+    cg[g] = (0.5 * (uk * uk + vk * vk) + (x[6] + sfc) / a.ref_dens) / (a.radius * a.radius);
+    vau_b = vau_a;
+    vav_b = vav_a;
+    uk = x[0];
+    vk = x[1];
+  }, above);
 }
 
 // w_out[l, c] += w_in[l, c] * s  (s = 1, or 1/(RefDens R^2) for the barotropic pressure term)
@@ -210,40 +216,67 @@ __global__ void k_lf_spec_axpy(double* __restrict__ wout, long slo, const double
   }
 }
 
-// predictor momentum (DOGCM_TInt_LFAM3_mod.f90:495-517): optional implicit Coriolis with
-// CoriImplFac = 0.5 (2 dt) f, then U = 5/6 dt U_RHS + (2 U_N + U_B)/3
-__global__ void k_lf_pred_uv(const double* __restrict__ urhs, const double* __restrict__ vrhs,
-                             const double* __restrict__ un, const double* __restrict__ ub,
-                             const double* __restrict__ vn, const double* __restrict__ vb,
-                             const double* __restrict__ two_omega, const double* __restrict__ mu, long npts, int I,
-                             int K, double half2dt, double c56dt, int implicit, long ncols, double* __restrict__ uo,
-                             double* __restrict__ vo) {
-  LF_CP(ncols, npts) {
-    const long g = c * npts + p;
-    const long r = c / K;
-    const int j = LF_ROW(p, I);
-    double ur = urhs[g], vr = vrhs[g];
-    if (implicit) {
-      const double cif = half2dt * (two_omega[r] * mu[j]);
-      const double ut = ur;
-      ur = (ut + cif * vr) / (1.0 + cif * cif);
-      vr = (vr - cif * ut) / (1.0 + cif * cif);
-    }
-    uo[g] = c56dt * ur + (2.0 * un[g] + ub[g]) / 3.0;
-    vo[g] = c56dt * vr + (2.0 * vn[g] + vb[g]) / 3.0;
-  }
+// The thickness-weighted layer means of U and V (HBEDiagnose_UVBarot, HBEDiagnose_hspm_vfvm_mod.f90:
+// 246-251) of the time levels N (grid z 0) and B (z 1), one walk each
+struct BarotArgs {
+  const double *u[2], *v[2];
+  double *ub[2], *vb[2];
+};
+__global__ __launch_bounds__(256) void k_lf_uvbarot(BarotArgs a, double depth, const double* __restrict__ cdk, long npts,
+                                                    int K) {
+#pragma clang fp contract(off)
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= npts) return;
+  const long o = (long)blockIdx.y * K * npts + p;
+  const double* __restrict__ u = a.u[blockIdx.z] + o;
+  const double* __restrict__ v = a.v[blockIdx.z] + o;
+  double dep = 0.0, su = 0.0, sv = 0.0;
+  const double* fld[2] = {u, v};
+  lf_walk<2, 8>(fld, npts, K, 0, 1, [&](int k, const double (&x)[2]) {
+    const double f = depth * cdk[k];
+    dep = dep + f;
+    su = su + x[0] * f;
+    sv = sv + x[1] * f;
+  });
+  a.ub[blockIdx.z][blockIdx.y * npts + p] = su / dep;
+  a.vb[blockIdx.z][blockIdx.y * npts + p] = sv / dep;
 }
 
-// x = x - xbar + xbar_ref for every layer (the barotropic part of x replaced, :520-528, 783-793)
-__global__ void k_lf_barot_shift(double* __restrict__ u, double* __restrict__ v, const double* __restrict__ ubt,
-                                 const double* __restrict__ vbt, const double* __restrict__ ubr,
-                                 const double* __restrict__ vbr, long npts, int K, long ncols) {
-  LF_CP(ncols, npts) {
-    const long g = c * npts + p;
-    const long q = (c / K) * npts + p;
-    u[g] = u[g] - ubt[q] + ubr[q];
-    v[g] = v[g] - vbt[q] + vbr[q];
-  }
+// predictor momentum (DOGCM_TInt_LFAM3_mod.f90:495-528): optional implicit Coriolis with
+// CoriImplFac = 0.5 (2 dt) f, U = 5/6 dt U_RHS + (2 U_N + U_B)/3, and U's barotropic part
+// replaced by that of level N.  U's layer mean follows from the means of U_RHS (a first walk)
+// and of U_N and U_B (known), so U itself is written once.
+__global__ __launch_bounds__(256) void k_lf_pred_uv(
+    const double* __restrict__ urhs, const double* __restrict__ vrhs, const double* __restrict__ un,
+    const double* __restrict__ ub, const double* __restrict__ vn, const double* __restrict__ vb,
+    const double* __restrict__ ubn, const double* __restrict__ vbn, const double* __restrict__ ubb,
+    const double* __restrict__ vbb, const double* __restrict__ two_omega, const double* __restrict__ mu, double depth,
+    const double* __restrict__ cdk, long npts, int I, int K, double half2dt, double c56dt, int implicit,
+    double* __restrict__ uo, double* __restrict__ vo) {
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= npts) return;
+  const long r = blockIdx.y, o = r * K * npts + p, q2 = r * npts + p;
+  const double cif = implicit ? half2dt * (two_omega[r] * mu[LF_ROW(p, I)]) : 0.0, den = 1.0 + cif * cif;
+  double dep = 0.0, su = 0.0, sv = 0.0;
+  const double* rhs[2] = {urhs + o, vrhs + o};
+  lf_walk<2, 8, false>(rhs, npts, K, 0, 1, [&](int k, const double (&x)[2]) {
+    const double f = depth * cdk[k];
+    dep = dep + f;
+    su = su + x[0] * f;
+    sv = sv + x[1] * f;
+  });
+  su /= dep;
+  sv /= dep;
+  const double ubr = ubn[q2], vbr = vbn[q2];
+  // barotropic part of level N minus that of U, V
+  const double du = ubr - (c56dt * ((su + cif * sv) / den) + (2.0 * ubr + ubb[q2]) / 3.0);
+  const double dv = vbr - (c56dt * ((sv - cif * su) / den) + (2.0 * vbr + vbb[q2]) / 3.0);
+  const double* fld[6] = {urhs + o, vrhs + o, un + o, ub + o, vn + o, vb + o};
+  lf_walk<6, 4>(fld, npts, K, 0, 1, [&](int k, const double (&x)[6]) {
+    const long g = o + k * npts;
+    uo[g] = (c56dt * ((x[0] + cif * x[1]) / den) + (2.0 * x[2] + x[3]) / 3.0) + du;
+    vo[g] = (c56dt * ((x[1] - cif * x[0]) / den) + (2.0 * x[4] + x[5]) / 3.0) + dv;
+  });
 }
 
 // The grid-space part of HBEBaroc_HTRCRHS (HBEBaroc_hspm_vfvm_mod.f90:162-172) for both tracers
@@ -279,47 +312,35 @@ __global__ __launch_bounds__(256) void k_lf_htrc(const double* __restrict__ ts, 
     t0[tr] = T(tr, K - 1);
     t1[tr] = T(tr, K - 2);
   }
-  for (int k0 = K - 1; k0 >= 0; k0 -= LG) {
-    double tn[2][LG], uu[LG], vv[LG], dv[LG];
+  // the tracers two layers ahead (above)
+  const double* fld[5] = {ts + ot, ts + ot + sec, u + o, v + o, div + o};
+  const int above[5] = {2, 2, 0, 0, 0};
+  lf_walk<5, 4>(fld, npts, K, K - 1, -1, [&](int k, const double (&x)[5]) {
+    const double dz = depth * cdk[k];
+    om = om - x[4] * dz;
 #pragma unroll
-    for (int q = 0; q < LG; q++) {
-      const long g = o + (long)(k0 - q > 0 ? k0 - q : 0) * npts;
-      tn[0][q] = T(0, k0 - q - 2);
-      tn[1][q] = T(1, k0 - q - 2);
-      uu[q] = lf_ld(u + g);
-      vv[q] = lf_ld(v + g);
-      dv[q] = lf_ld(div + g);
-    }
-#pragma unroll
-    for (int q = 0; q < LG; q++) {
-      const int k = k0 - q;
-      if (k < 0) break;
-      const double dz = depth * cdk[k];
-      om = om - dv[q] * dz;
-#pragma unroll
-      for (int tr = 0; tr < 2; tr++) {
-        const double t2 = tn[tr][q];  // T[k-2]
-        double da = 0.0, fl = 0.0;
-        if (k > 0) {
-          const double mid = m1[k] * t1[tr] + m2[k] * t0[tr];
-          if (k >= 2) da = lf_curvature(t2, t1[tr], t0[tr], rfdk[k - 1], rfdk[k]);
-          if (k >= 2 && k <= K - 2)
-            fl = om * (mid - dfac[k] * (da + db[tr])) + (fabs(om) * dfac[k]) * (da - db[tr]);
-          else
-            fl = om * mid;
-        }
-        const double tmp = hc * t0[tr];
-        const long g = ot + tr * sec + k * npts;
-        fu[g] = uu[q] * tmp;
-        fv[g] = vv[q] * tmp;
-        vf[g] = -(fl - fb[tr]) * rcdk[k];
-        fb[tr] = fl;
-        db[tr] = da;
-        t0[tr] = t1[tr];
-        t1[tr] = t2;
+    for (int tr = 0; tr < 2; tr++) {
+      const double t2 = x[tr];  // T[k-2]
+      double da = 0.0, fl = 0.0;
+      if (k > 0) {
+        const double mid = m1[k] * t1[tr] + m2[k] * t0[tr];
+        if (k >= 2) da = lf_curvature(t2, t1[tr], t0[tr], rfdk[k - 1], rfdk[k]);
+        if (k >= 2 && k <= K - 2)
+          fl = om * (mid - dfac[k] * (da + db[tr])) + (fabs(om) * dfac[k]) * (da - db[tr]);
+        else
+          fl = om * mid;
       }
+      const double tmp = hc * t0[tr];
+      const long g = ot + tr * sec + k * npts;
+      fu[g] = x[2] * tmp;
+      fv[g] = x[3] * tmp;
+      vf[g] = -(fl - fb[tr]) * rcdk[k];
+      fb[tr] = fl;
+      db[tr] = da;
+      t0[tr] = t1[tr];
+      t1[tr] = t2;
     }
-  }
+  }, above);
 }
 
 // w = AdvFilter (-w_alpha + w_vert) (HBEBaroc_hspm_vfvm_mod.f90:163-171), in place over w_alpha
@@ -333,81 +354,69 @@ __global__ void k_lf_htrc_spec(double* __restrict__ wa, const double* __restrict
 
 // predictor tracers (:535-541): ((H (2 T_N + T_B))/3 + 5/6 dt HTRC_RHS) / H
 __global__ void k_lf_pred_trc(const double* __restrict__ tn, const double* __restrict__ tb,
-                              const double* __restrict__ ht, const double* __restrict__ h, long npts, int K,
-                              double c56dt, long ncols, double* __restrict__ to) {
-  LF_CP(ncols, npts) {
-    const long g = c * npts + p;
-    const long q = ((c / K) / 2 * K + c % K) * npts + p;
-    const double hh = h[q] + 0.0;
-    to[g] = (hh * (2.0 * tn[g] + tb[g]) / 3.0 + c56dt * ht[g]) / hh;
-  }
+                              const double* __restrict__ ht, double h, double c56dt, long n, double* __restrict__ to) {
+  LF_LOOP(n) to[g] = (h * (2.0 * tn[g] + tb[g]) / 3.0 + c56dt * ht[g]) / h;
 }
 
-// U_RHS = (U_A - U_N)/dt after the implicit solves (:615-619)
-__global__ void k_lf_rhs_diff(const double* __restrict__ ua, const double* __restrict__ un,
-                              const double* __restrict__ va, const double* __restrict__ vn, double dt, long n,
-                              double* __restrict__ ur, double* __restrict__ vr) {
-  LF_LOOP(n) {
-    ur[g] = (ua[g] - un[g]) / dt;
-    vr[g] = (va[g] - vn[g]) / dt;
-  }
+// After the implicit solves (:615-646) and up to the barotropic forcing (HBEBarot_MOMRHS grid
+// part, HBEBarot_hspm_vfvm_mod.f90:197-201), one walk: U_RHS = (U_A - U_N)/dt and its layer
+// mean, the forcing UBarocForce - CoriVBarot, VBarocForce + CoriUBarot with CoriXBarot = f x_N
+// (:626-630), implicit Coriolis with CoriImplFac = alpha_ dt f, U_A = U_N + dt U_RHS and the
+// layer mean of that; -A and B of A = cos (f U - VBarocForce), B = cos (f V + UBarocForce); and
+// SfcPres - SfcPres_N, which is 0 in the one iteration of a rigid lid.
+__global__ __launch_bounds__(256) void k_lf_impl(
+    double* __restrict__ ua, double* __restrict__ va, const double* __restrict__ un, const double* __restrict__ vn,
+    const double* __restrict__ ubn, const double* __restrict__ vbn, const double* __restrict__ pn,
+    const double* __restrict__ two_omega, const double* __restrict__ mu, const double* __restrict__ cosj, double depth,
+    const double* __restrict__ cdk, long npts, int I, int K, double adt, double dt, double* __restrict__ ubt,
+    double* __restrict__ vbt, double* __restrict__ am, double* __restrict__ bg, double* __restrict__ spm) {
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= npts) return;
+  const long r = blockIdx.y, o = r * K * npts + p, q2 = r * npts + p;
+  const int j = LF_ROW(p, I);
+  const double f = two_omega[r] * mu[j], cif = adt * f, den = 1.0 + cif * cif;
+  double dep = 0.0, fu = 0.0, fv = 0.0, su = 0.0, sv = 0.0;
+  const double* fld[4] = {ua + o, va + o, un + o, vn + o};
+  lf_walk<4, 4>(fld, npts, K, 0, 1, [&](int k, const double (&x)[4]) {
+    const long g = o + k * npts;
+    const double w = depth * cdk[k];
+    const double ur = (x[0] - x[2]) / dt, vr = (x[1] - x[3]) / dt;
+    dep += w;
+    fu += ur * w;
+    fv += vr * w;
+    const double u1 = x[2] + dt * ((ur + cif * vr) / den), v1 = x[3] + dt * ((vr - cif * ur) / den);
+    su += u1 * w;
+    sv += v1 * w;
+    ua[g] = u1;
+    va[g] = v1;
+  });
+  ubt[q2] = su / dep;
+  vbt[q2] = sv / dep;
+  const double coru = f * ubn[q2], corv = f * vbn[q2];
+  const double ubf = fu / dep - corv, vbf = fv / dep + coru;
+  am[q2] = -(cosj[j] * (coru - vbf));
+  bg[q2] = cosj[j] * (corv + ubf);
+  spm[q2] = pn[q2] - pn[q2];
 }
 
-// barotropic forcing of the baroclinic tendencies (:626-630): UBarocForce - CoriVBarot,
-// VBarocForce + CoriUBarot, CoriXBarot = f (cn x_N + cb x_B)
-__global__ void k_lf_baroc_force(double* __restrict__ ubf, double* __restrict__ vbf, const double* __restrict__ ubn,
-                                 const double* __restrict__ vbn, const double* __restrict__ ubb,
-                                 const double* __restrict__ vbb, const double* __restrict__ two_omega,
-                                 const double* __restrict__ mu, long npts, int I, double cn, double cb, long nruns) {
-  LF_CP(nruns, npts) {
-    const long g = c * npts + p;
-    const double f = two_omega[c] * mu[LF_ROW(p, I)];
-    const double coru = f * (cn * ubn[g] + cb * ubb[g]);
-    const double corv = f * (cn * vbn[g] + cb * vbb[g]);
-    ubf[g] = ubf[g] - corv;
-    vbf[g] = vbf[g] + coru;
-  }
-}
-
-// implicit Coriolis with CoriImplFac = alpha_ dt f and U_A = U_N + dt U_RHS (:632-646); also the
-// barotropic velocity step of the sub-cycle (:712-721) when the inputs are 2-D
-__global__ void k_lf_cori_step(const double* __restrict__ ur_in, const double* __restrict__ vr_in,
-                               const double* __restrict__ u0, const double* __restrict__ v0,
-                               const double* __restrict__ two_omega, const double* __restrict__ mu, long npts, int I,
-                               int K, double adt, double dt, int form, long ncols, double* __restrict__ uo,
-                               double* __restrict__ vo) {
-  LF_CP(ncols, npts) {
-    const long g = c * npts + p;
-    const double cif = adt * (two_omega[c / K] * mu[LF_ROW(p, I)]);
-    const double ur = ur_in[g], vr = vr_in[g];
-    if (form == 0) {  // baroclinic: the tendency is replaced, then U_A = U_N + dt U_RHS
-      const double u2 = (ur + cif * vr) / (1.0 + cif * cif);
-      const double v2 = (vr - cif * ur) / (1.0 + cif * cif);
-      uo[g] = u0[g] + dt * u2;
-      vo[g] = v0[g] + dt * v2;
-    } else {  // barotropic sub-step: U + dts (U_RHS + c V_RHS)/(1 + c^2)
-      uo[g] = u0[g] + dt * (ur + cif * vr) / (1.0 + cif * cif);
-      vo[g] = v0[g] + dt * (vr - cif * ur) / (1.0 + cif * cif);
-    }
-  }
-}
-
-// HBEBarot_MOMRHS grid part (HBEBarot_hspm_vfvm_mod.f90:197-201): -A and B with
-// A = cos (f U - VBarocForce), B = cos (f V + UBarocForce); and SfcPres - SfcPres_N
-__global__ void k_lf_barot_rhs_grid(const double* __restrict__ ub, const double* __restrict__ vb,
-                                    const double* __restrict__ ubf, const double* __restrict__ vbf,
-                                    const double* __restrict__ sp, const double* __restrict__ spn,
-                                    const double* __restrict__ two_omega, const double* __restrict__ mu,
-                                    const double* __restrict__ cs, long npts, int I, long nruns, double* __restrict__ am,
-                                    double* __restrict__ bg, double* __restrict__ spm) {
+// The barotropic velocity step of the sub-cycle (:712-721), U + dts (U_RHS + c V_RHS)/(1 + c^2),
+// and the result times cos phi
+__global__ void k_lf_barot_step(const double* __restrict__ ur_in, const double* __restrict__ vr_in,
+                                const double* __restrict__ u0, const double* __restrict__ v0,
+                                const double* __restrict__ two_omega, const double* __restrict__ mu,
+                                const double* __restrict__ cosj, long npts, int I, double adt, double dt, long nruns,
+                                double* __restrict__ uo, double* __restrict__ vo, double* __restrict__ uc,
+                                double* __restrict__ vc) {
   LF_CP(nruns, npts) {
     const long g = c * npts + p;
     const int j = LF_ROW(p, I);
-    const double f = two_omega[c] * mu[j];
-    const double coru = f * ub[g], corv = f * vb[g];
-    am[g] = -(cs[j] * (coru - vbf[g]));
-    bg[g] = cs[j] * (corv + ubf[g]);
-    spm[g] = sp[g] - spn[g];
+    const double cif = adt * (two_omega[c] * mu[j]), ur = ur_in[g], vr = vr_in[g];
+    const double u = u0[g] + dt * (ur + cif * vr) / (1.0 + cif * cif);
+    const double v = v0[g] + dt * (vr - cif * ur) / (1.0 + cif * cif);
+    uo[g] = u;
+    vo[g] = v;
+    uc[g] = u * cosj[j];
+    vc[g] = v * cosj[j];
   }
 }
 
@@ -424,33 +433,50 @@ __global__ void k_lf_barot_proj(const double* __restrict__ wdiv, long sld, const
   }
 }
 
-__global__ void k_lf_add2(const double* __restrict__ a, const double* __restrict__ da, const double* __restrict__ b,
-                          const double* __restrict__ db, const double* __restrict__ c, const double* __restrict__ dc,
-                          long n, double* __restrict__ ao, double* __restrict__ bo, double* __restrict__ co) {
-  LF_LOOP(n) {
-    ao[g] = a[g] + da[g];
-    bo[g] = b[g] + db[g];
-    co[g] = c[g] + dc[g];
-  }
-}
-
-// full velocity and the time-centred fields of the tracer update (:783-795):
-// U_A = U_A - UBarot + UBarot_A; U = (5 U_A + 8 U_N - U_B)/12
-__global__ void k_lf_final_uv(double* __restrict__ ua, double* __restrict__ va, const double* __restrict__ ubt,
-                              const double* __restrict__ vbt, const double* __restrict__ uba,
-                              const double* __restrict__ vba, const double* __restrict__ un,
-                              const double* __restrict__ ub, const double* __restrict__ vn,
-                              const double* __restrict__ vb, long npts, int K, long ncols,
-                              double* __restrict__ uo, double* __restrict__ vo) {
+// The barotropic correction (UBarot + dUBarot, SfcPres + dSfcPres), the full velocity and the
+// time-centred winds of the tracer update (:783-795), U_A = U_A - UBarot + UBarot_A,
+// U = (5 U_A + 8 U_N - U_B)/12, and the time levels of momentum and pressure (B <- N, N <- A),
+// which nothing later in the step reads
+struct FinalArgs {
+  double *ua, *un, *ub, *uo;              // U: levels A, N, B; the time-centred wind
+  double *va, *vn, *vb, *vo;
+  const double *ubt, *vbt;                // layer means to take out
+  const double *ubar, *du, *vbar, *dv;    // barotropic velocity and its correction
+  const double* dsp;
+  double *pa, *pn, *pb;                   // surface pressure: levels A, N, B
+};
+__global__ void k_lf_final_uv(FinalArgs a, long npts, int K, long ncols) {
   LF_CP(ncols, npts) {
     const long g = c * npts + p;
     const long q = (c / K) * npts + p;
-    const double a = ua[g] - ubt[q] + uba[q];
-    const double b = va[g] - vbt[q] + vba[q];
-    ua[g] = a;
-    va[g] = b;
-    uo[g] = (5.0 * a + 8.0 * un[g] - ub[g]) / 12.0;
-    vo[g] = (5.0 * b + 8.0 * vn[g] - vb[g]) / 12.0;
+    const double u0 = a.un[g], v0 = a.vn[g];
+    const double u = a.ua[g] - a.ubt[q] + (a.ubar[q] + a.du[q]);
+    const double v = a.va[g] - a.vbt[q] + (a.vbar[q] + a.dv[q]);
+    a.uo[g] = (5.0 * u + 8.0 * u0 - a.ub[g]) / 12.0;
+    a.vo[g] = (5.0 * v + 8.0 * v0 - a.vb[g]) / 12.0;
+    a.ua[g] = u;
+    a.va[g] = v;
+    a.ub[g] = u0;
+    a.vb[g] = v0;
+    a.un[g] = u;
+    a.vn[g] = v;
+    if (c % K == 0) {
+      const double s0 = a.pn[q], s = s0 + a.dsp[q];
+      a.pa[q] = s;
+      a.pb[q] = s0;
+      a.pn[q] = s;
+    }
+  }
+}
+
+// T_A = H_0 T_A / H_A (DOGCM_Phys_hspm_vfvm_mod.f90:641) and the tracers' time levels
+__global__ void k_lf_trc_final(double* __restrict__ ta, double* __restrict__ tn, double* __restrict__ tb, double h,
+                               long n) {
+  LF_LOOP(n) {
+    const double t = h * ta[g] / h;
+    tb[g] = tn[g];
+    ta[g] = t;
+    tn[g] = t;
   }
 }
 
@@ -464,11 +490,11 @@ __global__ void k_lf_final_uv(double* __restrict__ ua, double* __restrict__ va, 
 // and a workspace of the general k_col_vdiff: at T170L60 two fields take 67 us (5.6 TB/s), there
 // 163; loading each group only when it is worked on took 111.  Grid y: sections of K layers,
 // grid z: field pairs.
+constexpr int VL = 8;  // layers whose loads are in flight together
 struct VSolve {
   const double *q0[2], *rhs[2];
   double* qa[2];
 };
-constexpr int VL = 8;  // layers whose loads are in flight together
 template <int KM, bool MOM>
 __global__ __launch_bounds__(256) void k_lf_vsolve(VSolve a, const double* __restrict__ fact,
                                                    const double* __restrict__ dd, const double* __restrict__ du,
@@ -545,23 +571,6 @@ __global__ __launch_bounds__(256) void k_lf_vsolve(VSolve a, const double* __res
   }
 }
 
-// T_A = H_0 T_A / H_A (DOGCM_Phys_hspm_vfvm_mod.f90:641)
-__global__ void k_lf_trc_final(double* __restrict__ ta, const double* __restrict__ h, long npts, int K, long ncols) {
-  LF_CP(ncols, npts) {
-    const long g = c * npts + p;
-    const long q = ((c / K) / 2 * K + c % K) * npts + p;
-    ta[g] = h[q] * ta[g] / h[q];
-  }
-}
-
-// time levels: B <- N, N <- A
-__global__ void k_lf_rotate(double* __restrict__ b, double* __restrict__ nn, const double* __restrict__ a, long n) {
-  LF_LOOP(n) {
-    b[g] = nn[g];
-    nn[g] = a[g];
-  }
-}
-
 }  // namespace
 }  // namespace dsht
 
@@ -580,7 +589,6 @@ struct dsht_lfam3 {
   double *d_m1 = nullptr, *d_m2 = nullptr, *d_dfac = nullptr;  // QUICK weights per half level
   double *d_dmom = nullptr, *d_dtrc = nullptr, *d_advf = nullptr, *d_nn1 = nullptr, *d_hcoef = nullptr,
          *d_e = nullptr;
-  double* H = nullptr;
   // state: levels B (0), N (1), A (2)
   double *U[3] = {}, *V[3] = {}, *TS[3] = {}, *SP[3] = {};
   // work
@@ -588,7 +596,7 @@ struct dsht_lfam3 {
   double *Geo = nullptr, *GLon = nullptr, *GLat = nullptr, *Am = nullptr, *Bg = nullptr, *Cg = nullptr;
   double *URHS = nullptr, *VRHS = nullptr, *Upr = nullptr, *Vpr = nullptr;
   double *TSpr = nullptr, *HT = nullptr, *FU = nullptr, *FV = nullptr, *VF = nullptr;
-  double *b2[20] = {};  // 2-D barotropic work, one grid per run each
+  double* b2[16] = {};  // 2-D barotropic work, one grid per run each
   double *wVD = nullptr, *wGeo = nullptr, *wC = nullptr, *w1 = nullptr, *w2 = nullptr;
   double *wB = nullptr, *wC2 = nullptr, *wDSP = nullptr, *wDDiv = nullptr, *wZero = nullptr;
   // the elimination of the constant vertical systems (momentum, tracers): fact, d, du, du2 and
@@ -599,7 +607,7 @@ struct dsht_lfam3 {
 
 namespace {
 
-enum B2 { UBN, VBN, UBB, VBB, UBT, VBT, UBF, VBF, UBR, VBR, UBAR, VBAR, UBA, VBA, DU, DV, DSP, SPM, AM2, BG2 };
+enum B2 { UBN, VBN, UBB, VBB, UBT, VBT, UBR, VBR, UBAR, VBAR, DU, DV, DSP, SPM, AM2, BG2, B2_COUNT };
 
 int lf_alloc(dsht_lfam3* s, double** out, size_t n) {
   void* ptr = nullptr;
@@ -636,23 +644,15 @@ void lf_free(dsht_lfam3* s) {
     DSHT_HIP(hipGetLastError());                                                         \
   } while (0)
 
-// column walks over the points of nr runs
-#define LF_LAUNCHC(kernel, npts, nr, s, ...)                                                  \
+// column walks over the points of nr runs and nz field sets
+#define LF_LAUNCHC(kernel, npts, nr, nz, s, ...)                                              \
   do {                                                                                        \
-    const int th_ = lf_threads(npts, nr);                                                     \
-    hipLaunchKernelGGL(kernel, lf_gridc(npts, nr, th_), dim3(th_), 0, s, __VA_ARGS__);        \
+    const int th_ = lf_threads(npts, (nr) * (nz));                                            \
+    dim3 grid_ = lf_gridc(npts, nr, th_);                                                     \
+    grid_.z = nz;                                                                             \
+    hipLaunchKernelGGL(kernel, grid_, dim3(th_), 0, s, __VA_ARGS__);                          \
     DSHT_HIP(hipGetLastError());                                                              \
   } while (0)
-
-// ---- the reference's diagnostics on every active run (column kernels)
-int lf_uvbarot(dsht_lfam3* s, const double* u, const double* v, double* ub, double* vb, int nr, hipStream_t st) {
-  const long np = s->np, K = s->K;
-  for (int r = 0; r < nr; r++)
-    if (int rc = launch_col_uvbarot(u + r * K * np, v + r * K * np, s->H + r * K * np, np, s->K, s->d_cdk,
-                                    ub + r * np, vb + r * np, (int)np, st))
-      return rc;
-  return 0;
-}
 
 // DGTSV's elimination (LAPACK 3.x SRC/dgtsv.f, partial pivoting by row interchange) of the
 // constant vertical system of momentum or of the tracers (rows as k_col_vdiff builds them):
@@ -742,8 +742,8 @@ int lf_mom_rhs(dsht_lfam3* s, const double* u, const double* v, const double* xa
   if (int rc = dsht_inv_vgrad_d(p, s->wGeo, nc, 1, nullptr, s->GLon, s->GLat, s->np, nc, nullptr, st)) return rc;
   const MomArgs a{s->cfg.ref_dens, p->R, s->cfg.depth, cn, cb, s->np, s->I, s->K};
   auto k = pred ? k_lf_mom<true> : k_lf_mom<false>;
-  LF_LAUNCHC(k, s->np, nr, st, a, u, v, xa, xb, s->VD + (long)nc * s->np, s->VD, s->Hyd, s->Dens, s->GLon, s->GLat, sp,
-             s->d_two_omega, s->d_mu, s->d_cs, s->d_cdk, s->d_rfdk, s->Am, s->Bg, s->Cg);
+  LF_LAUNCHC(k, s->np, nr, 1, st, a, u, v, xa, xb, s->VD + (long)nc * s->np, s->VD, s->Hyd, s->Dens, s->GLon, s->GLat,
+             sp, s->d_two_omega, s->d_mu, s->d_cs, s->d_cdk, s->d_rfdk, s->Am, s->Bg, s->Cg);
   // (w_Vor_RHS, w_Div_RHS) = (-H(A, B), H(B, -A)) = calc_UVCosLat2VorDiv(B, -A); then
   // w_Div_RHS - w_Lapla_w(w_xy(C)) = + n(n+1) w_xy(C)
   if (int rc = dsht_uv2vordiv_d(p, s->Bg, s->Am, s->np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, nullptr, st)) return rc;
@@ -758,7 +758,7 @@ int lf_htrc(dsht_lfam3* s, const double* ts, const double* u, const double* v, d
   dsht_plan* p = s->p;
   const long np = s->np;
   const int nc = nr * s->K, nt = 2 * nc;
-  LF_LAUNCHC(k_lf_htrc, np, nr, st, ts, u, v, s->VD + (long)nc * np, s->cfg.depth, h, s->d_cs, s->d_cdk, s->d_rcdk,
+  LF_LAUNCHC(k_lf_htrc, np, nr, 1, st, ts, u, v, s->VD + (long)nc * np, s->cfg.depth, h, s->d_cs, s->d_cdk, s->d_rcdk,
              s->d_rfdk, s->d_m1, s->d_m2, s->d_dfac, np, s->I, s->K, s->FU, s->FV, s->VF);
   if (int rc = dsht_alpha_fwd_d(p, s->FU, s->FV, np, s->w1, nt, 1, nt, nullptr, st)) return rc;
   if (int rc = dsht_fwd_d(p, DSHT_VAL, s->VF, np, s->w2, nt, 1, nt, nullptr, st)) return rc;
@@ -892,7 +892,6 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
   A(&s->d_dmom, L);
   A(&s->d_dtrc, L);
   A(&s->d_advf, L);
-  A(&s->H, NC * np);
   for (int lv = 0; lv < 3; lv++) {
     A(&s->U[lv], NC * np);
     A(&s->V[lv], NC * np);
@@ -952,8 +951,7 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
     DSHT_HIP(hipGetLastError());
     return 0;
   };
-  // xyz_H = D; the state starts at zero
-  if (!rc) rc = fill(s->H, c.depth, NC * np);
+  // the state starts at zero
   if (!rc) rc = fill(s->wZero, 0.0, (long)L * R);
   for (int lv = 0; lv < 3 && !rc; lv++) {
     rc = fill(s->U[lv], 0.0, NC * np);
@@ -1052,7 +1050,7 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   const int K = s->K, I = s->I, L = s->L;
   const long np = s->np;
   const int nc = nr * K, nt = 2 * nc;
-  const long n = (long)nc * np, ntr = (long)nt * np, n2 = (long)nr * np;
+  const long ntr = (long)nt * np;
   const double dt = c.dt;
   const double gamma = 1.0 - 2.0 * c.alpha;
   const double c56dt = 5.0 / 6.0 * dt;
@@ -1063,8 +1061,8 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   double *PN = s->SP[1], *PA = s->SP[2];
   int rc;
   // ---- preparation: barotropic velocities of levels N and B
-  if ((rc = lf_uvbarot(s, UN, VN, b2[UBN], b2[VBN], nr, st))) return rc;
-  if ((rc = lf_uvbarot(s, UB, VB, b2[UBB], b2[VBB], nr, st))) return rc;
+  const BarotArgs ba{{UN, UB}, {VN, VB}, {b2[UBN], b2[UBB]}, {b2[VBN], b2[VBB]}};
+  LF_LAUNCHC(k_lf_uvbarot, np, nr, 2, st, ba, c.depth, s->d_cdk, np, K);
   // ---- predictor
   if ((rc = lf_vordiv(s, UN, VN, nc, st))) return rc;
   EosArgs ea;
@@ -1076,17 +1074,16 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   ea.ref_salt = c.ref_salt;
   ea.depth = c.depth;
   ea.grav = c.grav;
-  LF_LAUNCHC(k_lf_eos_hyd, np, nr, st, TN, np, K, s->d_zck, s->d_cdk, ea, s->Dens, s->Hyd);
+  LF_LAUNCHC(k_lf_eos_hyd, np, nr, 1, st, TN, np, K, s->d_zck, s->d_cdk, ea, s->Dens, s->Hyd);
   if ((rc = lf_mom_rhs(s, UN, VN, UB, VB, true, gamma, 1.0 - gamma, PN, nr, st))) return rc;
-  LF_LAUNCH2(k_lf_pred_uv, nc, np, st, s->URHS, s->VRHS, UN, UB, VN, VB, s->d_two_omega, s->d_mu, np, I, K,
-             0.5 * (2.0 * dt), c56dt, c.alpha > 0.0 ? 1 : 0, (long)nc, s->Upr, s->Vpr);
-  if ((rc = lf_uvbarot(s, s->Upr, s->Vpr, b2[UBT], b2[VBT], nr, st))) return rc;
-  LF_LAUNCH2(k_lf_barot_shift, nc, np, st, s->Upr, s->Vpr, b2[UBT], b2[VBT], b2[UBN], b2[VBN], np, K, (long)nc);
+  LF_LAUNCHC(k_lf_pred_uv, np, nr, 1, st, s->URHS, s->VRHS, UN, UB, VN, VB, b2[UBN], b2[VBN], b2[UBB], b2[VBB],
+             s->d_two_omega, s->d_mu, c.depth, s->d_cdk, np, I, K, 0.5 * (2.0 * dt), c56dt, c.alpha > 0.0 ? 1 : 0,
+             s->Upr, s->Vpr);
   if ((rc = lf_htrc(s, TN, UN, VN, c.depth, nr, st))) return rc;
-  LF_LAUNCH2(k_lf_pred_trc, nt, np, st, TN, TB, s->HT, s->H, np, K, c56dt, (long)nt, s->TSpr);
+  LF_LAUNCH(k_lf_pred_trc, ntr, st, TN, TB, s->HT, c.depth + 0.0, c56dt, ntr, s->TSpr);
   // ---- corrector
   if ((rc = lf_vordiv(s, s->Upr, s->Vpr, nc, st))) return rc;
-  LF_LAUNCHC(k_lf_eos_hyd, np, nr, st, s->TSpr, np, K, s->d_zck, s->d_cdk, ea, s->Dens, s->Hyd);
+  LF_LAUNCHC(k_lf_eos_hyd, np, nr, 1, st, s->TSpr, np, K, s->d_zck, s->d_cdk, ea, s->Dens, s->Hyd);
   const double alpha_ = 0.5, gamma_ = 0.5;
   const double cn = gamma_ + alpha_, cb = 1.0 - alpha_ - gamma_;  // 1 and 0: the present level alone
   if ((rc = lf_mom_rhs(s, s->Upr, s->Vpr, UN, VN, false, cn, cb, PN, nr, st))) return rc;
@@ -1096,34 +1093,27 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   LF_LAUNCH2(k_lf_uvcos, nc, np, st, UA, VA, s->d_cs, np, I, (long)nc, s->ucos, s->vcos);
   if ((rc = dsht_uv2vordiv_d(p, s->ucos, s->vcos, np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, s->d_dmom, st))) return rc;
   if ((rc = dsht_vordiv2uv_d(p, s->wVD, s->wVD + nc, 2l * nc, 1, UA, VA, np, nc, st))) return rc;
-  LF_LAUNCH(k_lf_rhs_diff, n, st, UA, UN, VA, VN, dt, n, s->URHS, s->VRHS);
-  if ((rc = lf_uvbarot(s, s->URHS, s->VRHS, b2[UBF], b2[VBF], nr, st))) return rc;
-  LF_LAUNCH2(k_lf_baroc_force, nr, np, st, b2[UBF], b2[VBF], b2[UBN], b2[VBN], b2[UBB], b2[VBB], s->d_two_omega,
-             s->d_mu, np, I, cn, cb, (long)nr);
-  LF_LAUNCH2(k_lf_cori_step, nc, np, st, s->URHS, s->VRHS, UN, VN, s->d_two_omega, s->d_mu, np, I, K, alpha_ * dt, dt, 0,
-             (long)nc, UA, VA);
+  LF_LAUNCHC(k_lf_impl, np, nr, 1, st, UA, VA, UN, VN, b2[UBN], b2[VBN], PN, s->d_two_omega, s->d_mu, s->d_cs, c.depth,
+             s->d_cdk, np, I, K, alpha_ * dt, dt, b2[UBT], b2[VBT], b2[AM2], b2[BG2], b2[SPM]);
   // ---- barotropic mode: one iteration with dts = dt / SubCycleNum (rigid lid)
   const double dts = dt / c.sub_cycles;
-  LF_LAUNCH2(k_lf_barot_rhs_grid, nr, np, st, b2[UBN], b2[VBN], b2[UBF], b2[VBF], PN, PN, s->d_two_omega, s->d_mu,
-             s->d_cs, np, I, (long)nr, b2[AM2], b2[BG2], b2[SPM]);
   if ((rc = dsht_uv2vordiv_d(p, b2[BG2], b2[AM2], np, s->wB, s->wB + nr, 2l * nr, 1, nr, nullptr, st))) return rc;
   if ((rc = dsht_fwd_d(p, DSHT_VAL, b2[SPM], np, s->wC2, nr, 1, nr, s->d_nn1, st))) return rc;
   LF_LAUNCH2(k_lf_spec_axpy, L, nr, st, s->wB + nr, 2l * nr, s->wC2, (long)nr, L, nr, c.ref_dens * (p->R * p->R), 1);
   if ((rc = dsht_vordiv2uv_d(p, s->wB, s->wB + nr, 2l * nr, 1, b2[UBR], b2[VBR], np, nr, st))) return rc;
-  LF_LAUNCH2(k_lf_cori_step, nr, np, st, b2[UBR], b2[VBR], b2[UBN], b2[VBN], s->d_two_omega, s->d_mu, np, I, 1,
-             alpha_ * dts, dts, 1, (long)nr, b2[UBAR], b2[VBAR]);
+  LF_LAUNCH2(k_lf_barot_step, nr, np, st, b2[UBR], b2[VBR], b2[UBN], b2[VBN], s->d_two_omega, s->d_mu, s->d_cs, np, I,
+             alpha_ * dts, dts, (long)nr, b2[UBAR], b2[VBAR], b2[AM2], b2[BG2]);
   // HBEBarot_Update_LinFreeSfc, rigid lid: project onto the divergence-free part
-  LF_LAUNCH2(k_lf_uvcos, nr, np, st, b2[UBAR], b2[VBAR], s->d_cs, np, I, (long)nr, b2[AM2], b2[BG2]);
   if ((rc = dsht_uv2vordiv_d(p, b2[AM2], b2[BG2], np, s->wB, s->wB + nr, 2l * nr, 1, nr, nullptr, st))) return rc;
   LF_LAUNCH2(k_lf_barot_proj, L, nr, st, s->wB + nr, 2l * nr, s->d_hcoef, s->d_e, c.ref_dens, alpha_ * dts, L, nr,
              s->wDSP, s->wDDiv);
   if ((rc = dsht_inv_d(p, DSHT_VAL, s->wDSP, nr, 1, b2[DSP], np, nr, nullptr, st))) return rc;
   if ((rc = dsht_vordiv2uv_d(p, s->wZero, s->wDDiv, nr, 1, b2[DU], b2[DV], np, nr, st))) return rc;
-  LF_LAUNCH(k_lf_add2, n2, st, b2[UBAR], b2[DU], b2[VBAR], b2[DV], PN, b2[DSP], n2, b2[UBA], b2[VBA], PA);
-  // ---- full velocity, time-centred fields, tracers
-  if ((rc = lf_uvbarot(s, UA, VA, b2[UBT], b2[VBT], nr, st))) return rc;
-  LF_LAUNCH2(k_lf_final_uv, nc, np, st, UA, VA, b2[UBT], b2[VBT], b2[UBA], b2[VBA], UN, UB, VN, VB, np, K, (long)nc,
-             s->Upr, s->Vpr);
+  // ---- full velocity, time-centred fields, momentum's time levels
+  const FinalArgs fa{UA, UN, UB, s->Upr, VA, VN, VB, s->Vpr, b2[UBT], b2[VBT], b2[UBAR], b2[DU], b2[VBAR], b2[DV],
+                     b2[DSP], PA, PN, s->SP[0]};
+  LF_LAUNCH2(k_lf_final_uv, nc, np, st, fa, np, K, (long)nc);
+  // ---- tracers
   if ((rc = lf_vordiv(s, s->Upr, s->Vpr, nc, st))) return rc;
   const double hm = (5.0 * c.depth + 8.0 * c.depth - c.depth) / 12.0;  // the time-centred thickness factor
   if ((rc = lf_htrc(s, s->TSpr, s->Upr, s->Vpr, hm, nr, st))) return rc;
@@ -1131,12 +1121,7 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   if ((rc = lf_vsolve(s, false, VSolve{{TN, nullptr}, {s->HT, nullptr}, {TA, nullptr}}, 2 * nr, 1, st))) return rc;
   if ((rc = dsht_fwd_d(p, DSHT_VAL, TA, np, s->w1, nt, 1, nt, s->d_dtrc, st))) return rc;
   if ((rc = dsht_inv_d(p, DSHT_VAL, s->w1, nt, 1, TA, np, nt, nullptr, st))) return rc;
-  LF_LAUNCH2(k_lf_trc_final, nt, np, st, TA, s->H, np, K, (long)nt);
-  // ---- time levels
-  LF_LAUNCH(k_lf_rotate, n, st, UB, UN, UA, n);
-  LF_LAUNCH(k_lf_rotate, n, st, VB, VN, VA, n);
-  LF_LAUNCH(k_lf_rotate, ntr, st, TB, TN, TA, ntr);
-  LF_LAUNCH(k_lf_rotate, n2, st, s->SP[0], PN, PA, n2);
+  LF_LAUNCH(k_lf_trc_final, ntr, st, TA, TN, TB, c.depth, ntr);
   return 0;
 }
 
