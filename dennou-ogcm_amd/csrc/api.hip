@@ -133,7 +133,7 @@ static int check_plan(const dsht_plan* p) {
 // forward family: grids -> spectra
 static int run_fwd(dsht_plan* p, int op, const double* in0, const double* in1, long ldg, double* out0,
                    double* out1, long sl, long sc, int ncols, const double* diag0, const double* diag1,
-                   double scale, const double* cw, hipStream_t s) {
+                   double scale, const double* cw, hipStream_t s, const double* rowscale = nullptr) {
   if (ncols <= 0) return 0;
   const int nin = (op == F_ALPHA || op == F_UV2VORDIV) ? 2 : 1;
   const int ch = chunk_cols(p, ncols);
@@ -147,8 +147,9 @@ static int run_fwd(dsht_plan* p, int op, const double* in0, const double* in1, l
     double2* G0 = (double2*)wl.buf;
     double2* G1 = G0 + (size_t)(p->N + 1) * p->J * fourier_pitch(ch);
     const long gp = fourier_pitch(nc);
-    if ((rc = launch_fft_fwd(p, in0 + (long)c0 * ldg, ldg, nc, G0, gp, s))) return rc;
-    if (nin > 1 && (rc = launch_fft_fwd(p, in1 + (long)c0 * ldg, ldg, nc, G1, gp, s))) return rc;
+    const double* xs[2] = {in0 + (long)c0 * ldg, nin > 1 ? in1 + (long)c0 * ldg : nullptr};
+    double2* const gs[2] = {G0, G1};
+    if ((rc = launch_fft_fwd(p, xs, nin, ldg, nc, gs, gp, s, rowscale))) return rc;
     LegFwdArgs a;
     a.G0 = G0;
     a.G1 = nin > 1 ? G1 : nullptr;
@@ -214,7 +215,7 @@ static int run_inv(dsht_plan* p, int op, const double* in0, const double* in1, l
     a.sc = sc;
     // fused value/gradient: GradLon comes from the value's Fourier coefficients through the
     // derivative inverse FFT (i m X_m, 1/cos row scale), so the contraction writes two outputs
-    const bool dlon = op == I_VGRAD && out1 && fft_inv_deriv_ok(p);
+    const bool dlon = op == I_VGRAD && out1 && fft_reg_ok(p);
     a.G0 = out0 || dlon ? G0 : nullptr;
     a.G1 = nout > 1 && out1 && !dlon ? G1 : nullptr;
     a.G2 = nout > 2 && out2 ? G2 : nullptr;
@@ -231,16 +232,32 @@ static int run_inv(dsht_plan* p, int op, const double* in0, const double* in1, l
     a.J2 = p->J2;
     a.J2pad = p->J2pad;
     if ((rc = launch_leg_inv(p, op, a, s))) return rc;
-    hipStream_t fs = s;
     // the field and its longitude derivative as two launches over the same G0: the FP64
     // dual kernel (one read of G0, coefficients held in registers across both passes) ran
     // slower at T170L60 (2 x 125 against 2 x 80 us per step's worth), the FP32 one faster
-    if (out0 && (rc = launch_fft_inv(p, G0, a.gld, nc, out0 + (long)c0 * ldg, ldg, fs))) return rc;
-    if (dlon && (rc = launch_fft_inv(p, G0, a.gld, nc, out1 + (long)c0 * ldg, ldg, fs, p->d_rs_icos, 1))) return rc;
-    if (a.G1 && (rc = launch_fft_inv(p, G1, a.gld, nc, out1 + (long)c0 * ldg, ldg, fs))) return rc;
-    if (a.G2 && (rc = launch_fft_inv(p, G2, a.gld, nc, out2 + (long)c0 * ldg, ldg, fs))) return rc;
+    const double2* gs[3];
+    double* xs[3];
+    int nf = 0;
+    auto add = [&](const double2* g, double* x) {
+      gs[nf] = g;
+      xs[nf++] = x + (long)c0 * ldg;
+    };
+    if (out0) add(G0, out0);
+    if (a.G1) add(G1, out1);
+    if (a.G2) add(G2, out2);
+    if (nf && (rc = launch_fft_inv(p, gs, nf, a.gld, nc, xs, ldg, s))) return rc;
+    nf = 0;
+    if (dlon) add(G0, out1);
+    if (nf && (rc = launch_fft_inv(p, gs, nf, a.gld, nc, xs, ldg, s, p->d_rs_icos, 1))) return rc;
   }
   return 0;
+}
+
+bool uv_scaled_ok(const dsht_plan* p) { return p->prec == DSHT_PREC_FP64 && fft_reg_ok(p); }
+
+int uv2vordiv_scaled(dsht_plan* p, const double* u, const double* v, const double* rowscale, long ldg, double* vor,
+                     double* div, long sl, long sc, int ncols, const double* diag, hipStream_t s) {
+  return run_fwd(p, F_UV2VORDIV, u, v, ldg, vor, div, sl, sc, ncols, diag, diag, 1.0 / p->R, p->d_cwd, s, rowscale);
 }
 
 static int check_grid_ptr(const void* x, long ldg, const dsht_plan* p) {

@@ -107,6 +107,8 @@ struct FftPlan {
   float2* twI32 = nullptr;
 };
 
+constexpr int FFT_FIELDS_MAX = 3;
+
 struct FftArgs {
   int I, M, N, J;
   int ncols;
@@ -117,13 +119,17 @@ struct FftArgs {
   const double2* twM;
   const double2* twI;
   int rows_per_block;
-  const double* rowscale;  // optional per-latitude scale applied after the inverse (nullable)
+  const double* rowscale;  // optional per-latitude scale: of the inverse's output, of the FP64 forward's
+                           // input (nullable)
   int threads;             // workgroup size of the register kernels (128 or 256)
   int fp32;                // FP32 arithmetic (FP32 Fourier path of the split forms)
   int order;               // row-group order of the register kernels (0 packed, 1 latitude-major)
   int deriv;               // inverse: transform i m X_m (longitude derivative) instead of X_m
   void* xy2;               // inverse, dual form: the field into xy and its longitude derivative
                            // (times rowscale) into xy2 from one read of the coefficients (nullable)
+  int nf;                  // fields in one launch (FP64 register kernels; grid y), each of ncols columns
+  const void* more_in[FFT_FIELDS_MAX - 1];  // inputs and outputs of fields 1 .. nf-1
+  void* more_out[FFT_FIELDS_MAX - 1];
 };
 
 // ---------------------------------------------------------------- workspace
@@ -222,6 +228,11 @@ int fail(int code, const char* fmt, ...);
                           hipGetErrorString(e_));                                 \
   } while (0)
 
+// api.hip: calc_UVCosLat2VorDiv of (u rowscale, v rowscale), the row factor (J, device) applied as
+// the FFT reads the grids; FP64 form with a register FFT only (uv_scaled_ok)
+bool uv_scaled_ok(const dsht_plan* p);
+int uv2vordiv_scaled(dsht_plan* p, const double* u, const double* v, const double* rowscale, long ldg, double* vor,
+                     double* div, long sl, long sc, int ncols, const double* diag, hipStream_t s);
 // api.hip: per-stream scratch
 int workspace_acquire(dsht_plan* p, hipStream_t s, size_t bytes, WsHandle& out);
 // tables.hip
@@ -229,15 +240,15 @@ int build_tables(dsht_plan* p);
 // fft.hip
 int fft_plan_init(dsht_plan* p);
 void fft_plan_free(dsht_plan* p);
-int launch_fft_fwd(const dsht_plan* p, const double* xy, long ldg, int ncols, double2* G, long gld,
-                   hipStream_t s);
-// rowscale: per-latitude factor on the output (nullable); deriv: transform i m X_m (the
-// longitude derivative of the field), register kernels only (fft_inv_deriv_ok)
-bool fft_inv_deriv_ok(const dsht_plan* p);
-// xy2 (dual form, register kernels only): xy receives the field and xy2 its longitude
-// derivative times rowscale, from one read of the coefficients
-int launch_fft_inv(const dsht_plan* p, const double2* G, long gld, int ncols, double* xy, long ldg,
-                   hipStream_t s, const double* rowscale = nullptr, int deriv = 0, double* xy2 = nullptr);
+// FP64 FFTs of nf fields (one launch where a register kernel exists); rowscale: per-latitude
+// factor on the inputs (nullable; register kernels only: fft_reg_ok)
+int launch_fft_fwd(const dsht_plan* p, const double* const* xy, int nf, long ldg, int ncols, double2* const* G, long gld,
+                   hipStream_t s, const double* rowscale = nullptr);
+// rowscale: per-latitude factor on the outputs (nullable); deriv: transform i m X_m (the
+// longitude derivative of the field), register kernels only
+bool fft_reg_ok(const dsht_plan* p);
+int launch_fft_inv(const dsht_plan* p, const double2* const* G, int nf, long gld, int ncols, double* const* xy, long ldg,
+                   hipStream_t s, const double* rowscale = nullptr, int deriv = 0);
 // FP32 Fourier intermediates of the split-precision forms; colmax (nullable) receives the
 // per-column max |G| as float bits
 bool reg_fft_supported(int M);

@@ -455,6 +455,7 @@ static FftArgs fft_args(const dsht_plan* p, long ldg, int ncols, long gld) {
   a.order = p->fft_order;
   a.deriv = 0;
   a.xy2 = nullptr;
+  a.nf = 1;
   return a;
 }
 
@@ -489,21 +490,36 @@ static int p2_inv(const dsht_plan* p, const GT* G, const FftArgs& a, double* xy,
   return 0;
 }
 
+bool fft_reg_ok(const dsht_plan* p) { return p->fft_kind != 1 && reg_fft_supported(p->fft.M); }
+
 template <typename GT, typename XT>
-static int fft_fwd_any(const dsht_plan* p, const XT* xy, long ldg, int ncols, GT* G, long gld,
-                       unsigned* colmax, hipStream_t s) {
+static int fft_fwd_any(const dsht_plan* p, const XT* const* xys, int nf, long ldg, int ncols, GT* const* Gs, long gld,
+                       unsigned* colmax, hipStream_t s, const double* rowscale = nullptr) {
   FftArgs a = fft_args(p, ldg, ncols, gld);
+  a.rowscale = rowscale;
+  if (rowscale && !fft_reg_ok(p)) return fail(DSHT_EUNSUPPORTED, "scaled forward FFT needs a register kernel");
   // forward: FP32 arithmetic for the split forms' FP32 Fourier coefficients; the register
   // kernel transforms each row relative to its first sample (FP64), so a large zonal mean
   // does not cost the m > 0 coefficients their relative precision
   a.fp32 = (sizeof(GT) == 8 && p->fft_kind == 0) ? 1 : 0;
   long nrows = (long)p->J * ncols;
-  ProfScope ps("fft_fwd", s, (double)nrows * ((double)sizeof(XT) * p->I + (double)sizeof(GT) * (p->N + 1)),
-               (double)nrows * 2.5 * p->I * std::log2((double)p->I));
-  if (p->fft_kind != 1 && reg_fft_supported(a.M)) return reg_fft_fwd<GT, XT>(xy, a, G, colmax, s);
+  ProfScope ps("fft_fwd", s, (double)nf * nrows * ((double)sizeof(XT) * p->I + (double)sizeof(GT) * (p->N + 1)),
+               (double)nf * nrows * 2.5 * p->I * std::log2((double)p->I));
+  if (fft_reg_ok(p)) {
+    a.nf = nf;
+    for (int i = 1; i < nf; i++) {
+      a.more_in[i - 1] = xys[i];
+      a.more_out[i - 1] = Gs[i];
+    }
+    return reg_fft_fwd<GT, XT>(xys[0], a, Gs[0], colmax, s);
+  }
   if constexpr (sizeof(XT) == 4) {
     return fail(DSHT_EUNSUPPORTED, "FP32 grids need a register FFT kernel (DSHT_TUNE_FFT 0)");
   } else {
+    for (int i = 1; i < nf; i++)
+      if (int rc = fft_fwd_any<GT, XT>(p, xys + i, 1, ldg, ncols, Gs + i, gld, colmax, s)) return rc;
+    const XT* xy = xys[0];
+    GT* G = Gs[0];
     switch (a.M) {
       case 16: return p2_fwd<16>(p, xy, a, G, colmax, s);
       case 32: return p2_fwd<32>(p, xy, a, G, colmax, s);
@@ -520,27 +536,36 @@ static int fft_fwd_any(const dsht_plan* p, const XT* xy, long ldg, int ncols, GT
   }
 }
 
-bool fft_inv_deriv_ok(const dsht_plan* p) { return p->fft_kind != 1 && reg_fft_supported(p->fft.M); }
-
 template <typename GT, typename XT>
-static int fft_inv_any(const dsht_plan* p, const GT* G, long gld, int ncols, XT* xy, long ldg,
+static int fft_inv_any(const dsht_plan* p, const GT* const* Gs, int nf, long gld, int ncols, XT* const* xys, long ldg,
                        hipStream_t s, const double* rowscale, int deriv, XT* xy2) {
   FftArgs a = fft_args(p, ldg, ncols, gld);
   a.rowscale = rowscale;
   a.deriv = deriv;
   a.xy2 = xy2;
-  if ((deriv || xy2) && !fft_inv_deriv_ok(p))
+  if ((deriv || xy2) && !fft_reg_ok(p))
     return fail(DSHT_EUNSUPPORTED, "derivative inverse FFT needs a register kernel");
   // inverse: FP32 arithmetic on the split forms' FP32 Fourier coefficients (each output point
   // is a sum of already-FP32 terms; the error stays at FP32 rounding of the output scale)
   a.fp32 = (sizeof(GT) == 8 && p->fft_kind == 0) ? 1 : 0;
   long nrows = (long)p->J * ncols;
-  ProfScope ps("fft_inv", s, (double)nrows * ((xy2 ? 2.0 : 1.0) * sizeof(XT) * p->I + (double)sizeof(GT) * (p->N + 1)),
-               (double)nrows * (xy2 ? 2.0 : 1.0) * 2.5 * p->I * std::log2((double)p->I));
-  if (p->fft_kind != 1 && reg_fft_supported(a.M)) return reg_fft_inv<GT, XT>(G, a, xy, s);
+  ProfScope ps("fft_inv", s, (double)nf * nrows * ((xy2 ? 2.0 : 1.0) * sizeof(XT) * p->I + (double)sizeof(GT) * (p->N + 1)),
+               (double)nf * nrows * (xy2 ? 2.0 : 1.0) * 2.5 * p->I * std::log2((double)p->I));
+  if (fft_reg_ok(p)) {
+    a.nf = nf;
+    for (int i = 1; i < nf; i++) {
+      a.more_in[i - 1] = Gs[i];
+      a.more_out[i - 1] = xys[i];
+    }
+    return reg_fft_inv<GT, XT>(Gs[0], a, xys[0], s);
+  }
   if constexpr (sizeof(XT) == 4) {
     return fail(DSHT_EUNSUPPORTED, "FP32 grids need a register FFT kernel (DSHT_TUNE_FFT 0)");
   } else {
+    for (int i = 1; i < nf; i++)
+      if (int rc = fft_inv_any<GT, XT>(p, Gs + i, 1, gld, ncols, xys + i, ldg, s, rowscale, deriv, nullptr)) return rc;
+    const GT* G = Gs[0];
+    XT* xy = xys[0];
     switch (a.M) {
       case 16: return p2_inv<16>(p, G, a, xy, s);
       case 32: return p2_inv<32>(p, G, a, xy, s);
@@ -557,34 +582,34 @@ static int fft_inv_any(const dsht_plan* p, const GT* G, long gld, int ncols, XT*
   }
 }
 
-int launch_fft_fwd(const dsht_plan* p, const double* xy, long ldg, int ncols, double2* G, long gld,
-                   hipStream_t s) {
-  return fft_fwd_any<double2, double>(p, xy, ldg, ncols, G, gld, nullptr, s);
+int launch_fft_fwd(const dsht_plan* p, const double* const* xy, int nf, long ldg, int ncols, double2* const* G, long gld,
+                   hipStream_t s, const double* rowscale) {
+  return fft_fwd_any<double2, double>(p, xy, nf, ldg, ncols, G, gld, nullptr, s, rowscale);
 }
 
-int launch_fft_inv(const dsht_plan* p, const double2* G, long gld, int ncols, double* xy, long ldg,
-                   hipStream_t s, const double* rowscale, int deriv, double* xy2) {
-  return fft_inv_any<double2, double>(p, G, gld, ncols, xy, ldg, s, rowscale, deriv, xy2);
+int launch_fft_inv(const dsht_plan* p, const double2* const* G, int nf, long gld, int ncols, double* const* xy, long ldg,
+                   hipStream_t s, const double* rowscale, int deriv) {
+  return fft_inv_any<double2, double>(p, G, nf, gld, ncols, xy, ldg, s, rowscale, deriv, nullptr);
 }
 
 int launch_fft_fwd32(const dsht_plan* p, const double* xy, long ldg, int ncols, float2* G, long gld,
                      unsigned* colmax, hipStream_t s) {
-  return fft_fwd_any<float2, double>(p, xy, ldg, ncols, G, gld, colmax, s);
+  return fft_fwd_any<float2, double>(p, &xy, 1, ldg, ncols, &G, gld, colmax, s);
 }
 
 int launch_fft_inv32(const dsht_plan* p, const float2* G, long gld, int ncols, double* xy, long ldg,
                      hipStream_t s, const double* rowscale, int deriv, double* xy2) {
-  return fft_inv_any<float2, double>(p, G, gld, ncols, xy, ldg, s, rowscale, deriv, xy2);
+  return fft_inv_any<float2, double>(p, &G, 1, gld, ncols, &xy, ldg, s, rowscale, deriv, xy2);
 }
 
 int launch_fft_fwd32f(const dsht_plan* p, const float* xy, long ldg, int ncols, float2* G, long gld,
                       unsigned* colmax, hipStream_t s) {
-  return fft_fwd_any<float2, float>(p, xy, ldg, ncols, G, gld, colmax, s);
+  return fft_fwd_any<float2, float>(p, &xy, 1, ldg, ncols, &G, gld, colmax, s);
 }
 
 int launch_fft_inv32f(const dsht_plan* p, const float2* G, long gld, int ncols, float* xy, long ldg,
                       hipStream_t s, const double* rowscale, int deriv, float* xy2) {
-  return fft_inv_any<float2, float>(p, G, gld, ncols, xy, ldg, s, rowscale, deriv, xy2);
+  return fft_inv_any<float2, float>(p, &G, 1, gld, ncols, &xy, ldg, s, rowscale, deriv, xy2);
 }
 
 }  // namespace dsht

@@ -298,10 +298,18 @@ __device__ __forceinline__ void store_pair(float* x, double a, double b) {
 }
 
 // V: arithmetic type (double2, or float2 for the FP32 Fourier path of the split forms);
-// XT: grid element type (double, or float for the split forms' FP32 grid I/O)
-template <int R1, int R2, int NT, typename GT, typename V, typename XT>
+// XT: grid element type (double, or float for the split forms' FP32 grid I/O).  PRE (FP64
+// arithmetic): the rows times a.rowscale are transformed.  Grid y: fields of one
+// launch (FP64 coefficients).
+template <int R1, int R2, int NT, typename GT, typename V, typename XT, bool PRE>
 __global__ __launch_bounds__(NT, WPE<V>) void k_fft_fwd_r(const XT* __restrict__ xy, GT* __restrict__ G,
                                                   FftArgs a, unsigned* __restrict__ colmax) {
+  if constexpr (sizeof(GT) == 16) {
+    if (blockIdx.y) {
+      xy = static_cast<const XT*>(a.more_in[blockIdx.y - 1]);
+      G = static_cast<GT*>(a.more_out[blockIdx.y - 1]);
+    }
+  }
   using C = RegFft<R1, R2, NT, V>;
   using S = typename Cx<V>::S;
   constexpr int M = C::M, ROWS = C::ROWS, PY = C::PY, SR = C::SR;
@@ -342,6 +350,7 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_fwd_r(const XT* __restrict__
   RV raw[REF ? R2 : 1];
   double x0 = 0.0;  // reference sample of the thread's pass-1 row (REF)
   XT x0n = 0;       // the next group's, as loaded
+  double sc = 1.0;  // PRE: the row's factor, loaded with it and applied at the top of its group
   auto fetch = [&](long g) {
     int j = 0, c = 0;
     if constexpr (REF) {
@@ -352,6 +361,7 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_fwd_r(const XT* __restrict__
       for (int n2 = 0; n2 < R2; n2++) raw[n2] = load_raw(xr + 2 * (n1 + R1 * n2));
     } else if (rr1 < ROWS && map_row(a, g, rr1, ROWS, j, c)) {
       const XT* xr = xy + c * a.ldg + (long)j * (2 * M);
+      if constexpr (PRE) sc = a.rowscale[j];
       if constexpr (sizeof(XT) == 8) {
         const double2* x = reinterpret_cast<const double2*>(xr);
 #pragma unroll
@@ -372,6 +382,10 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_fwd_r(const XT* __restrict__
       x0 = (double)x0n;
 #pragma unroll
       for (int n2 = 0; n2 < R2; n2++) v[n2] = mk<V>((double)raw[n2].x - x0, (double)raw[n2].y - x0);
+    }
+    if constexpr (PRE) {
+#pragma unroll
+      for (int n2 = 0; n2 < R2; n2++) v[n2] = mk<V>((S)(v[n2].x * sc), (S)(v[n2].y * sc));
     }
     dft<R2, -1>(v);
     if (colmax && tid < ROWS) smax[tid] = 0u;
@@ -438,6 +452,12 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_fwd_r(const XT* __restrict__
 template <int R1, int R2, int NT, typename GT, typename V, int MODE, typename XT>
 __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__ G, XT* __restrict__ xy,
                                                   FftArgs a) {
+  if constexpr (sizeof(GT) == 16) {  // fields of one launch
+    if (blockIdx.y) {
+      G = static_cast<const GT*>(a.more_in[blockIdx.y - 1]);
+      xy = static_cast<XT*>(a.more_out[blockIdx.y - 1]);
+    }
+  }
   using C = RegFft<R1, R2, NT, V>;
   using S = typename Cx<V>::S;
   constexpr int M = C::M, ROWS = C::ROWS, PY = C::PY, SR = C::SR;
@@ -582,26 +602,38 @@ static long resident_grid(K kernel, int threads, size_t lds) {
   return (long)per_cu * cu_count();
 }
 
-template <int R1, int R2, int NT, typename GT, typename V, typename XT>
-static int reg_fwd_nt(const XT* xy, const FftArgs& a, GT* G, unsigned* colmax, hipStream_t s) {
+// workgroups per field of a launch of a.nf fields that keep the resident grid
+static long field_grid(long groups, long cap, int nf) {
+  cap /= nf;
+  return groups < cap ? groups : (cap > 0 ? cap : 1);
+}
+
+template <int R1, int R2, int NT, typename GT, typename V, typename XT, bool PRE>
+static int reg_fwd_pre(const XT* xy, const FftArgs& a, GT* G, unsigned* colmax, hipStream_t s) {
   using C = RegFft<R1, R2, NT, V>;
-  static const long cap = resident_grid(k_fft_fwd_r<R1, R2, NT, GT, V, XT>, C::THREADS, C::LDS);
-  long nb = row_groups(a, C::ROWS);
-  if (nb > cap) nb = cap;
-  hipLaunchKernelGGL((k_fft_fwd_r<R1, R2, NT, GT, V, XT>), dim3((unsigned)nb), dim3(C::THREADS), C::LDS, s, xy, G, a,
-                     colmax);
+  static const long cap = resident_grid(k_fft_fwd_r<R1, R2, NT, GT, V, XT, PRE>, C::THREADS, C::LDS);
+  const long nb = field_grid(row_groups(a, C::ROWS), cap, a.nf);
+  hipLaunchKernelGGL((k_fft_fwd_r<R1, R2, NT, GT, V, XT, PRE>), dim3((unsigned)nb, a.nf), dim3(C::THREADS), C::LDS, s,
+                     xy, G, a, colmax);
   DSHT_HIP(hipGetLastError());
   return 0;
+}
+
+template <int R1, int R2, int NT, typename GT, typename V, typename XT>
+static int reg_fwd_nt(const XT* xy, const FftArgs& a, GT* G, unsigned* colmax, hipStream_t s) {
+  if constexpr (sizeof(GT) == 16 && sizeof(XT) == 8) {
+    if (a.rowscale) return reg_fwd_pre<R1, R2, NT, GT, V, XT, true>(xy, a, G, colmax, s);
+  }
+  return reg_fwd_pre<R1, R2, NT, GT, V, XT, false>(xy, a, G, colmax, s);
 }
 
 template <int R1, int R2, int NT, typename GT, typename V, int MODE, typename XT>
 static int reg_inv_mode(const GT* G, const FftArgs& a, XT* xy, hipStream_t s) {
   using C = RegFft<R1, R2, NT, V>;
   static const long cap = resident_grid(k_fft_inv_r<R1, R2, NT, GT, V, MODE, XT>, C::THREADS, C::LDS);
-  long nb = row_groups(a, C::ROWS);
-  if (nb > cap) nb = cap;
-  hipLaunchKernelGGL((k_fft_inv_r<R1, R2, NT, GT, V, MODE, XT>), dim3((unsigned)nb), dim3(C::THREADS), C::LDS, s, G,
-                     xy, a);
+  const long nb = field_grid(row_groups(a, C::ROWS), cap, a.nf);
+  hipLaunchKernelGGL((k_fft_inv_r<R1, R2, NT, GT, V, MODE, XT>), dim3((unsigned)nb, a.nf), dim3(C::THREADS), C::LDS, s,
+                     G, xy, a);
   DSHT_HIP(hipGetLastError());
   return 0;
 }

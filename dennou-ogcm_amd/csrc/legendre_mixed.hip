@@ -368,7 +368,7 @@ int mixed_run_inv(dsht_plan* p, int op, const double* in0, const double* in1, lo
     const int nc = ncols - c0 < ch ? ncols - c0 : ch;
     // fused value/gradient: GradLon through the derivative inverse FFT of the value's
     // coefficients (i m X_m, 1/cos row scale); the contraction writes two outputs
-    const bool dlon = op == I_VGRAD && out1 && fft_inv_deriv_ok(p);
+    const bool dlon = op == I_VGRAD && out1 && fft_reg_ok(p);
     float2* O0 = out0 || dlon ? G0 : nullptr;
     float2* O1 = nout > 1 && out1 && !dlon ? G1 : nullptr;
     float2* O2 = nout > 2 && out2 ? G2 : nullptr;

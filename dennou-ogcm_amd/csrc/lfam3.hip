@@ -720,14 +720,22 @@ int lf_vsolve(dsht_lfam3* s, bool mom, const VSolve& a, int ny, int nz, hipStrea
   return 0;
 }
 
+// calc_UVCosLat2VorDiv of (U cos phi, V cos phi), the vorticity in wVD's columns [0, nc) and the
+// divergence in [nc, 2 nc): cos phi is applied as the FFT reads the winds, or, where that form
+// has no such kernel, by a pass over them
+int lf_uv2vordiv(dsht_lfam3* s, const double* u, const double* v, int nc, const double* diag, hipStream_t st) {
+  dsht_plan* p = s->p;
+  if (uv_scaled_ok(p))
+    return uv2vordiv_scaled(p, u, v, s->d_cs, s->np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, diag, st);
+  LF_LAUNCH2(k_lf_uvcos, nc, s->np, st, u, v, s->d_cs, s->np, s->I, (long)nc, s->ucos, s->vcos);
+  return dsht_uv2vordiv_d(p, s->ucos, s->vcos, s->np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, diag, st);
+}
+
 // HBEDiagnose_VorDiv (HBEDiagnose_hspm_vfvm_mod.f90:259-286) over every layer of the active
 // runs: vorticity into VD[0, nc), divergence into VD[nc, 2 nc)
 int lf_vordiv(dsht_lfam3* s, const double* u, const double* v, int nc, hipStream_t st) {
-  dsht_plan* p = s->p;
-  LF_LAUNCH2(k_lf_uvcos, nc, s->np, st, u, v, s->d_cs, s->np, s->I, (long)nc, s->ucos, s->vcos);
-  if (int rc = dsht_uv2vordiv_d(p, s->ucos, s->vcos, s->np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, nullptr, st))
-    return rc;
-  return dsht_inv_d(p, DSHT_VAL, s->wVD, 2l * nc, 1, s->VD, s->np, 2 * nc, nullptr, st);
+  if (int rc = lf_uv2vordiv(s, u, v, nc, nullptr, st)) return rc;
+  return dsht_inv_d(s->p, DSHT_VAL, s->wVD, 2l * nc, 1, s->VD, s->np, 2 * nc, nullptr, st);
 }
 
 // HBEBaroc_MOMRHS_VorDivForm (HBEBaroc_hspm_vfvm_mod.f90:321-443) -> URHS, VRHS, with the vorticity
@@ -1090,8 +1098,7 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   // ImplUV (DOGCM_Phys_hspm_vfvm_mod.f90:666-748): implicit vertical viscosity, then
   // backward-Euler lateral viscosity on vorticity and divergence
   if ((rc = lf_vsolve(s, true, VSolve{{UN, VN}, {s->URHS, s->VRHS}, {UA, VA}}, nr, 2, st))) return rc;
-  LF_LAUNCH2(k_lf_uvcos, nc, np, st, UA, VA, s->d_cs, np, I, (long)nc, s->ucos, s->vcos);
-  if ((rc = dsht_uv2vordiv_d(p, s->ucos, s->vcos, np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, s->d_dmom, st))) return rc;
+  if ((rc = lf_uv2vordiv(s, UA, VA, nc, s->d_dmom, st))) return rc;
   if ((rc = dsht_vordiv2uv_d(p, s->wVD, s->wVD + nc, 2l * nc, 1, UA, VA, np, nc, st))) return rc;
   LF_LAUNCHC(k_lf_impl, np, nr, 1, st, UA, VA, UN, VN, b2[UBN], b2[VBN], PN, s->d_two_omega, s->d_mu, s->d_cs, c.depth,
              s->d_cdk, np, I, K, alpha_ * dt, dt, b2[UBT], b2[VBT], b2[AM2], b2[BG2], b2[SPM]);

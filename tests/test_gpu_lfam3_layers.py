@@ -53,3 +53,28 @@ def test_layers_match_oracle(gpu, km, cfg):
         for f in ("U", "V", "T", "S", "P"):
             assert rel_l2(got[f], ref[f + "N"]) < TOL, (r, f)
         assert np.array_equal(got["UB"], ref["UB"])
+
+
+def test_winds_scaled_in_fft_or_before(gpu):
+    """cos(lat) applied as the register FFT reads the winds, and by a pass over them where the
+    plan uses the LDS FFT (DSHT_TUNE_FFT = 1): one step either way, 1e-9 as above."""
+    import torch
+    import dsht
+    import lfam3
+    import oracle
+    from conftest import rel_l2
+    N, I, J, km = 21, 64, 32, 6
+    o = oracle.Oracle(N, I, J, 6.371e6)
+    st = lfam3.initial_state(o, km, seed=5)
+    got = []
+    for kind in (0, 1):
+        p, pool = _pool(N, I, J, km, 1, dt=1800.0)
+        p.set_tuning(dsht.TUNE_FFT, kind)
+        _load(pool, 0, st)
+        pool.set_rotation(0, OMEGA)
+        torch.cuda.synchronize()
+        pool.step(1)
+        torch.cuda.synchronize()
+        got.append(_read(pool, 0))
+    for f in ("U", "V", "T", "S", "P"):
+        assert rel_l2(got[1][f], got[0][f]) < TOL, f
