@@ -68,37 +68,39 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_inv_wk(LegInvArgs a, int 
   const double* Win[2] = {a.W0, a.W1};
   const double dm = (double)m;
 
-  // ---- stage: every load of a round is issued (padding reads element 0) before any is used
-  for (int e0 = tid; e0 < KR * C8; e0 += NTH * UB) {
+  // ---- stage: a thread stays in one column and takes every RS-th row; every load of a round is
+  // issued (padding reads element 0) before any is used
+  constexpr int RS = NTH / C8;
+  const int cc = tid % C8;
+  const bool cok = c0 + cc < a.ncols;
+  const long co = cok ? (long)(c0 + cc) * a.sc : 0;
+  double* put = wk_lds + (cc / 8) * KR * 16 + 2 * (cc % 8);
+  for (int r0 = tid / C8; r0 < KR; r0 += RS * UB) {
     double re[NIN][UB], im[NIN][UB], pr[UB];
     bool ok[UB];
 #pragma unroll
     for (int q = 0; q < UB; q++) {
-      const int e = e0 + q * NTH;
-      const int r = e / C8, c = c0 + e % C8;
-      const int par = r < 4 * ks0n ? 0 : 1, k = par ? r - 4 * ks0n : r;
-      const int n = m + par + 2 * k;
-      ok[q] = e < KR * C8 && n <= N && c < a.ncols;
-      const long l0 = ok[q] ? (long)n * (n + 1) : 0, mm = ok[q] ? m : 0;
-      const long co = ok[q] ? (long)c * a.sc : 0;
-      pr[q] = a.pro ? a.pro[l0 + mm] : 1.0;
+      const int r = r0 + q * RS;
+      const int n = r < 4 * ks0n ? m + 2 * r : m + 1 + 2 * (r - 4 * ks0n);
+      ok[q] = r < KR && n <= N && cok;
+      const int l = ok[q] ? n * (n + 1) + m : 0, li = ok[q] ? l - 2 * m : 0;
+      pr[q] = a.pro ? a.pro[l] : 1.0;
 #pragma unroll
       for (int i = 0; i < NIN; i++) {
-        re[i][q] = __builtin_nontemporal_load(Win[i] + (l0 + mm) * a.sl + co);
-        im[i][q] = __builtin_nontemporal_load(Win[i] + (l0 - mm) * a.sl + co);
+        re[i][q] = __builtin_nontemporal_load(Win[i] + l * a.sl + co);
+        im[i][q] = __builtin_nontemporal_load(Win[i] + li * a.sl + co);
       }
     }
 #pragma unroll
     for (int q = 0; q < UB; q++) {
-      const int e = e0 + q * NTH;
-      if (e < KR * C8) {
-        const int r = e / C8, cc = e % C8;
+      const int r = r0 + q * RS;
+      if (r < KR) {
 #pragma unroll
         for (int i = 0; i < NIN; i++) {
           double2 v;
           v.x = ok[q] ? pr[q] * re[i][q] : 0.0;
           v.y = ok[q] && m > 0 ? pr[q] * im[i][q] : 0.0;
-          *(double2*)(wk_lds + ((i * NCT + cc / 8) * KR + r) * 16 + 2 * (cc % 8)) = v;
+          *(double2*)(put + i * NCT * KR * 16 + r * 16) = v;
         }
       }
     }
@@ -118,14 +120,26 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_inv_wk(LegInvArgs a, int 
         for (int ct = 0; ct < NCT; ct++) acc[x][i][ct][0] = acc[x][i][ct][1] = double4_t{0, 0, 0, 0};
     const long b0 = (long)t * kp0 * 16, b1 = (long)a.J2pad * kp0 + (long)t * kp1 * 16;
     double cur[NTB][U], nxt[NTB][U];
-    auto fetch = [&](double (&x)[NTB][U], long base, int ks, int nks) {
+    // whole chunks: a tile's steps are padded to them in the table (steps past the last one that
+    // is needed are not multiplied)
+    static_assert(KCH % (4 * U) == 0, "chunks of the padded table");
+    auto fetch = [&](double (&x)[NTB][U], long at) {
+      const double *P = tabP + at, *H = tabH + at;
 #pragma unroll
       for (int u = 0; u < U; u++) {
-        const int k = ks + u < nks ? ks + u : nks - 1;  // past the end: a step that is not multiplied
-        if constexpr (UP) x[0][u] = tabP[base + (long)k * 64];
-        if constexpr (UH) x[NTB - 1][u] = tabH[base + (long)k * 64];
+        if constexpr (UP) x[0][u] = P[u * 64];
+        if constexpr (UH) x[NTB - 1][u] = H[u * 64];
       }
     };
+    // the row scales are in registers by the time the products are done
+    const int jr0 = t * TILE + krow;
+    double sN[4], sS[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int jr = jr0 + 4 * i < J2 ? jr0 + 4 * i : 0;
+      sN[i] = a.rs ? a.rs[J2 + jr] : 1.0;
+      sS[i] = a.rs ? a.rs[J2 - 1 - jr] : 1.0;
+    }
     auto chain = [&](auto PAR) {
       constexpr int par = decltype(PAR)::value, sP = par, sH = 1 - par;
       const int nks = par ? ks1n : ks0n;
@@ -133,8 +147,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_inv_wk(LegInvArgs a, int 
       for (int ks = 0; ks < nks; ks += U) {
         // the next chunk's fragments: of this parity, or the other one's first
         const bool more = ks + U < nks;
-        if (more || (par == 0 && ks1n > 0))
-          fetch(nxt, more ? (par ? b1 : b0) : b1, more ? ks + U : 0, more ? nks : ks1n);
+        if (more || (par == 0 && ks1n > 0)) fetch(nxt, more ? (par ? b1 : b0) + (ks + U) * 64l : b1);
 #pragma unroll
         for (int u = 0; u < U; u++) {
           if (ks + u < nks) {
@@ -163,7 +176,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_inv_wk(LegInvArgs a, int 
           for (int u = 0; u < U; u++) cur[x][u] = nxt[x][u];
       }
     };
-    fetch(cur, b0, 0, ks0n);
+    fetch(cur, b0);
     // vmcnt(0): with nothing in flight at its entry, the loop waits only for its own loads (the
     // wait counts that the compiler merges over the loop's two entries would otherwise also
     // cover the chunk just requested)
@@ -174,41 +187,39 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_inv_wk(LegInvArgs a, int 
     // ---- epilogue: north = sym + anti, south = sym - anti, i m, row scale
     const int part = col & 1;
     const double im = part ? dm : -dm;  // (i m z) = (-m z.im, m z.re)
+    const bool zero = m == 0 && part;
+    const long at = ((long)m * a.gmst + c0) * 2 + col, rowN = (long)(J2 + jr0) * a.gld * 2,
+               rowS = (long)(J2 - 1 - jr0) * a.gld * 2, step = 8 * a.gld;
 #pragma unroll
     for (int ct = 0; ct < NCT; ct++) {
-      const int c = c0 + ct * 8 + (col >> 1);
-      if (c >= a.ncols) continue;
+      if (c0 + ct * 8 + (col >> 1) >= a.ncols) continue;
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const int jr = t * TILE + krow + 4 * i;
-        if (jr >= J2) continue;
-        const int jN = J2 + jr, jS = J2 - 1 - jr;
-        const double sN = a.rs ? a.rs[jN] : 1.0, sS = a.rs ? a.rs[jS] : 1.0;
+        if (jr0 + 4 * i >= J2) continue;
         auto put = [&](double2* G, double n, double s) {
-          if (m == 0 && part) n = s = 0.0;
-          double* g = (double*)(G + (long)m * a.gmst + c) + part;
-          g[2l * jN * a.gld] = n;
-          g[2l * jS * a.gld] = s;
+          double* g = (double*)G + at + ct * 16;
+          g[rowN + i * step] = zero ? 0.0 : n;
+          g[rowS - i * step] = zero ? 0.0 : s;
         };
         auto north = [&](int x, int in) { return acc[x][in][ct][0][i] + acc[x][in][ct][1][i]; };
         auto south = [&](int x, int in) { return acc[x][in][ct][0][i] - acc[x][in][ct][1][i]; };
         if constexpr (OP == I_VAL || OP == I_GRADMU) {
-          put(a.G0, north(0, 0) * sN, south(0, 0) * sS);
+          put(a.G0, north(0, 0) * sN[i], south(0, 0) * sS[i]);
         } else if constexpr (OP == I_GRADLAMBDA) {
-          put(a.G0, im * other_part(north(0, 0)) * sN, im * other_part(south(0, 0)) * sS);
+          put(a.G0, im * other_part(north(0, 0)) * sN[i], im * other_part(south(0, 0)) * sS[i]);
         } else if constexpr (OP == I_VGRAD) {  // no row scale on the value
           const double n = north(0, 0), s = south(0, 0);
           if (a.G0) put(a.G0, n, s);
-          if (a.G1) put(a.G1, im * other_part(n) * sN, im * other_part(s) * sS);
-          if (a.G2) put(a.G2, north(NTB - 1, 0) * sN, south(NTB - 1, 0) * sS);
+          if (a.G1) put(a.G1, im * other_part(n) * sN[i], im * other_part(s) * sS[i]);
+          if (a.G2) put(a.G2, north(NTB - 1, 0) * sN[i], south(NTB - 1, 0) * sS[i]);
         } else if constexpr (OP == I_ALPHA) {  // i m P.A + H.B
-          put(a.G0, (im * other_part(north(0, 0)) + north(NTB - 1, 0)) * sN,
-              (im * other_part(south(0, 0)) + south(NTB - 1, 0)) * sS);
+          put(a.G0, (im * other_part(north(0, 0)) + north(NTB - 1, 0)) * sN[i],
+              (im * other_part(south(0, 0)) + south(NTB - 1, 0)) * sS[i]);
         } else {  // U = i m P.chi - H.psi, V = i m P.psi + H.chi
-          put(a.G0, (im * other_part(north(0, NP - 1)) - north(NTB - 1, 0)) * sN,
-              (im * other_part(south(0, NP - 1)) - south(NTB - 1, 0)) * sS);
-          put(a.G1, (im * other_part(north(0, 0)) + north(NTB - 1, NP - 1)) * sN,
-              (im * other_part(south(0, 0)) + south(NTB - 1, NP - 1)) * sS);
+          put(a.G0, (im * other_part(north(0, NP - 1)) - north(NTB - 1, 0)) * sN[i],
+              (im * other_part(south(0, NP - 1)) - south(NTB - 1, 0)) * sS[i]);
+          put(a.G1, (im * other_part(north(0, 0)) + north(NTB - 1, NP - 1)) * sN[i],
+              (im * other_part(south(0, 0)) + south(NTB - 1, NP - 1)) * sS[i]);
         }
       }
     }
@@ -240,28 +251,34 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
   const double2* Gm[2] = {a.G0 + (long)m * a.gmst, NIN > 1 ? a.G1 + (long)m * a.gmst : nullptr};
   const double dm = (double)m;
 
-  for (int e0 = tid; e0 < KR * C8; e0 += NTH * UB) {
+  // ---- stage: a thread stays in one column and takes every RS-th latitude pair; every load of a
+  // round is issued (padding reads the first pair) before any is used
+  constexpr int RS = NTH / C8;
+  const int cc = tid % C8;
+  const bool cok = c0 + cc < a.ncols;
+  const long co = cok ? c0 + cc : 0;
+  double* put = wk_lds + (cc / 8) * KR * 16 + 2 * (cc % 8);
+  for (int j0 = tid / C8; j0 < KR; j0 += RS * UB) {
     double2 gn[NIN][UB], gs[NIN][UB];
     double cw[UB];
     bool ok[UB];
 #pragma unroll
     for (int q = 0; q < UB; q++) {
-      const int e = e0 + q * NTH;
-      const int j = e / C8, c = c0 + e % C8;
-      ok[q] = j < J2 && c < a.ncols;
-      const long jj = ok[q] ? j : 0, co = ok[q] ? c : 0;
+      const int j = j0 + q * RS;
+      ok[q] = j < J2 && cok;
+      const int jj = ok[q] ? j : 0;
       cw[q] = a.cw[jj];
+      const long n = (J2 + jj) * a.gld + co, s = (J2 - 1 - jj) * a.gld + co;
 #pragma unroll
       for (int i = 0; i < NIN; i++) {
-        gn[i][q] = Gm[i][(J2 + jj) * a.gld + co];
-        gs[i][q] = Gm[i][(J2 - 1 - jj) * a.gld + co];
+        gn[i][q] = Gm[i][n];
+        gs[i][q] = Gm[i][s];
       }
     }
 #pragma unroll
     for (int q = 0; q < UB; q++) {
-      const int e = e0 + q * NTH;
-      if (e < KR * C8) {
-        const int j = e / C8, cc = e % C8;
+      const int j = j0 + q * RS;
+      if (j < KR) {
 #pragma unroll
         for (int i = 0; i < NIN; i++) {
           double2 s, d;
@@ -269,7 +286,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
           s.y = ok[q] ? cw[q] * (gn[i][q].y + gs[i][q].y) : 0.0;
           d.x = ok[q] ? cw[q] * (gn[i][q].x - gs[i][q].x) : 0.0;
           d.y = ok[q] ? cw[q] * (gn[i][q].y - gs[i][q].y) : 0.0;
-          double* at = wk_lds + ((i * 2 * NCT + cc / 8) * KR + j) * 16 + 2 * (cc % 8);
+          double* at = put + i * 2 * NCT * KR * 16 + j * 16;
           *(double2*)at = s;
           *(double2*)(at + NCT * KR * 16) = d;
         }
@@ -344,8 +361,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           const int n = m + par + 2 * ((par ? t - tE : t) * TILE + krow + 4 * i);
-          const long l = n <= N ? (long)n * (n + 1) + (part ? -m : m) : 0;
-          dv[o][i] = dg ? dg[l] : 1.0;
+          dv[o][i] = dg ? dg[n <= N ? n * (n + 1) + (part ? -m : m) : 0] : 1.0;
         }
       }
 #pragma unroll
@@ -365,12 +381,9 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
           v[NOUT - 1] = im * other_part(acc[0][0][ct][i]) - acc[NTB - 1][NP - 1][ct][i];
         }
         if (n > N || (m == 0 && part)) continue;
-        const long l = (long)n * (n + 1) + (part ? -m : m);
+        const long at = (n * (n + 1) + (part ? -m : m)) * a.sl + (long)c * a.sc;
 #pragma unroll
-        for (int o = 0; o < NOUT; o++) {
-          double* W = o == 0 ? a.W0 : a.W1;
-          W[l * a.sl + (long)c * a.sc] = v[o] * a.scale * dv[o][i];
-        }
+        for (int o = 0; o < NOUT; o++) (o == 0 ? a.W0 : a.W1)[at] = v[o] * a.scale * dv[o][i];
       }
     }
   }
