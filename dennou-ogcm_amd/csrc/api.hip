@@ -133,9 +133,10 @@ static int check_plan(const dsht_plan* p) {
 // forward family: grids -> spectra
 static int run_fwd(dsht_plan* p, int op, const double* in0, const double* in1, long ldg, double* out0,
                    double* out1, long sl, long sc, int ncols, const double* diag0, const double* diag1,
-                   double scale, const double* cw, hipStream_t s, const double* rowscale = nullptr) {
+                   double scale, const double* cw, hipStream_t s, const double* rowscale = nullptr,
+                   const double* in2 = nullptr, int add = 0) {
   if (ncols <= 0) return 0;
-  const int nin = (op == F_ALPHA || op == F_UV2VORDIV) ? 2 : 1;
+  const int nin = op == F_VALSUBALPHA ? 3 : (op == F_ALPHA || op == F_UV2VORDIV) ? 2 : 1;
   const int ch = chunk_cols(p, ncols);
   const int nchunks = cdiv(ncols, ch);
   const size_t slot_bytes = nin * fourier_bytes(p, ch);
@@ -147,12 +148,18 @@ static int run_fwd(dsht_plan* p, int op, const double* in0, const double* in1, l
     double2* G0 = (double2*)wl.buf;
     double2* G1 = G0 + (size_t)(p->N + 1) * p->J * fourier_pitch(ch);
     const long gp = fourier_pitch(nc);
-    const double* xs[2] = {in0 + (long)c0 * ldg, nin > 1 ? in1 + (long)c0 * ldg : nullptr};
-    double2* const gs[2] = {G0, G1};
+    double2* G2 = G1 + (size_t)(p->N + 1) * p->J * fourier_pitch(ch);
+    const double* xs[3] = {in0 + (long)c0 * ldg, nin > 1 ? in1 + (long)c0 * ldg : nullptr,
+                           nin > 2 ? in2 + (long)c0 * ldg : nullptr};
+    double2* const gs[3] = {G0, G1, G2};
     if ((rc = launch_fft_fwd(p, xs, nin, ldg, nc, gs, gp, s, rowscale))) return rc;
     LegFwdArgs a;
     a.G0 = G0;
     a.G1 = nin > 1 ? G1 : nullptr;
+    a.G2 = nin > 2 ? G2 : nullptr;
+    a.cw2 = p->d_cwv;
+    a.ralpha = 1.0 / p->R;
+    a.add = add;
     a.W0 = out0 + (long)c0 * sc;
     a.W1 = out1 ? out1 + (long)c0 * sc : nullptr;
     a.sl = sl;
@@ -258,6 +265,21 @@ bool uv_scaled_ok(const dsht_plan* p) { return p->prec == DSHT_PREC_FP64 && fft_
 int uv2vordiv_scaled(dsht_plan* p, const double* u, const double* v, const double* rowscale, long ldg, double* vor,
                      double* div, long sl, long sc, int ncols, const double* diag, hipStream_t s) {
   return run_fwd(p, F_UV2VORDIV, u, v, ldg, vor, div, sl, sc, ncols, diag, diag, 1.0 / p->R, p->d_cwd, s, rowscale);
+}
+
+bool fwd_fused_ok(const dsht_plan* p) {
+  return p->prec == DSHT_PREC_FP64 && p->leg_kind == 0 && leg_fwd_staged_ok(p, F_VALSUBALPHA);
+}
+
+int val_sub_alpha(dsht_plan* p, const double* a, const double* b, const double* c, long ldg, double* w, long sl, long sc,
+                  int ncols, const double* diag, hipStream_t s) {
+  return run_fwd(p, F_VALSUBALPHA, a, b, ldg, w, nullptr, sl, sc, ncols, diag, nullptr, 1.0, p->d_cwd, s, nullptr, c);
+}
+
+int fwd_add(dsht_plan* p, const double* xy, long ldg, double* w, long sl, long sc, int ncols, const double* diag,
+            hipStream_t s) {
+  return run_fwd(p, F_VAL, xy, nullptr, ldg, w, nullptr, sl, sc, ncols, diag, nullptr, 1.0, p->d_cwv, s, nullptr,
+                 nullptr, 1);
 }
 
 static int check_grid_ptr(const void* x, long ldg, const dsht_plan* p) {

@@ -32,7 +32,8 @@ __host__ __device__ inline int n_par(int N, int m, int p) {
 }
 
 // ---------------------------------------------------------------- ops
-enum FwdOp { F_VAL = 0, F_DIVLAMBDA = 1, F_DIVMU = 2, F_ALPHA = 3, F_UV2VORDIV = 4 };
+// F_VALSUBALPHA: w_xy(C) - w_AlphaOptr_xy(A, B) in one pass (staged FP64 contraction only)
+enum FwdOp { F_VAL = 0, F_DIVLAMBDA = 1, F_DIVMU = 2, F_ALPHA = 3, F_UV2VORDIV = 4, F_VALSUBALPHA = 5 };
 // I_VGRAD: value, GradLon and GradLat of one field from one contraction pass (P and H
 // share the data; GradLon is i m times the P result)
 enum InvOp { I_VAL = 0, I_GRADLAMBDA = 1, I_GRADMU = 2, I_ALPHA = 3, I_VORDIV2UV = 4, I_VGRAD = 5 };
@@ -40,10 +41,11 @@ enum InvOp { I_VAL = 0, I_GRADLAMBDA = 1, I_GRADMU = 2, I_ALPHA = 3, I_VORDIV2UV
 // inputs, outputs and tables of each operator
 template <int OP>
 struct FwdTraits {
-  static constexpr int NIN = (OP == F_ALPHA || OP == F_UV2VORDIV) ? 2 : 1;
+  // operands of the products (F_VALSUBALPHA merges its three inputs into two)
+  static constexpr int NIN = (OP == F_ALPHA || OP == F_UV2VORDIV || OP == F_VALSUBALPHA) ? 2 : 1;
   static constexpr int NOUT = (OP == F_UV2VORDIV) ? 2 : 1;
   static constexpr bool USE_P = (OP != F_DIVMU);
-  static constexpr bool USE_H = (OP == F_DIVMU || OP == F_ALPHA || OP == F_UV2VORDIV);
+  static constexpr bool USE_H = (OP == F_DIVMU || OP == F_ALPHA || OP == F_UV2VORDIV || OP == F_VALSUBALPHA);
 };
 
 template <int OP>
@@ -62,6 +64,7 @@ inline int inv_nout(int op) { return op == I_VORDIV2UV ? 2 : (op == I_VGRAD ? 3 
 struct LegFwdArgs {
   const double2* G0;  // Fourier coefficients [m][j*gld + c] (complex), input 0
   const double2* G1;  // input 1 (two-input ops)
+  const double2* G2 = nullptr;  // input 2 (F_VALSUBALPHA: C)
   double* W0;         // spectral output 0 (element (l, c) at l*sl + c*sc)
   double* W1;         // spectral output 1
   long sl, sc;
@@ -75,6 +78,9 @@ struct LegFwdArgs {
   const double* diag0;  // per-l epilogue multipliers (nullable)
   const double* diag1;
   double scale;       // extra scalar factor (1/R for the H operator)
+  const double* cw2 = nullptr;  // weights of input 2
+  double ralpha = 0.0;          // F_VALSUBALPHA: 1/R of the AlphaOptr inputs
+  int add = 0;        // F_VAL: add to the output instead of writing it (staged kernel only)
   int N, J2, J2pad;
 };
 
@@ -231,6 +237,13 @@ int fail(int code, const char* fmt, ...);
 // api.hip: calc_UVCosLat2VorDiv of (u rowscale, v rowscale), the row factor (J, device) applied as
 // the FFT reads the grids; FP64 form with a register FFT only (uv_scaled_ok)
 bool uv_scaled_ok(const dsht_plan* p);
+// w_xy(c) - w_AlphaOptr_xy(a, b), and w += diag w_xy(xy), each in one contraction: FP64 staged
+// form only (fwd_fused_ok)
+bool fwd_fused_ok(const dsht_plan* p);
+int val_sub_alpha(dsht_plan* p, const double* a, const double* b, const double* c, long ldg, double* w, long sl, long sc,
+                  int ncols, const double* diag, hipStream_t s);
+int fwd_add(dsht_plan* p, const double* xy, long ldg, double* w, long sl, long sc, int ncols, const double* diag,
+            hipStream_t s);
 int uv2vordiv_scaled(dsht_plan* p, const double* u, const double* v, const double* rowscale, long ldg, double* vor,
                      double* div, long sl, long sc, int ncols, const double* diag, hipStream_t s);
 // api.hip: per-stream scratch

@@ -573,12 +573,14 @@ static void leg_work(const dsht_plan* p, int nin, int nout, int nterm, int ntab,
 int launch_leg_fwd(const dsht_plan* p, int op, const LegFwdArgs& a, hipStream_t s) {
   const bool wide = p->leg_cb ? p->leg_cb == 32 : a.ncols > 16;
   double by, fl;
-  static const int nin[] = {1, 1, 1, 2, 2}, nout[] = {1, 1, 1, 1, 2}, nt[] = {1, 1, 1, 2, 4}, ntab[] = {1, 1, 1, 2, 2};
+  static const int nin[] = {1, 1, 1, 2, 2, 3}, nout[] = {1, 1, 1, 1, 2, 1}, nt[] = {1, 1, 1, 2, 4, 2},
+                   ntab[] = {1, 1, 1, 2, 2, 2};
   leg_work(p, nin[op], nout[op], nt[op], ntab[op], true, a.ncols, &by, &fl);
   ProfScope ps("leg_fwd", s, by, fl);
   // forward: the per-wave fragment-stream kernel by default (measured 165 against 174 us at
   // T170 x 360); DSHT_TUNE_LEG = 1 or 3 selects the LDS-staged kernel
   if (p->leg_kind == 0 && leg_fwd_staged_ok(p, op)) return launch_leg_fwd_staged(p, op, a, s);
+  if (op == F_VALSUBALPHA || a.add) return fail(DSHT_EUNSUPPORTED, "launch_leg_fwd: op %d needs the staged kernel", op);
   if (p->leg_kind == 0 || p->leg_kind == 2) return launch_leg_fwd_direct(p, op, a, s);
   switch (op) {
     case F_VAL: return wide ? fwd_pick<F_VAL, 32>(p, a, s) : fwd_pick<F_VAL, 16>(p, a, s);

@@ -238,6 +238,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
   constexpr int NTB = (UP ? 1 : 0) + (UH ? 1 : 0);
   constexpr int U = 4;                  // K steps of table fragments per chunk
   constexpr int NP = NOUT;              // inputs multiplied by each table
+  constexpr int NLD = OP == F_VALSUBALPHA ? 3 : NIN;  // Fourier arrays read
   constexpr int UB = NIN == 2 ? 2 : 4;  // staged latitude pairs per thread and round
   int m, sub;
   if (!xcd_decode_wk(a.N, CB * RG, m, sub)) return;
@@ -248,7 +249,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
   const int tE = cdiv(nE, TILE), RT = tE + cdiv(nO, TILE);
   const int nks = a.J2pad / 4, KR = a.J2pad;  // whole chunks: J2pad is a multiple of 16
   const int c0 = cb * C8;
-  const double2* Gm[2] = {a.G0 + (long)m * a.gmst, NIN > 1 ? a.G1 + (long)m * a.gmst : nullptr};
+  const double2* Gm[3] = {a.G0 + (long)m * a.gmst, NLD > 1 ? a.G1 + (long)m * a.gmst : nullptr,
+                          NLD > 2 ? a.G2 + (long)m * a.gmst : nullptr};
   const double dm = (double)m;
 
   // ---- stage: a thread stays in one column and takes every RS-th latitude pair; every load of a
@@ -259,8 +261,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
   const long co = cok ? c0 + cc : 0;
   double* put = wk_lds + (cc / 8) * KR * 16 + 2 * (cc % 8);
   for (int j0 = tid / C8; j0 < KR; j0 += RS * UB) {
-    double2 gn[NIN][UB], gs[NIN][UB];
-    double cw[UB];
+    double2 gn[NLD][UB], gs[NLD][UB];
+    double cw[UB], cw2[UB];
     bool ok[UB];
 #pragma unroll
     for (int q = 0; q < UB; q++) {
@@ -268,9 +270,10 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
       ok[q] = j < J2 && cok;
       const int jj = ok[q] ? j : 0;
       cw[q] = a.cw[jj];
+      if constexpr (NLD == 3) cw2[q] = a.cw2[jj];
       const long n = (J2 + jj) * a.gld + co, s = (J2 - 1 - jj) * a.gld + co;
 #pragma unroll
-      for (int i = 0; i < NIN; i++) {
+      for (int i = 0; i < NLD; i++) {
         gn[i][q] = Gm[i][n];
         gs[i][q] = Gm[i][s];
       }
@@ -281,11 +284,25 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
       if (j < KR) {
 #pragma unroll
         for (int i = 0; i < NIN; i++) {
-          double2 s, d;
-          s.x = ok[q] ? cw[q] * (gn[i][q].x + gs[i][q].x) : 0.0;
-          s.y = ok[q] ? cw[q] * (gn[i][q].y + gs[i][q].y) : 0.0;
-          d.x = ok[q] ? cw[q] * (gn[i][q].x - gs[i][q].x) : 0.0;
-          d.y = ok[q] ? cw[q] * (gn[i][q].y - gs[i][q].y) : 0.0;
+          double2 s = make_double2(gn[i][q].x + gs[i][q].x, gn[i][q].y + gs[i][q].y);
+          double2 d = make_double2(gn[i][q].x - gs[i][q].x, gn[i][q].y - gs[i][q].y);
+          if constexpr (OP == F_VALSUBALPHA) {
+            const double f = cw[q] * a.ralpha;
+            if (i == 0) {  // with P: c' C - c i m A / R
+              const double2 sa = s, da = d;
+              s.x = cw2[q] * (gn[2][q].x + gs[2][q].x) + f * (dm * sa.y);
+              s.y = cw2[q] * (gn[2][q].y + gs[2][q].y) - f * (dm * sa.x);
+              d.x = cw2[q] * (gn[2][q].x - gs[2][q].x) + f * (dm * da.y);
+              d.y = cw2[q] * (gn[2][q].y - gs[2][q].y) - f * (dm * da.x);
+            } else {  // with H: c B / R
+              s = make_double2(f * s.x, f * s.y);
+              d = make_double2(f * d.x, f * d.y);
+            }
+          } else {
+            s = make_double2(cw[q] * s.x, cw[q] * s.y);
+            d = make_double2(cw[q] * d.x, cw[q] * d.y);
+          }
+          if (!ok[q]) s = d = make_double2(0.0, 0.0);
           double* at = put + i * 2 * NCT * KR * 16 + j * 16;
           *(double2*)at = s;
           *(double2*)(at + NCT * KR * 16) = d;
@@ -333,10 +350,10 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
 #pragma unroll
           for (int i = 0; i < NP; i++) {
             const int o = ct * KR * 16 + (ks + u) * 64, in = 2 * NCT * KR * 16;
-            // ALPHA: P with input 0, H with input 1; UV2VORDIV: both with both
+            // ALPHA, VALSUBALPHA: P with input 0, H with input 1; UV2VORDIV: both with both
             if constexpr (UP) acc[0][i][ct] = mfma64(cur[0][u], BP[o + i * in], acc[0][i][ct]);
             if constexpr (UH)
-              acc[NTB - 1][i][ct] = mfma64(cur[NTB - 1][u], BH[o + (OP == F_ALPHA ? 1 : i) * in], acc[NTB - 1][i][ct]);
+              acc[NTB - 1][i][ct] = mfma64(cur[NTB - 1][u], BH[o + (NIN == 2 && NOUT == 1 ? 1 : i) * in], acc[NTB - 1][i][ct]);
           }
       // the copies (and their wait for the fragments) stay behind the products
       __builtin_amdgcn_sched_barrier(0);
@@ -353,15 +370,17 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
     for (int ct = 0; ct < NCT; ct++) {
       const int c = c0 + ct * 8 + (col >> 1);
       if (c >= a.ncols) continue;
-      // the four rows' diagonals in one round of loads
-      double dv[NOUT][4];
+      // the four rows' diagonals, and the values to add to, in one round of loads
+      double dv[NOUT][4], old[NOUT][4];
 #pragma unroll
       for (int o = 0; o < NOUT; o++) {
         const double* dg = o == 0 ? a.diag0 : a.diag1;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           const int n = m + par + 2 * ((par ? t - tE : t) * TILE + krow + 4 * i);
-          dv[o][i] = dg ? dg[n <= N ? n * (n + 1) + (part ? -m : m) : 0] : 1.0;
+          const int l = n <= N ? n * (n + 1) + (part ? -m : m) : 0;
+          dv[o][i] = dg ? dg[l] : 1.0;
+          if constexpr (OP == F_VAL) old[o][i] = a.add ? a.W0[l * a.sl + (long)c * a.sc] : 0.0;
         }
       }
 #pragma unroll
@@ -376,6 +395,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
           v[0] = -acc[0][0][ct][i];
         } else if constexpr (OP == F_ALPHA) {  // i m P.A - H.B
           v[0] = im * other_part(acc[0][0][ct][i]) - acc[NTB - 1][0][ct][i];
+        } else if constexpr (OP == F_VALSUBALPHA) {
+          v[0] = acc[0][0][ct][i] + acc[NTB - 1][0][ct][i];
         } else {  // inputs U cos (0), V cos (1): vor = i m P.V + H.U, div = i m P.U - H.V
           v[0] = im * other_part(acc[0][NP - 1][ct][i]) + acc[NTB - 1][0][ct][i];
           v[NOUT - 1] = im * other_part(acc[0][0][ct][i]) - acc[NTB - 1][NP - 1][ct][i];
@@ -383,7 +404,11 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
         if (n > N || (m == 0 && part)) continue;
         const long at = (n * (n + 1) + (part ? -m : m)) * a.sl + (long)c * a.sc;
 #pragma unroll
-        for (int o = 0; o < NOUT; o++) (o == 0 ? a.W0 : a.W1)[at] = v[o] * a.scale * dv[o][i];
+        for (int o = 0; o < NOUT; o++) {
+          double* W = (o == 0 ? a.W0 : a.W1) + at;
+          const double x = v[o] * a.scale * dv[o][i];
+          *W = OP == F_VAL && a.add ? old[o][i] + x : x;
+        }
       }
     }
   }
@@ -471,7 +496,7 @@ bool leg_inv_staged_ok(const dsht_plan* p, int op) {
   return (inv_nin(op) == 2 ? inv_lds<I_ALPHA, 1>(p) : inv_lds<I_VAL, 1>(p)) <= WK_LDS_MAX;
 }
 bool leg_fwd_staged_ok(const dsht_plan* p, int op) {
-  return (op == F_ALPHA || op == F_UV2VORDIV ? fwd_lds<F_ALPHA, 1>(p) : fwd_lds<F_VAL, 1>(p)) <= WK_LDS_MAX;
+  return (op >= F_ALPHA ? fwd_lds<F_ALPHA, 1>(p) : fwd_lds<F_VAL, 1>(p)) <= WK_LDS_MAX;
 }
 
 int launch_leg_inv_staged(const dsht_plan* p, int op, const LegInvArgs& a, hipStream_t s) {
@@ -493,6 +518,7 @@ int launch_leg_fwd_staged(const dsht_plan* p, int op, const LegFwdArgs& a, hipSt
     case F_DIVMU: return fwd_op<F_DIVMU>(p, a, s);
     case F_ALPHA: return fwd_op<F_ALPHA>(p, a, s);
     case F_UV2VORDIV: return fwd_op<F_UV2VORDIV>(p, a, s);
+    case F_VALSUBALPHA: return fwd_op<F_VALSUBALPHA>(p, a, s);
   }
   return fail(DSHT_EARG, "launch_leg_fwd_staged: bad op %d", op);
 }

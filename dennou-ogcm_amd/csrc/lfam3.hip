@@ -207,13 +207,10 @@ __global__ __launch_bounds__(256) void k_lf_mom(
   }, above);
 }
 
-// w_out[l, c] += w_in[l, c] * s  (s = 1, or 1/(RefDens R^2) for the barotropic pressure term)
-__global__ void k_lf_spec_axpy(double* __restrict__ wout, long slo, const double* __restrict__ win, long sli, int L,
-                               int ncols, double s, int divide) {
-  LF_CP(L, ncols) {
-    const double x = win[c * sli + p];
-    wout[c * slo + p] += divide ? x / s : x;
-  }
+// w_out[l, c] += w_in[l, c]
+__global__ void k_lf_spec_add(double* __restrict__ wout, long slo, const double* __restrict__ win, long sli, int L,
+                              int ncols) {
+  LF_CP(L, ncols) wout[c * slo + p] += win[c * sli + p];
 }
 
 // The thickness-weighted layer means of U and V (HBEDiagnose_UVBarot, HBEDiagnose_hspm_vfvm_mod.f90:
@@ -587,7 +584,7 @@ struct dsht_lfam3 {
   double *d_cdk = nullptr, *d_fdk = nullptr, *d_rcdk = nullptr, *d_rfdk = nullptr, *d_zck = nullptr;
   double *d_mu = nullptr, *d_cs = nullptr, *d_two_omega = nullptr;
   double *d_m1 = nullptr, *d_m2 = nullptr, *d_dfac = nullptr;  // QUICK weights per half level
-  double *d_dmom = nullptr, *d_dtrc = nullptr, *d_advf = nullptr, *d_nn1 = nullptr, *d_hcoef = nullptr,
+  double *d_dmom = nullptr, *d_dtrc = nullptr, *d_advf = nullptr, *d_nn1 = nullptr, *d_nn1p = nullptr, *d_hcoef = nullptr,
          *d_e = nullptr;
   // state: levels B (0), N (1), A (2)
   double *U[3] = {}, *V[3] = {}, *TS[3] = {}, *SP[3] = {};
@@ -731,6 +728,15 @@ int lf_uv2vordiv(dsht_lfam3* s, const double* u, const double* v, int nc, const 
   return dsht_uv2vordiv_d(p, s->ucos, s->vcos, s->np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, diag, st);
 }
 
+// w += diag w_xy(x) over nc columns of pitch sl (tmp: spectra for forms that do not add)
+int lf_fwd_add(dsht_lfam3* s, const double* x, double* w, long sl, double* tmp, int nc, const double* diag,
+               hipStream_t st) {
+  if (fwd_fused_ok(s->p)) return fwd_add(s->p, x, s->np, w, sl, 1, nc, diag, st);
+  if (int rc = dsht_fwd_d(s->p, DSHT_VAL, x, s->np, tmp, nc, 1, nc, diag, st)) return rc;
+  LF_LAUNCH2(k_lf_spec_add, s->L, nc, st, w, sl, tmp, (long)nc, s->L, nc);
+  return 0;
+}
+
 // HBEDiagnose_VorDiv (HBEDiagnose_hspm_vfvm_mod.f90:259-286) over every layer of the active
 // runs: vorticity into VD[0, nc), divergence into VD[nc, 2 nc)
 int lf_vordiv(dsht_lfam3* s, const double* u, const double* v, int nc, hipStream_t st) {
@@ -755,8 +761,7 @@ int lf_mom_rhs(dsht_lfam3* s, const double* u, const double* v, const double* xa
   // (w_Vor_RHS, w_Div_RHS) = (-H(A, B), H(B, -A)) = calc_UVCosLat2VorDiv(B, -A); then
   // w_Div_RHS - w_Lapla_w(w_xy(C)) = + n(n+1) w_xy(C)
   if (int rc = dsht_uv2vordiv_d(p, s->Bg, s->Am, s->np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, nullptr, st)) return rc;
-  if (int rc = dsht_fwd_d(p, DSHT_VAL, s->Cg, s->np, s->wC, nc, 1, nc, s->d_nn1, st)) return rc;
-  LF_LAUNCH2(k_lf_spec_axpy, s->L, nc, st, s->wVD + nc, 2l * nc, s->wC, (long)nc, s->L, nc, 1.0, 0);
+  if (int rc = lf_fwd_add(s, s->Cg, s->wVD + nc, 2l * nc, s->wC, nc, s->d_nn1, st)) return rc;
   return dsht_vordiv2uv_d(p, s->wVD, s->wVD + nc, 2l * nc, 1, s->URHS, s->VRHS, s->np, nc, st);
 }
 
@@ -768,9 +773,14 @@ int lf_htrc(dsht_lfam3* s, const double* ts, const double* u, const double* v, d
   const int nc = nr * s->K, nt = 2 * nc;
   LF_LAUNCHC(k_lf_htrc, np, nr, 1, st, ts, u, v, s->VD + (long)nc * np, s->cfg.depth, h, s->d_cs, s->d_cdk, s->d_rcdk,
              s->d_rfdk, s->d_m1, s->d_m2, s->d_dfac, np, s->I, s->K, s->FU, s->FV, s->VF);
-  if (int rc = dsht_alpha_fwd_d(p, s->FU, s->FV, np, s->w1, nt, 1, nt, nullptr, st)) return rc;
-  if (int rc = dsht_fwd_d(p, DSHT_VAL, s->VF, np, s->w2, nt, 1, nt, nullptr, st)) return rc;
-  LF_LAUNCH2(k_lf_htrc_spec, s->L, nt, st, s->w1, s->w2, s->d_advf, s->L, nt);
+  // w = AdvFilter (-w_AlphaOptr_xy(fluxes) + w_xy(divergence)) (:163-171)
+  if (fwd_fused_ok(p)) {
+    if (int rc = val_sub_alpha(p, s->FU, s->FV, s->VF, np, s->w1, nt, 1, nt, s->d_advf, st)) return rc;
+  } else {
+    if (int rc = dsht_alpha_fwd_d(p, s->FU, s->FV, np, s->w1, nt, 1, nt, nullptr, st)) return rc;
+    if (int rc = dsht_fwd_d(p, DSHT_VAL, s->VF, np, s->w2, nt, 1, nt, nullptr, st)) return rc;
+    LF_LAUNCH2(k_lf_htrc_spec, s->L, nt, st, s->w1, s->w2, s->d_advf, s->L, nt);
+  }
   return dsht_inv_d(p, DSHT_VAL, s->w1, nt, 1, s->HT, np, nt, nullptr, st);
 }
 
@@ -867,12 +877,13 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
     m2[h] = s->cdk[h - 1] / sum;
     dfac[h] = (0.125 * s->cdk[h]) * s->cdk[h - 1];
   }
-  std::vector<double> cs(J), nn1(L), e(L), hcoef(L);
+  std::vector<double> cs(J), nn1(L), nn1p(L), e(L), hcoef(L);
   for (int j = 0; j < J; j++) cs[j] = std::sqrt((1.0 - p->mu[j]) * (1.0 + p->mu[j]));
   for (int n = 0; n <= p->N; n++)
     for (int m = -n; m <= n; m++) {
       const int l = n * (n + 1) + m;
       nn1[l] = (double)n * (n + 1.0);
+      nn1p[l] = nn1[l] / (c.ref_dens * (p->R * p->R));  // of the barotropic pressure term
       e[l] = (double)n * (n + 1.0) / (p->R * p->R);
       hcoef[l] = l == 0 ? 0.0 : 1.0 / (e[l] + 0.0);  // w_Coef, HBEBarot_hspm_vfvm_mod.f90:281-290
     }
@@ -894,6 +905,7 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
   U(&s->d_mu, p->mu);
   U(&s->d_cs, cs);
   U(&s->d_nn1, nn1);
+  U(&s->d_nn1p, nn1p);
   U(&s->d_e, e);
   U(&s->d_hcoef, hcoef);
   U(&s->d_two_omega, std::vector<double>(R, 2.0 * 7.292115e-5));
@@ -1105,8 +1117,7 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   // ---- barotropic mode: one iteration with dts = dt / SubCycleNum (rigid lid)
   const double dts = dt / c.sub_cycles;
   if ((rc = dsht_uv2vordiv_d(p, b2[BG2], b2[AM2], np, s->wB, s->wB + nr, 2l * nr, 1, nr, nullptr, st))) return rc;
-  if ((rc = dsht_fwd_d(p, DSHT_VAL, b2[SPM], np, s->wC2, nr, 1, nr, s->d_nn1, st))) return rc;
-  LF_LAUNCH2(k_lf_spec_axpy, L, nr, st, s->wB + nr, 2l * nr, s->wC2, (long)nr, L, nr, c.ref_dens * (p->R * p->R), 1);
+  if ((rc = lf_fwd_add(s, b2[SPM], s->wB + nr, 2l * nr, s->wC2, nr, s->d_nn1p, st))) return rc;
   if ((rc = dsht_vordiv2uv_d(p, s->wB, s->wB + nr, 2l * nr, 1, b2[UBR], b2[VBR], np, nr, st))) return rc;
   LF_LAUNCH2(k_lf_barot_step, nr, np, st, b2[UBR], b2[VBR], b2[UBN], b2[VBN], s->d_two_omega, s->d_mu, s->d_cs, np, I,
              alpha_ * dts, dts, (long)nr, b2[UBAR], b2[VBAR], b2[AM2], b2[BG2]);

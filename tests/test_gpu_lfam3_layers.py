@@ -55,9 +55,11 @@ def test_layers_match_oracle(gpu, km, cfg):
         assert np.array_equal(got["UB"], ref["UB"])
 
 
-def test_winds_scaled_in_fft_or_before(gpu):
-    """cos(lat) applied as the register FFT reads the winds, and by a pass over them where the
-    plan uses the LDS FFT (DSHT_TUNE_FFT = 1): one step either way, 1e-9 as above."""
+@pytest.mark.parametrize("key", ["TUNE_FFT", "TUNE_LEG"])
+def test_fused_equals_separate(gpu, key):
+    """The step's fused transforms (cos(lat) inside the FFT, w_xy(C) - w_AlphaOptr_xy(A, B) and
+    w += w_xy(x) in one contraction) against the separate passes it takes where the plan uses the
+    LDS FFT (DSHT_TUNE_FFT = 1) or the fragment-stream contractions (DSHT_TUNE_LEG = 2)."""
     import torch
     import dsht
     import lfam3
@@ -67,9 +69,9 @@ def test_winds_scaled_in_fft_or_before(gpu):
     o = oracle.Oracle(N, I, J, 6.371e6)
     st = lfam3.initial_state(o, km, seed=5)
     got = []
-    for kind in (0, 1):
+    for kind in (0, {"TUNE_FFT": 1, "TUNE_LEG": 2}[key]):
         p, pool = _pool(N, I, J, km, 1, dt=1800.0)
-        p.set_tuning(dsht.TUNE_FFT, kind)
+        p.set_tuning(getattr(dsht, key), kind)
         _load(pool, 0, st)
         pool.set_rotation(0, OMEGA)
         torch.cuda.synchronize()
