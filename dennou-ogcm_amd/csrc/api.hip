@@ -239,23 +239,24 @@ static int run_inv(dsht_plan* p, int op, const double* in0, const double* in1, l
     a.J2 = p->J2;
     a.J2pad = p->J2pad;
     if ((rc = launch_leg_inv(p, op, a, s))) return rc;
-    // the field and its longitude derivative as two launches over the same G0: the FP64
-    // dual kernel (one read of G0, coefficients held in registers across both passes) ran
-    // slower at T170L60 (2 x 125 against 2 x 80 us per step's worth), the FP32 one faster
+    // every grid from one launch, the longitude derivative as a second reader of G0 (the FP64
+    // kernel that holds the coefficients in registers for both ran slower: 2 x 125 against
+    // 2 x 80 us per T170L60 step's worth; the FP32 one faster)
     const double2* gs[3];
     double* xs[3];
-    int nf = 0;
+    int nf = 0, deriv = 0;
     auto add = [&](const double2* g, double* x) {
       gs[nf] = g;
       xs[nf++] = x + (long)c0 * ldg;
     };
     if (out0) add(G0, out0);
+    if (dlon) {
+      deriv = 1 << nf;
+      add(G0, out1);
+    }
     if (a.G1) add(G1, out1);
     if (a.G2) add(G2, out2);
-    if (nf && (rc = launch_fft_inv(p, gs, nf, a.gld, nc, xs, ldg, s))) return rc;
-    nf = 0;
-    if (dlon) add(G0, out1);
-    if (nf && (rc = launch_fft_inv(p, gs, nf, a.gld, nc, xs, ldg, s, p->d_rs_icos, 1))) return rc;
+    if ((rc = launch_fft_inv(p, gs, nf, a.gld, nc, xs, ldg, s, dlon ? p->d_rs_icos : nullptr, deriv))) return rc;
   }
   return 0;
 }

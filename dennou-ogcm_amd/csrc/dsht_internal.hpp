@@ -130,7 +130,8 @@ struct FftArgs {
   int threads;             // workgroup size of the register kernels (128 or 256)
   int fp32;                // FP32 arithmetic (FP32 Fourier path of the split forms)
   int order;               // row-group order of the register kernels (0 packed, 1 latitude-major)
-  int deriv;               // inverse: transform i m X_m (longitude derivative) instead of X_m
+  int deriv;               // inverse: transform i m X_m (longitude derivative) instead of X_m; with
+                           // several fields bit i for field i, and rowscale only for those
   void* xy2;               // inverse, dual form: the field into xy and its longitude derivative
                            // (times rowscale) into xy2 from one read of the coefficients (nullable)
   int nf;                  // fields in one launch (FP64 register kernels; grid y), each of ncols columns
@@ -258,7 +259,8 @@ void fft_plan_free(dsht_plan* p);
 int launch_fft_fwd(const dsht_plan* p, const double* const* xy, int nf, long ldg, int ncols, double2* const* G, long gld,
                    hipStream_t s, const double* rowscale = nullptr);
 // rowscale: per-latitude factor on the outputs (nullable); deriv: transform i m X_m (the
-// longitude derivative of the field), register kernels only
+// longitude derivative of the field), register kernels only; with several fields bit i stands
+// for field i and rowscale applies to those fields alone
 bool fft_reg_ok(const dsht_plan* p);
 int launch_fft_inv(const dsht_plan* p, const double2* const* G, int nf, long gld, int ncols, double* const* xy, long ldg,
                    hipStream_t s, const double* rowscale = nullptr, int deriv = 0);

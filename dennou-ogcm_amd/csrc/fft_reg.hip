@@ -447,8 +447,9 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_fwd_r(const XT* __restrict__
 // MODE 0: the field; 1: its longitude derivative (transform i m X_m, times a.rowscale);
 // 2 (dual): both from one read of the coefficients -- the field into xy, then the
 // derivative, times a.rowscale, into a.xy2 -- the coefficients stay in registers between the
-// two passes.  Separate instantiations keep each form's register allocation.  XT: grid
-// element type.
+// two passes; 3: fields of one launch (grid y) of either kind, bit y of a.deriv set for the
+// derivative of field y.  Separate instantiations keep each form's register allocation.  XT:
+// grid element type.
 template <int R1, int R2, int NT, typename GT, typename V, int MODE, typename XT>
 __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__ G, XT* __restrict__ xy,
                                                   FftArgs a) {
@@ -506,7 +507,7 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__
     if (!PF) fetch(g0);
 #pragma unroll
   for (int pass = 0; pass < NPASS; pass++) {
-    const bool deriv = MODE == 1 || (MODE == 2 && pass == 1);
+    const bool deriv = MODE == 1 || (MODE == 2 && pass == 1) || (MODE == 3 && ((a.deriv >> blockIdx.y) & 1));
     __syncthreads();  // the previous rows are out of buf
 #pragma unroll
     for (int q = 0; q < NL; q++) {
@@ -565,7 +566,7 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__
       int j, c;
       if (map_row(a, g0, rr2, ROWS, j, c)) {
         // dual: the field unscaled into xy, the derivative times the row scale into xy2
-        const double s = (a.rowscale && (MODE != 2 || pass == 1)) ? a.rowscale[j] : 1.0;
+        const double s = (a.rowscale && (MODE < 2 || deriv)) ? a.rowscale[j] : 1.0;
         XT* out = (MODE == 2 && pass == 1) ? reinterpret_cast<XT*>(a.xy2) : xy;
         XT* x = out + c * a.ldg + (long)j * (2 * M);
 #pragma unroll
@@ -641,6 +642,9 @@ static int reg_inv_mode(const GT* G, const FftArgs& a, XT* xy, hipStream_t s) {
 template <int R1, int R2, int NT, typename GT, typename V, typename XT>
 static int reg_inv_nt(const GT* G, const FftArgs& a, XT* xy, hipStream_t s) {
   if (a.xy2) return reg_inv_mode<R1, R2, NT, GT, V, 2, XT>(G, a, xy, s);
+  if constexpr (sizeof(GT) == 16) {
+    if (a.deriv && a.nf > 1) return reg_inv_mode<R1, R2, NT, GT, V, 3, XT>(G, a, xy, s);
+  }
   if (a.deriv) return reg_inv_mode<R1, R2, NT, GT, V, 1, XT>(G, a, xy, s);
   return reg_inv_mode<R1, R2, NT, GT, V, 0, XT>(G, a, xy, s);
 }
