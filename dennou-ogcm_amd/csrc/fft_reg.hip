@@ -484,11 +484,12 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__
   GT gr[NL];
   // with THREADS a multiple of ROWS every item idx = tid + q * THREADS is in row tid % ROWS
   constexpr bool FIXR = C::THREADS % ROWS == 0;
-  auto fetch = [&](long g) {
+  // items [FROM, TO) of a thread's NL
+  auto fetch = [&](long g, auto FROM, auto TO) {
     int j0 = 0, c0 = 0;
     const bool ok0 = FIXR && map_row(a, g, tid % ROWS, ROWS, j0, c0);
 #pragma unroll
-    for (int q = 0; q < NL; q++) {
+    for (int q = decltype(FROM)::value; q < decltype(TO)::value; q++) {
       const int idx = tid + q * C::THREADS;
       const int m = idx / ROWS;
       gr[q] = cvt<GT>(make_float2(0.f, 0.f));
@@ -497,14 +498,24 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__
       if (ok && idx < M * ROWS && m <= N) gr[q] = G[(long)m * a.gmst + (long)j * a.gld + c];
     }
   };
-  // prefetching holds the next group in registers through the whole pipeline: only where
-  // that fits the register budget (FP32 coefficients, M <= 256)
-  constexpr bool PF = sizeof(GT) == 8 && M <= 256;
+  // prefetching holds the next group in registers through the whole pipeline: everything where
+  // that fits the register budget (FP32 coefficients, M <= 256).  Of FP64 coefficients the items
+  // below two thirds of M, all that an alias-free grid's truncation has, where the kernel runs
+  // two waves per SIMD either way and the registers are free (M = 192 and 256; 120 fields of
+  // 512 x 256: 45.6 -> 42.4 us).  Not at M = 128 (50 -> 56 us: a wave per SIMD less) and not with
+  // the per-field derivative, whose several fields a launch already overlap (258 -> 256..260 us)
+  constexpr int PF = sizeof(GT) == 8 && M <= 256 ? NL
+                     : sizeof(GT) == 16 && (M == 192 || M == 256) && MODE < 2
+                         ? ((2 * M / 3 + 2) * ROWS + C::THREADS - 1) / C::THREADS
+                         : 0;
+  const std::integral_constant<int, 0> i0;
+  const std::integral_constant<int, PF> ipf;
+  const std::integral_constant<int, NL> inl;
   constexpr int NPASS = MODE == 2 ? 2 : 1;
   const long gstep = gridDim.x;
-  if (PF && (long)blockIdx.x < ngroups) fetch(blockIdx.x);
+  if (PF && (long)blockIdx.x < ngroups) fetch(blockIdx.x, i0, ipf);
   for (long g0 = blockIdx.x; g0 < ngroups; g0 += gstep) {
-    if (!PF) fetch(g0);
+    if (PF < NL) fetch(g0, ipf, inl);
 #pragma unroll
   for (int pass = 0; pass < NPASS; pass++) {
     const bool deriv = MODE == 1 || (MODE == 2 && pass == 1) || (MODE == 3 && ((a.deriv >> blockIdx.y) & 1));
@@ -518,7 +529,7 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__
         buf[(idx % ROWS) * SR + idx / ROWS] = v;
       }
     }
-    if (PF && pass == NPASS - 1 && g0 + gstep < ngroups) fetch(g0 + gstep);
+    if (PF && pass == NPASS - 1 && g0 + gstep < ngroups) fetch(g0 + gstep, i0, ipf);
     __syncthreads();
     // packed spectrum Z_m from the half-complex pair (X_m, X_{M-m}); X_M = 0 for m = 0
     for (int idx = tid; idx < ROWS * (M / 2 + 1); idx += C::THREADS) {
