@@ -2,13 +2,13 @@
 // (LPhys_RediGM_hspm_vfvm_AddMixingTerm, model/dogcm/src/physics/lphys/
 // LPhys_RediGM_hspm_vfvm_mod.f90:218-372) on device grids.
 //
-// One thread per grid point walks its column.  A first pass finds the two LDD95 tapering
-// depths (the surface and bottom scans of TaperingFunc_LDD95, LPhys_RediGMHelper_mod.f90:
-// 392-428): it evaluates the slopes of the top layers down to the first layer deeper than
-// the eddy displacement and of the bottom layers up to the first one higher than it above
-// the bottom, and stops there, as the reference's scans exit.  The second pass walks every
-// layer once with a one-layer window: vertical differences on the half levels (calc_GradTRC
-// :412-424), the JM95 expansion coefficients and the slopes (calc_IsoNeutralSlope_new
+// k_redigm_scan finds the two LDD95 tapering depths of each column (the surface and bottom scans
+// of TaperingFunc_LDD95, LPhys_RediGMHelper_mod.f90:392-428; one thread a column and direction):
+// it evaluates the slopes of the top layers down to the first layer deeper than the eddy
+// displacement and of the bottom layers up to the first one higher than it above the bottom, and
+// stops there, as the reference's scans exit.  k_redigm_col then walks the layers, one thread a
+// column and segment of layers, with a one-layer window: vertical differences on the half levels
+// (calc_GradTRC :412-424), the JM95 expansion coefficients and the slopes (calc_IsoNeutralSlope_new
 // :745-775), the taper (DM95 or GKW91 times LDD95), the Redi and skew fluxes of both tracers
 // on the layer and on the half level above it (calc_IsopycDiffFlux :497-553, calc_SkewFlux
 // :607-676), and writes per tracer (FLonRedi + FLonGM) cos(lat), (FLatRedi + FLatGM)
@@ -17,13 +17,19 @@
 // operations and no multiply-add is contracted, so the results equal the reference loops in
 // FP64 up to the last bit of tanh and sin.
 //
-// Bound: HBM.  Algorithmic bytes per call: the 8 input layer fields (ptemp, salt, h, z, the
-// four gradients) and the 6 output layer fields once: (14 km + 1) I J 8 bytes; the first
-// pass rereads the few layers of the scans.
+// Bound: HBM and, close to it, the vector issue (about 410 instructions a layer, 285 of them FP64).
+// Algorithmic bytes per call: the 8 input layer fields (ptemp, salt, h, z, the four gradients)
+// and the 6 output layer fields once: (14 km + 1) I J 8 bytes; the scans reread a few layers.
+// 512 x 256 x 60: scan 46 us, walk 189 us (4.9 TB/s); both in one kernel of one thread a column
+// took 284 us.  What the difference was: the layer thicknesses' reciprocals were loaded from memory
+// behind the next layer's loads, and so waited for them (rfdk is in LDS now); 13 full divisions a
+// layer (now 4 reciprocals and corrected quotients); tanh (now one exp); 208 registers.
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "dsht_internal.hpp"
 
@@ -49,9 +55,46 @@ struct RediArgs {
   const double *pt, *sa, *h, *z, *topo, *cdk, *rfdk, *glon, *glat, *lat_cs;
   double *flon, *flat, *vdiv;
   long ldg, ldgr, ldo, npts;  // pitches: inputs, gradients, outputs
-  int km, I, J, gkw91;
-  double R, rg, kr, kg, smax, sd, two_omega;
+  int km, I, J, gkw91, seg;  // seg: layers a thread of the walk writes
+  double R, rR, rg, kr, kg, smax, sd, two_omega;  // rR: 1/R, or 0 where R is outside recip_ok
 };
+
+// Quotients by one divisor d from its reciprocal: two Newton steps on the hardware estimate, and a
+// quotient corrected by its exact remainder (Markstein, IBM J. Res. Dev. 34, 1990), which rounds as
+// the division does where no intermediate leaves the normal range.  A divisor outside
+// (2^-900, 2^900), 0, an infinity or NaN is divided by as such.
+__device__ inline bool recip_ok(double d) {
+  const double m = fabs(d);
+  return m > 0x1p-900 && m < 0x1p900;
+}
+__device__ inline double recip(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+}
+__device__ inline double quot(double n, double d, double r) {
+  const double q = n * r;
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d, q, n), r, q), d, n);
+}
+__device__ inline void div2(double n0, double n1, double d, double r, double& q0, double& q1) {
+  if (__builtin_expect(recip_ok(d), 1)) {
+    q0 = quot(n0, d, r);
+    q1 = quot(n1, d, r);
+  } else {
+    q0 = n0 / d;
+    q1 = n1 / d;
+  }
+}
+
+// tanh(x): 1 - 2 / (exp(2|x|) + 1) with x's sign where |x| >= 1, whose subtrahend is below 0.24,
+// so that its rounding stays under that of the difference
+__device__ inline double taper_tanh(double x) {
+  const double y = fabs(x);
+  if (!(y >= 1.0)) return tanh(x);  // and NaN
+  const double d = exp(y > 25.0 ? 50.0 : 2.0 * y) + 1.0;
+  const double r = recip(d), q = 2.0 * r;
+  return copysign(1.0 - __builtin_fma(__builtin_fma(-d, q, 2.0), r, q), x);
+}
 
 // EOSDriver_alpha_beta with p = -RefDens*Grav*z [Pa] (calc_IsoNeutralSlope_new :740-743):
 // K2degC(theta), Pa2bar(p)*10 (EOSDriver_mod.f90), then the JM95 polynomials
@@ -85,10 +128,10 @@ struct Lay {
 };
 
 // the slopes of layer k (calc_IsoNeutralSlope_new :745-775)
-__device__ inline void layer_slopes(const RediArgs& a, int k, double tm, double tc, double tp, double sm, double sc,
+__device__ inline void layer_slopes(const RediArgs& a, const double* rfdk, int k, double tm, double tc, double tp, double sm, double sc,
                                     double sp, double z, Lay& L) {
-  dsig_pair(k, a.km, a.rfdk, tm, tc, tp, L.da[0], L.db[0]);
-  dsig_pair(k, a.km, a.rfdk, sm, sc, sp, L.da[1], L.db[1]);
+  dsig_pair(k, a.km, rfdk, tm, tc, tp, L.da[0], L.db[0]);
+  dsig_pair(k, a.km, rfdk, sm, sc, sp, L.da[1], L.db[1]);
   double al, be;
   jm95_alpha_beta(tc, sc, z, a.rg, al, be);
   const double den = (1e-10 + (al * 0.5) * (L.da[0] + L.db[0])) - (be * 0.5) * (L.da[1] + L.db[1]);
@@ -103,19 +146,131 @@ struct Pre {
   double h, z, g0, a0, g1, a1, tn, sn;
 };
 
-constexpr int RING = 2;  // layers whose loads are in flight ahead of the one being computed
+constexpr int SRING = 2;  // layers whose loads the scans have in flight ahead of the one being computed
 
 constexpr int REDI_LDS_LAYERS = 1024;  // layers whose half-level weights the block keeps in LDS
 
-__global__ __launch_bounds__(256, 2) void k_redigm_col(RediArgs a) {
+// a uniform layer base and the point's byte offset (I J < 2^29)
+__device__ inline double ld(const double* base, unsigned qb) { return *(const double*)((const char*)base + qb); }
+__device__ inline void st(double* base, unsigned qb, double v) { *(double*)((char*)base + qb) = v; }
+
+// dir = +1: the next layer is k+1 (downward walk); -1: k-1 (upward)
+__device__ inline void fetch_layer(const RediArgs& a, unsigned qb, int k, int dir, Pre& f) {
+  const long g = (long)k * a.ldg, gr = (long)k * a.ldgr, TS = (long)a.km * a.ldgr;
+  f.h = ld(a.h + g, qb);
+  f.z = ld(a.z + g, qb);
+  f.g0 = ld(a.glon + gr, qb);
+  f.a0 = ld(a.glat + gr, qb);
+  f.g1 = ld(a.glon + TS + gr, qb);
+  f.a1 = ld(a.glat + TS + gr, qb);
+  const int kn = k + dir;
+  const bool in = kn >= 0 && kn < a.km;
+  f.tn = in ? ld(a.pt + g + dir * a.ldg, qb) : 0.0;
+  f.sn = in ? ld(a.sa + g + dir * a.ldg, qb) : 0.0;
+}
+
+// layer k's slopes from its loads and ptemp/salt at k-1, k, k+1
+__device__ inline void slopes_of(const RediArgs& a, const double* rfdk, int k, const Pre& f, double tm, double tc,
+                                 double tp, double sm, double sc, double sp, Lay& L) {
+  L.h = f.h;
+  if (a.rR != 0.0) {
+    L.gl[0] = quot(f.g0, a.R, a.rR);
+    L.ga[0] = quot(f.a0, a.R, a.rR);
+    L.gl[1] = quot(f.g1, a.R, a.rR);
+    L.ga[1] = quot(f.a1, a.R, a.rR);
+  } else {
+    L.gl[0] = f.g0 / a.R;
+    L.ga[0] = f.a0 / a.R;
+    L.gl[1] = f.g1 / a.R;
+    L.ga[1] = f.a1 / a.R;
+  }
+  layer_slopes(a, rfdk, k, tm, tc, tp, sm, sc, sp, f.z, L);
+}
+
+// The LDD95 scans (TaperingFunc_LDD95 :392-428), each stopping at its first hit: blockIdx.y = 0
+// from the surface (depth tmps, layer ks), 1 from the bottom (tmpb, kb).  The pair (depth, layer)
+// goes to the first layer of each segment of the walk, where the segment's own thread reads it
+// before it stores its fluxes there: temperature and salinity planes of flon (surface) or flat
+// (bottom).
+__global__ __launch_bounds__(256) void k_redigm_scan(RediArgs a) {
+  __shared__ double wfd[REDI_LDS_LAYERS];
+  for (int k = threadIdx.x; k < a.km; k += 256) wfd[k] = a.rfdk[k];
+  __syncthreads();
+  const long q = (long)blockIdx.x * 256 + threadIdx.x;
+  if (q >= a.npts) return;
+  const int km = a.km;
+  const unsigned qb = (unsigned)q * 8u;
+  const double asn = a.lat_cs[a.J + q / a.I];
+  double disph = 2.0 / (a.two_omega * asn);
+  disph = fmin(fmax(15e3, disph), 100e3);
+  const double dzmax = a.smax * disph;
+  auto scan = [&](auto DIR) {
+    constexpr int dir = decltype(DIR)::value;
+    const int k0 = dir > 0 ? 0 : km - 1;
+    const double topo = dir > 0 ? 0.0 : a.topo[q];
+    double depth = 0.0;
+    int hit = dir > 0 ? -1 : km;
+    Pre ring[SRING];
+#pragma unroll
+    for (int u = 0; u < SRING; u++)
+      if (u < km) fetch_layer(a, qb, k0 + dir * u, dir, ring[u]);
+    double xc = ld(a.pt + (long)k0 * a.ldg, qb), yc = ld(a.sa + (long)k0 * a.ldg, qb);
+    double xb = xc, yb = yc;  // the layer behind in the walk (k0 itself at the start)
+    double mx = 0.0;
+    bool done = false;
+    for (int i0 = 0; i0 < km && !done; i0 += SRING) {
+#pragma unroll
+      for (int u = 0; u < SRING; u++) {
+        const int i = i0 + u;
+        if (done || i >= km) continue;
+        const int k = k0 + dir * i;
+        const Pre c = ring[u];
+        if (i + SRING < km) fetch_layer(a, qb, k + dir * SRING, dir, ring[u]);
+        const bool end = i + 1 == km;
+        const double xn = end ? xc : c.tn, yn = end ? yc : c.sn;
+        Lay L;
+        if (dir > 0)
+          slopes_of(a, wfd, k, c, xb, xc, xn, yb, yc, yn, L);
+        else
+          slopes_of(a, wfd, k, c, xn, xc, xb, yn, yc, yb, L);
+        const double sab = sqrt(L.slon * L.slon + L.slat * L.slat);
+        if (sab > mx) mx = sab;
+        if (dir > 0 ? (0.0 - c.z) > dzmax : (c.z - (-topo)) > dzmax) {
+          hit = k;
+          depth = fmin(mx, a.smax) * disph;
+          done = true;
+        }
+        xb = xc, yb = yc, xc = xn, yc = yn;
+      }
+    }
+    double* o = dir > 0 ? a.flon : a.flat;
+    const long oS = (long)km * a.ldo;
+    for (int k = 0; k < km; k += a.seg) {
+      st(o + (long)k * a.ldo, qb, depth);
+      st(o + oS + (long)k * a.ldo, qb, (double)hit);
+    }
+  };
+  if (blockIdx.y == 0)
+    scan(std::integral_constant<int, 1>{});
+  else
+    scan(std::integral_constant<int, -1>{});
+}
+
+// Segment blockIdx.y of the walk: layers k0 .. k1-1, with the layer above (its half-level terms)
+// and the layer below (the flux into the segment's last layer) computed again.
+__global__ __launch_bounds__(256, 3) void k_redigm_col(RediArgs a) {
   // per layer k: m1 = cdk[k]/(cdk[k-1]+cdk[k]), m2 = cdk[k-1]/(cdk[k-1]+cdk[k]) (r_m1, r_m2 of
   // the half level on top of layer k, calc_IsopycDiffFlux :491-494) and z_RCDK = 1/cdk[k]
   // (DOGCM_Admin_Grid_mod.f90:315), each the same IEEE division as in the loop
   __shared__ double wm1[REDI_LDS_LAYERS], wm2[REDI_LDS_LAYERS], wrc[REDI_LDS_LAYERS];
+  __shared__ double wfd[REDI_LDS_LAYERS];
   const int km = a.km;
-  for (int k = threadIdx.x; k < km; k += 256) {
+  const int k0 = blockIdx.y * a.seg, k1 = min(k0 + a.seg, km);
+  const int ka = max(k0 - 1, 0), kz = min(k1 + 1, km);
+  for (int k = ka + threadIdx.x; k < min(kz + 1, km); k += 256) {
     const double c1 = a.cdk[k];
     wrc[k] = 1.0 / c1;
+    wfd[k] = a.rfdk[k];
     if (k > 0) {
       const double c0 = a.cdk[k - 1];
       wm1[k] = c1 / (c0 + c1);
@@ -125,165 +280,90 @@ __global__ __launch_bounds__(256, 2) void k_redigm_col(RediArgs a) {
   __syncthreads();
   const long q = (long)blockIdx.x * 256 + threadIdx.x;
   if (q >= a.npts) return;
-  const int j = (int)(q / a.I);
-  const double cs = a.lat_cs[j], asn = a.lat_cs[a.J + j];
+  const unsigned qb = (unsigned)q * 8u;
+  const double cs = a.lat_cs[q / a.I];
   const double topo = a.topo[q];
-  const long TS = (long)km * a.ldgr;  // salinity block of the gradient inputs
-  // dir = +1: the next layer is k+1 (downward walk); -1: k-1 (upward)
-  auto fetch = [&](int k, int dir, Pre& f) {
-    const long g = (long)k * a.ldg + q, gr = (long)k * a.ldgr + q;
-    f.h = a.h[g];
-    f.z = a.z[g];
-    f.g0 = a.glon[gr];
-    f.a0 = a.glat[gr];
-    f.g1 = a.glon[TS + gr];
-    f.a1 = a.glat[TS + gr];
-    const int kn = k + dir;
-    const bool in = kn >= 0 && kn < km;
-    f.tn = in ? a.pt[g + dir * a.ldg] : 0.0;
-    f.sn = in ? a.sa[g + dir * a.ldg] : 0.0;
-  };
-  // layer k's slopes from its loads and ptemp/salt at k-1, k, k+1
-  auto slopes_of = [&](int k, const Pre& f, double tm, double tc, double tp, double sm, double sc, double sp,
-                       Lay& L) {
-    L.h = f.h;
-    L.gl[0] = f.g0 / a.R;
-    L.ga[0] = f.a0 / a.R;
-    L.gl[1] = f.g1 / a.R;
-    L.ga[1] = f.a1 / a.R;
-    layer_slopes(a, k, tm, tc, tp, sm, sc, sp, f.z, L);
-  };
-
-  // ---- pass 1: the LDD95 scans (TaperingFunc_LDD95 :392-428), each stopping at its first hit
-  double disph = 2.0 / (a.two_omega * asn);
-  disph = fmin(fmax(15e3, disph), 100e3);
-  const double dzmax = a.smax * disph;
-  int ks = -1, kb = km;
-  double tmps = 0.0, tmpb = 0.0;
-  for (int dir = 1; dir >= -1; dir -= 2) {
-    const int k0 = dir > 0 ? 0 : km - 1;
-    Pre ring[RING];
-#pragma unroll
-    for (int u = 0; u < RING; u++)
-      if (u < km) fetch(k0 + dir * u, dir, ring[u]);
-    double xc = a.pt[(long)k0 * a.ldg + q], yc = a.sa[(long)k0 * a.ldg + q];
-    double xb = xc, yb = yc;  // the layer behind in the walk (k0 itself at the start)
-    double mx = 0.0;
-    bool done = false;
-    for (int i0 = 0; i0 < km && !done; i0 += RING) {
-#pragma unroll
-      for (int u = 0; u < RING; u++) {
-        const int i = i0 + u;
-        if (done || i >= km) continue;
-        const int k = k0 + dir * i;
-        const Pre c = ring[u];
-        if (i + RING < km) fetch(k0 + dir * (i + RING), dir, ring[u]);
-        const bool end = i + 1 == km;
-        const double xn = end ? xc : c.tn, yn = end ? yc : c.sn;
-        Lay L;
-        if (dir > 0)
-          slopes_of(k, c, xb, xc, xn, yb, yc, yn, L);
-        else
-          slopes_of(k, c, xn, xc, xb, yn, yc, yb, L);
-        const double sab = sqrt(L.slon * L.slon + L.slat * L.slat);
-        if (sab > mx) mx = sab;
-        const bool hit = dir > 0 ? (0.0 - c.z) > dzmax : (c.z - (-topo)) > dzmax;
-        if (hit) {
-          if (dir > 0) {
-            ks = k;
-            tmps = fmin(mx, a.smax) * disph;
-          } else {
-            kb = k;
-            tmpb = fmin(mx, a.smax) * disph;
-          }
-          done = true;
-        }
-        xb = xc, yb = yc, xc = xn, yc = yn;
-      }
-    }
-  }
-
-  // ---- pass 2: every layer, the half level above it, and the divergence of the layer above
+  const long oS = (long)km * a.ldo, o0 = (long)k0 * a.ldo;
+  const double tmps = ld(a.flon + o0, qb), tmpb = ld(a.flat + o0, qb);
+  const int ks = (int)ld(a.flon + oS + o0, qb), kb = (int)ld(a.flat + oS + o0, qb);
   const double kr = a.kr, kg = a.kg;
-  Lay P;                                          // layer k-1
-  double pl[2] = {0.0, 0.0}, pa[2] = {0.0, 0.0};  // psi of layer k-1 (GM)
-  double fs_up[2] = {0.0, 0.0};                   // FSig on the half level above layer k-1
-  double tc = a.pt[q], sc = a.sa[q], tm = tc, sm = sc;
-  const long oS = (long)km * a.ldo;
+  Lay P;                         // layer k-1
+  double rPh = 0.0;              // 1 / P.h
+  double fs_up[2] = {0.0, 0.0};  // FSig on the half level above layer k-1
+  double tc = ld(a.pt + (long)ka * a.ldg, qb), sc = ld(a.sa + (long)ka * a.ldg, qb), tm = tc, sm = sc;
+  if (ka > 0) tm = ld(a.pt + (long)(ka - 1) * a.ldg, qb), sm = ld(a.sa + (long)(ka - 1) * a.ldg, qb);
   auto body = [&](int k, const Pre& f) {
     const bool last = k + 1 == km;
     const double tp = last ? tc : f.tn, sp = last ? sc : f.sn;
     Lay C;
-    slopes_of(k, f, tm, tc, tp, sm, sc, sp, C);
+    slopes_of(a, wfd, k, f, tm, tc, tp, sm, sc, sp, C);
+    const double rCh = recip(C.h);
     const double z = f.z;
     // taper (prepare_SlopeTapering: T1 T2)
     const double mag2 = C.slon * C.slon + C.slat * C.slat;
     const double t1 =
-        a.gkw91 ? fmin(1.0, (a.smax * a.smax) / mag2) : 0.5 * (1.0 + tanh((a.smax - sqrt(mag2)) / a.sd));
+        a.gkw91 ? fmin(1.0, (a.smax * a.smax) / mag2) : 0.5 * (1.0 + taper_tanh((a.smax - sqrt(mag2)) / a.sd));
     double r = 1.0;
     if (k <= ks) r = fmin((0.0 - z) / (tmps + 1e-13), 1.0);
     if (k >= kb) r = fmin((z - (-topo)) / (tmpb + 1e-13), 1.0);
     // r = 1 gives 0.5 (1 + sin(pi/2)) = 1 exactly; sin only where the ratio is below 1
     const double t2 = r == 1.0 ? 1.0 : 0.5 * (1.0 + sin(PI_REF * (r - 0.5)));
     C.tap = t1 * t2;
-    const long o = (long)k * a.ldo + q;
-    double cl[2], ca[2];
+    if (k >= k0 && k < k1) {
+      double dz[2];
+      div2(0.5 * (C.da[0] + C.db[0]), 0.5 * (C.da[1] + C.db[1]), C.h, rCh, dz[0], dz[1]);
+      const long o = (long)k * a.ldo;
 #pragma unroll
-    for (int x = 0; x < 2; x++) {
-      const double dz = (0.5 * (C.da[x] + C.db[x])) / C.h;
-      const double flr = kr * (C.gl[x] + (C.tap * C.slon) * dz);
-      const double far_ = kr * (C.ga[x] + (C.tap * C.slat) * dz);
-      cl[x] = -((kg * C.tap) * C.slat);  // Psi(LON)
-      ca[x] = (kg * C.tap) * C.slon;     // Psi(LAT)
-      const double flg = -(ca[x] * dz);
-      const double fag = cl[x] * dz;
-      a.flon[x * oS + o] = (flr + flg) * cs;
-      a.flat[x * oS + o] = (far_ + fag) * cs;
+      for (int x = 0; x < 2; x++) {
+        const double flr = kr * (C.gl[x] + (C.tap * C.slon) * dz[x]);
+        const double far_ = kr * (C.ga[x] + (C.tap * C.slat) * dz[x]);
+        const double flg = -(((kg * C.tap) * C.slon) * dz[x]);  // -Psi(LAT) dz
+        const double fag = -((kg * C.tap) * C.slat) * dz[x];    // Psi(LON) dz
+        st(a.flon + x * oS + o, qb, (flr + flg) * cs);
+        st(a.flat + x * oS + o, qb, (far_ + fag) * cs);
+      }
     }
-    if (k > 0) {  // the half level between layers k-1 (up) and k (lo)
+    if (k > ka) {  // the half level between layers k-1 (up) and k (lo)
       const double m1 = wm1[k], m2 = wm2[k];
       const double sl = (m1 * P.tap) * P.slon + (m2 * C.tap) * C.slon;
       const double sa_ = (m1 * P.tap) * P.slat + (m2 * C.tap) * C.slat;
       const double hden = m1 * P.h + m2 * C.h;
-      const double rc = wrc[k - 1];
+      const double rc = wrc[k - 1], ss = sl * sl + sa_ * sa_;
+      // Psi(LON) and Psi(LAT) of both layers
+      const double pln = m1 * -((kg * P.tap) * P.slat) + m2 * -((kg * C.tap) * C.slat);
+      const double pat = m1 * ((kg * P.tap) * P.slon) + m2 * ((kg * C.tap) * C.slon);
+      double dv[2], fs[2];
+      div2(ss * C.da[0], ss * C.da[1], hden, recip(hden), dv[0], dv[1]);
 #pragma unroll
       for (int x = 0; x < 2; x++) {
         const double glon = m1 * P.gl[x] + m2 * C.gl[x];
         const double glat = m1 * P.ga[x] + m2 * C.ga[x];
-        const double fr = kr * ((sl * glon + sa_ * glat) + ((sl * sl + sa_ * sa_) * C.da[x]) / hden);
-        const double pln = m1 * pl[x] + m2 * cl[x];
-        const double pat = m1 * pa[x] + m2 * ca[x];
+        const double fr = kr * ((sl * glon + sa_ * glat) + dv[x]);
         const double fg = pat * glon - pln * glat;
-        const double fs = fr + fg;
-        a.vdiv[x * oS + (long)(k - 1) * a.ldo + q] = ((fs_up[x] - fs) * rc) / P.h;
-        fs_up[x] = fs;
+        fs[x] = fr + fg;
       }
+      if (k > k0) {
+        div2((fs_up[0] - fs[0]) * rc, (fs_up[1] - fs[1]) * rc, P.h, rPh, dv[0], dv[1]);
+        st(a.vdiv + (long)(k - 1) * a.ldo, qb, dv[0]);
+        st(a.vdiv + oS + (long)(k - 1) * a.ldo, qb, dv[1]);
+      }
+      fs_up[0] = fs[0], fs_up[1] = fs[1];
     }
     P = C;
-    pl[0] = cl[0], pl[1] = cl[1], pa[0] = ca[0], pa[1] = ca[1];
+    rPh = rCh;
     tm = tc, sm = sc, tc = tp, sc = sp;
   };
-  {
-    Pre ring[RING];
-#pragma unroll
-    for (int u = 0; u < RING; u++)
-      if (u < km) fetch(u, 1, ring[u]);
-    for (int k0 = 0; k0 < km; k0 += RING) {
-#pragma unroll
-      for (int u = 0; u < RING; u++) {
-        const int k = k0 + u;
-        if (k < km) {
-          const Pre c = ring[u];
-          if (k + RING < km) fetch(k + RING, 1, ring[u]);
-          body(k, c);
-        }
-      }
-    }
+  Pre nx;
+  fetch_layer(a, qb, ka, 1, nx);
+  for (int k = ka; k < kz; k++) {
+    const Pre c = nx;
+    if (k + 1 < kz) fetch_layer(a, qb, k + 1, 1, nx);
+    body(k, c);
   }
-  {  // the bottom layer: FSig below it is zero
+  if (k1 == km) {  // the bottom layer: FSig below it is zero
     const double rc = wrc[km - 1];
     for (int x = 0; x < 2; x++)
-      a.vdiv[x * oS + (long)(km - 1) * a.ldo + q] = ((fs_up[x] - 0.0) * rc) / P.h;
+      st(a.vdiv + x * oS + (long)(km - 1) * a.ldo, qb, ((fs_up[x] - 0.0) * rc) / P.h);
   }
 }
 
@@ -312,10 +392,18 @@ int launch_redigm_col(const dsht_plan* p, const RediParams& c, const double* pt,
   a.ldg = ldg, a.ldgr = ldgr, a.ldo = ldo, a.npts = (long)p->I * p->J;
   a.km = km, a.I = p->I, a.J = p->J, a.gkw91 = c.gkw91;
   a.R = p->R, a.rg = c.ref_dens * c.grav, a.kr = c.kappa_redi, a.kg = c.kappa_gm, a.smax = c.slope_max, a.sd = c.sd;
+  a.rR = fabs(p->R) > 0x1p-900 && fabs(p->R) < 0x1p900 ? 1.0 / p->R : 0.0;
   a.two_omega = 2.0 * c.omega;
   const double bytes = (14.0 * km + 1.0) * (double)a.npts * 8.0;
   ProfScope prof("redigm_col", s, bytes, 0.0);
-  hipLaunchKernelGGL(k_redigm_col, dim3((unsigned)((a.npts + 255) / 256)), dim3(256), 0, s, a);
+  // Segments: at least 5120 waves (3 a SIMD on 1024 SIMDs run at once) of 3 layers or
+  // more.  Whole column (one segment) against this rule: 512 x 256 x 60 (3 segments) 229 and
+  // 227 us, 256 x 128 x 60 (10) 133 and 76 us, 128 x 64 x 20 (7) 49 and 25 us
+  const long nseg = std::max(1l, std::min((5120l * 64 + a.npts - 1) / a.npts, (km + 2l) / 3));
+  a.seg = (int)((km + nseg - 1) / nseg);
+  const unsigned nb = (unsigned)((a.npts + 255) / 256);
+  hipLaunchKernelGGL(k_redigm_scan, dim3(nb, 2), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(k_redigm_col, dim3(nb, (unsigned)((km + a.seg - 1) / a.seg)), dim3(256), 0, s, a);
   DSHT_HIP(hipGetLastError());
   return 0;
 }
