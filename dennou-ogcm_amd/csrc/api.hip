@@ -261,11 +261,21 @@ static int run_inv(dsht_plan* p, int op, const double* in0, const double* in1, l
   return 0;
 }
 
+int workspace_reserve(dsht_plan* p, int nfields, int ncols, hipStream_t s) {
+  WsHandle wl;
+  return workspace_acquire(p, s, nfields * fourier_bytes(p, chunk_cols(p, ncols)), wl);
+}
+
 bool uv_scaled_ok(const dsht_plan* p) { return p->prec == DSHT_PREC_FP64 && fft_reg_ok(p); }
 
 int uv2vordiv_scaled(dsht_plan* p, const double* u, const double* v, const double* rowscale, long ldg, double* vor,
                      double* div, long sl, long sc, int ncols, const double* diag, hipStream_t s) {
   return run_fwd(p, F_UV2VORDIV, u, v, ldg, vor, div, sl, sc, ncols, diag, diag, 1.0 / p->R, p->d_cwd, s, rowscale);
+}
+
+int div_scaled(dsht_plan* p, const double* u, const double* v, const double* rowscale, long ldg, double* div, long sl,
+               long sc, int ncols, hipStream_t s) {
+  return run_fwd(p, F_ALPHA, u, v, ldg, div, nullptr, sl, sc, ncols, nullptr, nullptr, 1.0 / p->R, p->d_cwd, s, rowscale);
 }
 
 bool fwd_fused_ok(const dsht_plan* p) {
@@ -1417,6 +1427,8 @@ int dsht_redigm_d(dsht_plan* p, const dsht_redigm_config* cfg, const double* pte
   double* vdv = flat + n2 * IJ;
   double* w = vdv + n2 * IJ;  // 2 km spectra, coefficient-major (sl = 2 km)
   int rc;
+  // the fused inverse takes the most scratch: one allocation on a plan's first call
+  if (p->prec == DSHT_PREC_FP64 && (rc = workspace_reserve(p, inv_nout(I_VGRAD), (int)n2, s))) return rc;
   // calc_GradTRC (:431-442): w_xy of each layer, xy_GradLon_w and xy_GradLat_w
   if (salt == ptemp + (long)km * ldg) {  // both tracers in one array (xyza_TRC): one call
     if ((rc = dsht_fwd_d(p, DSHT_VAL, ptemp, ldg, w, n2, 1, (int)n2, nullptr, s))) return rc;

@@ -247,8 +247,14 @@ int fwd_add(dsht_plan* p, const double* xy, long ldg, double* w, long sl, long s
             hipStream_t s);
 int uv2vordiv_scaled(dsht_plan* p, const double* u, const double* v, const double* rowscale, long ldg, double* vor,
                      double* div, long sl, long sc, int ncols, const double* diag, hipStream_t s);
+// its divergence alone
+int div_scaled(dsht_plan* p, const double* u, const double* v, const double* rowscale, long ldg, double* div, long sl,
+               long sc, int ncols, hipStream_t s);
 // api.hip: per-stream scratch
 int workspace_acquire(dsht_plan* p, hipStream_t s, size_t bytes, WsHandle& out);
+// the FP64 transforms' scratch for nfields grids of ncols columns in one call, so that a sequence of
+// calls whose first are smaller does not grow it step by step
+int workspace_reserve(dsht_plan* p, int nfields, int ncols, hipStream_t s);
 // tables.hip
 int build_tables(dsht_plan* p);
 // fft.hip

@@ -5,18 +5,21 @@
 // Configuration: hydrostatic Boussinesq dynamics on the hspm_vfvm grid with a rigid lid
 // (one barotropic iteration, :147-170, 685-774), a flat bottom (xyz_H = D, xyz_Z = D z_CK,
 // DOGCM_Admin_Grid_mod.f90:376-388), the linear equation of state (EOS_Linear_mod.f90) and
-// no physics forcing.  Per layer a step makes the reference's 42 forward and 28 inverse
+// no physics forcing.  Per layer a step stands for the reference's 42 forward and 28 inverse
 // transform units (VorDivDiag x3, MOMBarocRHS x2, HTRCRHS x2 over two tracers, ImplUV,
 // ImplTRC) and per run 9 forward and 9 inverse 2-D units of the barotropic mode; every
-// transform runs over all layers of all active runs in one library call.  The grid-space
+// transform runs over all layers of all active runs in one library call.  It makes fewer: the
+// constant geopotential's gradient is computed once a step, the vorticity that only the divergence
+// is wanted with is not, and in the FP64 form the implicit solves work on spectra.  The grid-space
 // work between the transforms is fused into the kernels below; the column work (omega,
-// hydrostatic pressure, barotropic velocity, QUICK flux, the implicit vertical solves) uses
-// the library's column kernels.
+// hydrostatic pressure, barotropic velocity, QUICK flux, the implicit vertical solves) is
+// done in them too, a thread walking a column.
 //
 // Layout (FP64 device memory): run r, layer k of a layered field is grid column r*K + k;
 // tracers are run-major with temperature then salinity: column (2r + t)*K + k; 2-D fields
 // one column per run; half-level fields (K+1) levels per run (per run and tracer for the
 // vertical fluxes).  Spectra of internal transforms use the fast "LC" layout.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -568,6 +571,127 @@ __global__ __launch_bounds__(256) void k_lf_vsolve(VSolve a, const double* __res
   }
 }
 
+// The same solve on spectra: the matrix is the same at every point, so it commutes with the
+// horizontal transform, and w = diag (q0 + x) from the spectra q0 of the field and w of its
+// tendency takes the place of an inverse of the tendency, the solve on the grid (which has 4.5
+// times the values of a T170 spectrum at 512 x 256) and a forward transform.  The columns of one
+// coefficient are contiguous, K to a system: SB systems a block go through LDS (an odd row of
+// doubles each, so that a wave's rows start in different banks), loaded and stored by the whole
+// block, solved by a thread each.  The factors are padded to KP layers, a multiple of VL, with rows
+// that leave zeros, so that a group's reads of LDS and factors all come before its first store.
+// Elimination as k_lf_vsolve.  Bound by latency: a wave's solve takes 11 us of T170L60's 30, and
+// loads and stores go out in one burst each; up to 64 layers (REG) a thread's loads, q0's too, all
+// go out first (rows of more in rounds: 41 us there).  32 or 16 systems a block: 38 and 45 us.
+constexpr int WS_SB = 64;  // most systems a block of k_lf_wsolve holds
+template <bool MOM, bool REG>
+__global__ __launch_bounds__(256) void k_lf_wsolve(const double* __restrict__ q0, double* __restrict__ w,
+                                                   const double* __restrict__ diag, const double* __restrict__ fac,
+                                                   const int* __restrict__ swapped, double dt, double e3,
+                                                   unsigned nsys, unsigned per, int K, int KP, int SB) {
+#pragma clang fp contract(off)
+  extern __shared__ double sh[];
+  const int P = KP + 1;
+  const double *__restrict__ dd = fac + KP, *__restrict__ du = dd + KP, *__restrict__ du2 = du + KP;
+  const unsigned s0 = blockIdx.x * SB;
+  const int ns = (int)(nsys - s0 < (unsigned)SB ? nsys - s0 : (unsigned)SB);
+  const long g0 = (long)s0 * K;
+  const int l16 = threadIdx.x % 16, row0 = threadIdx.x / 16;
+  auto right = [&](double x) {
+    const double bt = dt * x;
+    return MOM ? bt : bt / e3;
+  };
+  double qv[REG ? WS_SB / 16 : 1][4];
+  if constexpr (REG) {
+    double wv[WS_SB / 16][4];
+    auto load = [&](const double* __restrict__ f, double (&to)[WS_SB / 16][4]) {
+#pragma unroll
+      for (int r = 0; r < WS_SB / 16; r++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int q = row0 + 16 * r, k = l16 + 16 * u;
+          if (16 * u < K) to[r][u] = f[g0 + (q < ns ? q : 0) * K + (k < K ? k : 0)];
+        }
+    };
+    load(w, wv);
+    load(q0, qv);
+#pragma unroll
+    for (int r = 0; r < WS_SB / 16; r++)
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int q = row0 + 16 * r, k = l16 + 16 * u;
+        if (q < ns && k < KP) sh[q * P + k] = k < K ? right(wv[r][u]) : 0.0;
+      }
+  } else {
+    for (int q = row0; q < ns; q += 16) {
+#pragma unroll 4
+      for (int k = l16; k < KP; k += 16) sh[q * P + k] = k < K ? right(w[g0 + (long)q * K + k]) : 0.0;
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < ns) {
+    double* x = sh + threadIdx.x * P;
+    double up = 0.0;  // row k-1; the step into row 0 (fac 0, not swapped) takes row 0 as it is
+    for (int k0 = 0; k0 < KP; k0 += VL) {
+      double v[VL + 1], f[VL];
+      bool sw[VL];
+#pragma unroll
+      for (int u = 0; u < VL; u++) {
+        v[u] = x[k0 + u];
+        f[u] = u + k0 > 0 ? fac[k0 + u - 1] : 0.0;
+        sw[u] = u + k0 > 0 ? swapped[k0 + u - 1] != 0 : false;
+      }
+#pragma unroll
+      for (int u = 0; u < VL; u++) {
+        const double a = sw[u] ? up : v[u], b = sw[u] ? v[u] : up;
+        v[u] = b;
+        up = k0 + u < K ? a - f[u] * b : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < VL; u++)
+        if (k0 + u > 0) x[k0 + u - 1] = v[u];
+    }
+    if (K == KP) x[K - 1] = up;
+    double xa = 0.0, xb = 0.0;  // x[k+1], x[k+2]
+    for (int k0 = KP - VL; k0 >= 0; k0 -= VL) {
+      double v[VL], d[VL], e[VL], e2[VL];
+#pragma unroll
+      for (int u = 0; u < VL; u++) {
+        v[u] = x[k0 + u];
+        d[u] = dd[k0 + u], e[u] = du[k0 + u], e2[u] = du2[k0 + u];
+      }
+#pragma unroll
+      for (int u = VL - 1; u >= 0; u--) {
+        const double t = v[u] - e[u] * xa;
+        v[u] = (t - e2[u] * xb) / d[u];
+        xb = xa;
+        xa = v[u];
+      }
+#pragma unroll
+      for (int u = 0; u < VL; u++) x[k0 + u] = v[u];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < WS_SB / 16; r++) {
+    const int q = row0 + 16 * r;
+    if (q >= ns) break;
+    const double dg = diag[(s0 + q) / per];
+    if constexpr (REG) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int k = l16 + 16 * u;
+        if (k < K) w[g0 + q * K + k] = (qv[r][u] + sh[q * P + k]) * dg;
+      }
+    } else {
+#pragma unroll 4
+      for (int k = l16; k < K; k += 16) {
+        const long g = g0 + (long)q * K + k;
+        w[g] = (q0[g] + sh[q * P + k]) * dg;
+      }
+    }
+  }
+}
+
 }  // namespace
 }  // namespace dsht
 
@@ -597,7 +721,7 @@ struct dsht_lfam3 {
   double *wVD = nullptr, *wGeo = nullptr, *wC = nullptr, *w1 = nullptr, *w2 = nullptr;
   double *wB = nullptr, *wC2 = nullptr, *wDSP = nullptr, *wDDiv = nullptr, *wZero = nullptr;
   // the elimination of the constant vertical systems (momentum, tracers): fact, d, du, du2 and
-  // the interchanges, K each
+  // the interchanges, lf_kp(K) each
   double* d_vf[2] = {};
   int* d_vs[2] = {};
 };
@@ -651,9 +775,12 @@ void lf_free(dsht_lfam3* s) {
     DSHT_HIP(hipGetLastError());                                                              \
   } while (0)
 
+// layers of a padded factor array
+int lf_kp(int K) { return (K + VL - 1) / VL * VL; }
+
 // DGTSV's elimination (LAPACK 3.x SRC/dgtsv.f, partial pivoting by row interchange) of the
 // constant vertical system of momentum or of the tracers (rows as k_col_vdiff builds them):
-// fac = fact, d, du, du2 (K each), swapped = 1 where a step interchanged its rows
+// fac = fact, d, du, du2 (lf_kp(K) each, rows of the identity behind K), swapped = 1 where a step interchanged its rows
 void lf_vfactor(const dsht_lfam3* s, bool mom, std::vector<double>& fac, std::vector<int>& swapped) {
 #pragma clang fp contract(off)
   const dsht_lfam3_config& c = s->cfg;
@@ -679,10 +806,11 @@ void lf_vfactor(const dsht_lfam3* s, bool mom, std::vector<double>& fac, std::ve
     else
       ad[k] = 1.0 + ac * (r[k] + r[k + 1]);
   }
-  fac.assign(4 * (size_t)K, 0.0);
-  swapped.assign(K, 0);
-  double *fact = fac.data(), *d = fact + K, *du = d + K, *du2 = du + K;
-  for (int k = 0; k < K; k++) d[k] = ad[k], du[k] = au[k];
+  const int KP = lf_kp(K);
+  fac.assign(4 * (size_t)KP, 0.0);
+  swapped.assign(KP, 0);
+  double *fact = fac.data(), *d = fact + KP, *du = d + KP, *du2 = du + KP;
+  for (int k = 0; k < KP; k++) d[k] = k < K ? ad[k] : 1.0, du[k] = k < K ? au[k] : 0.0;
   for (int j = 0; j < K - 1; j++) {
     const double dl = al[j + 1];
     if (std::fabs(d[j]) >= std::fabs(dl)) {
@@ -705,27 +833,51 @@ void lf_vfactor(const dsht_lfam3* s, bool mom, std::vector<double>& fac, std::ve
 
 // one or two fields (z) of ny sections through the constant solve
 int lf_vsolve(dsht_lfam3* s, bool mom, const VSolve& a, int ny, int nz, hipStream_t st) {
-  const int K = s->K, w = mom ? 0 : 1, th = lf_threads(s->np, ny * nz);
+  const int K = s->K, KP = lf_kp(K), w = mom ? 0 : 1, th = lf_threads(s->np, ny * nz);
   auto k = mom ? (K <= 32 ? k_lf_vsolve<32, true> : K <= 64 ? k_lf_vsolve<64, true> : k_lf_vsolve<0, true>)
                : (K <= 32 ? k_lf_vsolve<32, false> : K <= 64 ? k_lf_vsolve<64, false> : k_lf_vsolve<0, false>);
   dim3 grid = lf_gridc(s->np, ny, th);
   grid.z = nz;
   const double* f = s->d_vf[w];
-  hipLaunchKernelGGL(k, grid, dim3(th), 0, st, a, f, f + K, f + 2 * K, f + 3 * K, s->d_vs[w], s->cfg.dt, s->cfg.depth,
+  hipLaunchKernelGGL(k, grid, dim3(th), 0, st, a, f, f + KP, f + 2 * KP, f + 3 * KP, s->d_vs[w], s->cfg.dt, s->cfg.depth,
                      s->np, K);
   DSHT_HIP(hipGetLastError());
   return 0;
 }
 
-// calc_UVCosLat2VorDiv of (U cos phi, V cos phi), the vorticity in wVD's columns [0, nc) and the
+// systems a block of k_lf_wsolve holds: 64, fewer where K is large (64 KB of LDS) or where that
+// leaves fewer than 1024 blocks
+int lf_wsolve_sb(long nsys, int K) {
+  const long fit = 8192 / (lf_kp(K) + 1), spread = nsys / 1024;
+  return (int)std::min({(long)WS_SB, fit, std::max(8l, spread)});
+}
+
+// w = diag (q0 + x) for the spectra of per sections of K layers, where the solve fits
+// k_lf_wsolve and the form's transforms return a spectrum to FP64 rounding
+bool lf_wsolve_ok(const dsht_lfam3* s) { return fwd_fused_ok(s->p) && lf_wsolve_sb(1 << 20, s->K) >= 8; }
+int lf_wsolve(dsht_lfam3* s, bool mom, const double* q0, double* w, const double* diag, int per, hipStream_t st) {
+  const int K = s->K, f = mom ? 0 : 1;
+  const long nsys = (long)s->L * per;
+  const int sb = lf_wsolve_sb(nsys, K);
+  auto k = lf_kp(K) <= 64 ? (mom ? k_lf_wsolve<true, true> : k_lf_wsolve<false, true>)
+                          : (mom ? k_lf_wsolve<true, false> : k_lf_wsolve<false, false>);
+  hipLaunchKernelGGL(k, dim3((unsigned)((nsys + sb - 1) / sb)), dim3(256),
+                     sizeof(double) * sb * (lf_kp(K) + 1), st, q0, w, diag, s->d_vf[f], s->d_vs[f],
+                     s->cfg.dt, s->cfg.depth, (unsigned)nsys, (unsigned)per, K, lf_kp(K), sb);
+  DSHT_HIP(hipGetLastError());
+  return 0;
+}
+
+// calc_UVCosLat2VorDiv of (U cos phi, V cos phi), the vorticity in w's columns [0, nc) and the
 // divergence in [nc, 2 nc): cos phi is applied as the FFT reads the winds, or, where that form
 // has no such kernel, by a pass over them
-int lf_uv2vordiv(dsht_lfam3* s, const double* u, const double* v, int nc, const double* diag, hipStream_t st) {
+int lf_uv2vordiv(dsht_lfam3* s, const double* u, const double* v, double* w, int nc, const double* diag,
+                 hipStream_t st) {
   dsht_plan* p = s->p;
   if (uv_scaled_ok(p))
-    return uv2vordiv_scaled(p, u, v, s->d_cs, s->np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, diag, st);
+    return uv2vordiv_scaled(p, u, v, s->d_cs, s->np, w, w + nc, 2l * nc, 1, nc, diag, st);
   LF_LAUNCH2(k_lf_uvcos, nc, s->np, st, u, v, s->d_cs, s->np, s->I, (long)nc, s->ucos, s->vcos);
-  return dsht_uv2vordiv_d(p, s->ucos, s->vcos, s->np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, diag, st);
+  return dsht_uv2vordiv_d(p, s->ucos, s->vcos, s->np, w, w + nc, 2l * nc, 1, nc, diag, st);
 }
 
 // w += diag w_xy(x) over nc columns of pitch sl (tmp: spectra for forms that do not add)
@@ -738,22 +890,31 @@ int lf_fwd_add(dsht_lfam3* s, const double* x, double* w, long sl, double* tmp, 
 }
 
 // HBEDiagnose_VorDiv (HBEDiagnose_hspm_vfvm_mod.f90:259-286) over every layer of the active
-// runs: vorticity into VD[0, nc), divergence into VD[nc, 2 nc)
-int lf_vordiv(dsht_lfam3* s, const double* u, const double* v, int nc, hipStream_t st) {
-  if (int rc = lf_uv2vordiv(s, u, v, nc, nullptr, st)) return rc;
-  return dsht_inv_d(s->p, DSHT_VAL, s->wVD, 2l * nc, 1, s->VD, s->np, 2 * nc, nullptr, st);
+// runs: vorticity into VD[0, nc), divergence into VD[nc, 2 nc), their spectra in w
+int lf_vordiv(dsht_lfam3* s, const double* u, const double* v, double* w, int nc, hipStream_t st) {
+  if (int rc = lf_uv2vordiv(s, u, v, w, nc, nullptr, st)) return rc;
+  return dsht_inv_d(s->p, DSHT_VAL, w, 2l * nc, 1, s->VD, s->np, 2 * nc, nullptr, st);
 }
 
-// HBEBaroc_MOMRHS_VorDivForm (HBEBaroc_hspm_vfvm_mod.f90:321-443) -> URHS, VRHS, with the vorticity
-// and divergence of (u, v) in VD.  pred: the Coriolis terms f (cn (u, v) + cb (xa, xb)), else
-// f (xa, xb)
+// its divergence alone, all that the tracers' right-hand side reads
+int lf_div(dsht_lfam3* s, const double* u, const double* v, int nc, hipStream_t st) {
+  if (!uv_scaled_ok(s->p)) return lf_vordiv(s, u, v, s->wVD, nc, st);
+  if (int rc = div_scaled(s->p, u, v, s->d_cs, s->np, s->wVD, nc, 1, nc, st)) return rc;
+  return dsht_inv_d(s->p, DSHT_VAL, s->wVD, nc, 1, s->VD + (long)nc * s->np, s->np, nc, nullptr, st);
+}
+
+// HBEBaroc_MOMRHS_VorDivForm (HBEBaroc_hspm_vfvm_mod.f90:321-443), the spectra in wVD, with the
+// vorticity and divergence of (u, v) in VD.  pred: the Coriolis terms f (cn (u, v) + cb (xa, xb)),
+// else f (xa, xb).  The geopotential's gradient is that of the whole step: the predictor, which
+// comes first, computes it
 int lf_mom_rhs(dsht_lfam3* s, const double* u, const double* v, const double* xa, const double* xb, bool pred, double cn,
                double cb, const double* sp, int nr, hipStream_t st) {
   dsht_plan* p = s->p;
   const int nc = nr * s->K;
-  // w_GeoPot = w_xy(GeoPot); xy_GradLat_w, xy_GradLon_w of it
-  if (int rc = dsht_fwd_d(p, DSHT_VAL, s->Geo, s->np, s->wGeo, nc, 1, nc, nullptr, st)) return rc;
-  if (int rc = dsht_inv_vgrad_d(p, s->wGeo, nc, 1, nullptr, s->GLon, s->GLat, s->np, nc, nullptr, st)) return rc;
+  if (pred) {  // w_GeoPot = w_xy(GeoPot); xy_GradLat_w, xy_GradLon_w of it
+    if (int rc = dsht_fwd_d(p, DSHT_VAL, s->Geo, s->np, s->wGeo, nc, 1, nc, nullptr, st)) return rc;
+    if (int rc = dsht_inv_vgrad_d(p, s->wGeo, nc, 1, nullptr, s->GLon, s->GLat, s->np, nc, nullptr, st)) return rc;
+  }
   const MomArgs a{s->cfg.ref_dens, p->R, s->cfg.depth, cn, cb, s->np, s->I, s->K};
   auto k = pred ? k_lf_mom<true> : k_lf_mom<false>;
   LF_LAUNCHC(k, s->np, nr, 1, st, a, u, v, xa, xb, s->VD + (long)nc * s->np, s->VD, s->Hyd, s->Dens, s->GLon, s->GLat,
@@ -761,12 +922,11 @@ int lf_mom_rhs(dsht_lfam3* s, const double* u, const double* v, const double* xa
   // (w_Vor_RHS, w_Div_RHS) = (-H(A, B), H(B, -A)) = calc_UVCosLat2VorDiv(B, -A); then
   // w_Div_RHS - w_Lapla_w(w_xy(C)) = + n(n+1) w_xy(C)
   if (int rc = dsht_uv2vordiv_d(p, s->Bg, s->Am, s->np, s->wVD, s->wVD + nc, 2l * nc, 1, nc, nullptr, st)) return rc;
-  if (int rc = lf_fwd_add(s, s->Cg, s->wVD + nc, 2l * nc, s->wC, nc, s->d_nn1, st)) return rc;
-  return dsht_vordiv2uv_d(p, s->wVD, s->wVD + nc, 2l * nc, 1, s->URHS, s->VRHS, s->np, nc, st);
+  return lf_fwd_add(s, s->Cg, s->wVD + nc, 2l * nc, s->wC, nc, s->d_nn1, st);
 }
 
-// HBEBaroc_HTRCRHS (HBEBaroc_hspm_vfvm_mod.f90:119-202) for both tracers of the active runs, with
-// the divergence of (u, v) in VD and the thickness factor h
+// HBEBaroc_HTRCRHS (HBEBaroc_hspm_vfvm_mod.f90:119-202) for both tracers of the active runs, the
+// spectra in w1, with the divergence of (u, v) in VD and the thickness factor h
 int lf_htrc(dsht_lfam3* s, const double* ts, const double* u, const double* v, double h, int nr, hipStream_t st) {
   dsht_plan* p = s->p;
   const long np = s->np;
@@ -781,7 +941,15 @@ int lf_htrc(dsht_lfam3* s, const double* ts, const double* u, const double* v, d
     if (int rc = dsht_fwd_d(p, DSHT_VAL, s->VF, np, s->w2, nt, 1, nt, nullptr, st)) return rc;
     LF_LAUNCH2(k_lf_htrc_spec, s->L, nt, st, s->w1, s->w2, s->d_advf, s->L, nt);
   }
-  return dsht_inv_d(p, DSHT_VAL, s->w1, nt, 1, s->HT, np, nt, nullptr, st);
+  return 0;
+}
+
+// the grids of lf_mom_rhs and lf_htrc
+int lf_mom_grid(dsht_lfam3* s, int nc, hipStream_t st) {
+  return dsht_vordiv2uv_d(s->p, s->wVD, s->wVD + nc, 2l * nc, 1, s->URHS, s->VRHS, s->np, nc, st);
+}
+int lf_htrc_grid(dsht_lfam3* s, int nt, hipStream_t st) {
+  return dsht_inv_d(s->p, DSHT_VAL, s->w1, nt, 1, s->HT, s->np, nt, nullptr, st);
 }
 
 }  // namespace
@@ -955,9 +1123,9 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
     lf_vfactor(s, w == 0, vf, vs);
     U(&s->d_vf[w], vf);
     double* d = nullptr;
-    A(&d, (K + 1) / 2);
+    A(&d, (vs.size() + 1) / 2);
     s->d_vs[w] = (int*)d;
-    if (!rc && hipMemcpy(d, vs.data(), sizeof(int) * K, hipMemcpyHostToDevice) != hipSuccess)
+    if (!rc && hipMemcpy(d, vs.data(), sizeof(int) * vs.size(), hipMemcpyHostToDevice) != hipSuccess)
       rc = fail(DSHT_EDEVICE, "LF-AM3 pool: upload failed");
   }
   if (rc) {
@@ -1080,11 +1248,15 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   double *TB = s->TS[0], *TN = s->TS[1], *TA = s->TS[2];
   double *PN = s->SP[1], *PA = s->SP[2];
   int rc;
+  // val_sub_alpha takes the most scratch: allocated at once, the first step of a plan at T42L20
+  // takes 0.47 ms; three allocations and two frees within it made that 1.25
+  if (fwd_fused_ok(p) && (rc = workspace_reserve(p, 3, nt, st))) return rc;
   // ---- preparation: barotropic velocities of levels N and B
   const BarotArgs ba{{UN, UB}, {VN, VB}, {b2[UBN], b2[UBB]}, {b2[VBN], b2[VBB]}};
   LF_LAUNCHC(k_lf_uvbarot, np, nr, 2, st, ba, c.depth, s->d_cdk, np, K);
-  // ---- predictor
-  if ((rc = lf_vordiv(s, UN, VN, nc, st))) return rc;
+  // ---- predictor; the spectra of (UN, VN) wait in w2, which the fused forms use for nothing else
+  const bool spec = lf_wsolve_ok(s);
+  if ((rc = lf_vordiv(s, UN, VN, spec ? s->w2 : s->wVD, nc, st))) return rc;
   EosArgs ea;
   ea.ref_dens = c.ref_dens;
   ea.ptemp_dep = -c.beta_t;
@@ -1096,21 +1268,29 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
   ea.grav = c.grav;
   LF_LAUNCHC(k_lf_eos_hyd, np, nr, 1, st, TN, np, K, s->d_zck, s->d_cdk, ea, s->Dens, s->Hyd);
   if ((rc = lf_mom_rhs(s, UN, VN, UB, VB, true, gamma, 1.0 - gamma, PN, nr, st))) return rc;
+  if ((rc = lf_mom_grid(s, nc, st))) return rc;
   LF_LAUNCHC(k_lf_pred_uv, np, nr, 1, st, s->URHS, s->VRHS, UN, UB, VN, VB, b2[UBN], b2[VBN], b2[UBB], b2[VBB],
              s->d_two_omega, s->d_mu, c.depth, s->d_cdk, np, I, K, 0.5 * (2.0 * dt), c56dt, c.alpha > 0.0 ? 1 : 0,
              s->Upr, s->Vpr);
   if ((rc = lf_htrc(s, TN, UN, VN, c.depth, nr, st))) return rc;
+  if ((rc = lf_htrc_grid(s, nt, st))) return rc;
   LF_LAUNCH(k_lf_pred_trc, ntr, st, TN, TB, s->HT, c.depth + 0.0, c56dt, ntr, s->TSpr);
   // ---- corrector
-  if ((rc = lf_vordiv(s, s->Upr, s->Vpr, nc, st))) return rc;
+  if ((rc = lf_vordiv(s, s->Upr, s->Vpr, s->wVD, nc, st))) return rc;
   LF_LAUNCHC(k_lf_eos_hyd, np, nr, 1, st, s->TSpr, np, K, s->d_zck, s->d_cdk, ea, s->Dens, s->Hyd);
   const double alpha_ = 0.5, gamma_ = 0.5;
   const double cn = gamma_ + alpha_, cb = 1.0 - alpha_ - gamma_;  // 1 and 0: the present level alone
   if ((rc = lf_mom_rhs(s, s->Upr, s->Vpr, UN, VN, false, cn, cb, PN, nr, st))) return rc;
   // ImplUV (DOGCM_Phys_hspm_vfvm_mod.f90:666-748): implicit vertical viscosity, then
-  // backward-Euler lateral viscosity on vorticity and divergence
-  if ((rc = lf_vsolve(s, true, VSolve{{UN, VN}, {s->URHS, s->VRHS}, {UA, VA}}, nr, 2, st))) return rc;
-  if ((rc = lf_uv2vordiv(s, UA, VA, nc, s->d_dmom, st))) return rc;
+  // backward-Euler lateral viscosity on vorticity and divergence.  On spectra (see k_lf_wsolve), or
+  // on the grid for forms whose transforms round more than FP64 does
+  if (spec) {
+    if ((rc = lf_wsolve(s, true, s->w2, s->wVD, s->d_dmom, 2 * nr, st))) return rc;
+  } else {
+    if ((rc = lf_mom_grid(s, nc, st))) return rc;
+    if ((rc = lf_vsolve(s, true, VSolve{{UN, VN}, {s->URHS, s->VRHS}, {UA, VA}}, nr, 2, st))) return rc;
+    if ((rc = lf_uv2vordiv(s, UA, VA, s->wVD, nc, s->d_dmom, st))) return rc;
+  }
   if ((rc = dsht_vordiv2uv_d(p, s->wVD, s->wVD + nc, 2l * nc, 1, UA, VA, np, nc, st))) return rc;
   LF_LAUNCHC(k_lf_impl, np, nr, 1, st, UA, VA, UN, VN, b2[UBN], b2[VBN], PN, s->d_two_omega, s->d_mu, s->d_cs, c.depth,
              s->d_cdk, np, I, K, alpha_ * dt, dt, b2[UBT], b2[VBT], b2[AM2], b2[BG2], b2[SPM]);
@@ -1132,12 +1312,18 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
                      b2[DSP], PA, PN, s->SP[0]};
   LF_LAUNCH2(k_lf_final_uv, nc, np, st, fa, np, K, (long)nc);
   // ---- tracers
-  if ((rc = lf_vordiv(s, s->Upr, s->Vpr, nc, st))) return rc;
+  if ((rc = lf_div(s, s->Upr, s->Vpr, nc, st))) return rc;
   const double hm = (5.0 * c.depth + 8.0 * c.depth - c.depth) / 12.0;  // the time-centred thickness factor
   if ((rc = lf_htrc(s, s->TSpr, s->Upr, s->Vpr, hm, nr, st))) return rc;
   // ImplTRC (DOGCM_Phys_hspm_vfvm_mod.f90:544-662)
-  if ((rc = lf_vsolve(s, false, VSolve{{TN, nullptr}, {s->HT, nullptr}, {TA, nullptr}}, 2 * nr, 1, st))) return rc;
-  if ((rc = dsht_fwd_d(p, DSHT_VAL, TA, np, s->w1, nt, 1, nt, s->d_dtrc, st))) return rc;
+  if (spec) {
+    if ((rc = dsht_fwd_d(p, DSHT_VAL, TN, np, s->w2, nt, 1, nt, nullptr, st))) return rc;
+    if ((rc = lf_wsolve(s, false, s->w2, s->w1, s->d_dtrc, 2 * nr, st))) return rc;
+  } else {
+    if ((rc = lf_htrc_grid(s, nt, st))) return rc;
+    if ((rc = lf_vsolve(s, false, VSolve{{TN, nullptr}, {s->HT, nullptr}, {TA, nullptr}}, 2 * nr, 1, st))) return rc;
+    if ((rc = dsht_fwd_d(p, DSHT_VAL, TA, np, s->w1, nt, 1, nt, s->d_dtrc, st))) return rc;
+  }
   if ((rc = dsht_inv_d(p, DSHT_VAL, s->w1, nt, 1, TA, np, nt, nullptr, st))) return rc;
   LF_LAUNCH(k_lf_trc_final, ntr, st, TA, TN, TB, c.depth, ntr);
   return 0;

@@ -337,9 +337,10 @@ int dsht_prof_query(const char* name, double* total_ms, long* count, double* byt
  * A device-resident LF-AM3 dynamics step (DOGCM_TInt_LFAM3_advance_Dyn,
  * model/dogcm/src/tint/DOGCM_TInt_LFAM3_mod.f90:281-880) for up to max_runs independent runs
  * of one plan (truncation) and km layers: rigid lid, flat bottom of depth `depth`, linear
- * equation of state (EOS_Linear_mod.f90), no physics forcing.  Per run and step it makes the
- * reference's 42 forward and 28 inverse transform units per layer plus 9 + 9 barotropic
- * ones (dsht_lfam3_units), each transform over every layer of every active run in one call.
+ * equation of state (EOS_Linear_mod.f90), no physics forcing.  Per run and step it does the work
+ * of the reference's 42 forward and 28 inverse transform units per layer plus 9 + 9 barotropic
+ * ones (dsht_lfam3_units; it leaves out those whose results the step has or does not read), each
+ * transform over every layer of every active run in one call.
  * State in device memory (dsht_lfam3_state): U, V (km grids per run, run r layer k at grid
  * column r*km + k), tracers (potential temperature [K] then salinity per run: column
  * (2r + t)*km + k), surface pressure (one grid per run), at time levels B and N; a step
@@ -375,7 +376,7 @@ int dsht_lfam3_state(dsht_lfam3* pool, int field, int level, double** ptr, long*
 int dsht_lfam3_step(dsht_lfam3* pool, int nruns, void* stream);
 /* copies run src's state (levels B and N, rotation rate) into slot dst (pool compaction) */
 int dsht_lfam3_copy_run(dsht_lfam3* pool, int dst, int src, void* stream);
-/* transform units of one step of nruns runs (42 km + 9 forward, 28 km + 9 inverse each)   */
+/* transform units of the reference's step for nruns runs (42 km + 9 forward, 28 km + 9 inverse each)   */
 int dsht_lfam3_units(const dsht_lfam3* pool, int nruns, long* fwd_units, long* inv_units);
 
 /* ---------------------------------------------------------------- Redi/GM mixing

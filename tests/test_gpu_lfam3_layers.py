@@ -80,3 +80,32 @@ def test_fused_equals_separate(gpu, key):
         got.append(_read(pool, 0))
     for f in ("U", "V", "T", "S", "P"):
         assert rel_l2(got[1][f], got[0][f]) < TOL, f
+
+
+@pytest.mark.parametrize("km", [2, 8, 20, 64, 66, 120, 510, 960])
+@pytest.mark.parametrize("cfg", [{}, {"vvisc": 50.0, "vdiff": 20.0, "trc_sfc_bc": "D"}])
+def test_spectral_solve_equals_grid_solve(gpu, km, cfg):
+    """The implicit vertical solves on spectra, with the loads of up to 64 layers at once, in rounds
+    and with fewer systems a block where the layers fill the LDS (960: the grid form on both
+    sides), against the solves on the grid (taken with DSHT_TUNE_LEG = 2), for two of three runs."""
+    import torch
+    import dsht
+    import lfam3
+    import oracle
+    from conftest import rel_l2
+    N, I, J = 10, 32, 16
+    o = oracle.Oracle(N, I, J, 6.371e6)
+    got = []
+    for kind in (0, 2):
+        p, pool = _pool(N, I, J, km, 3, dt=1800.0, **cfg)
+        p.set_tuning(dsht.TUNE_LEG, kind)
+        for r in range(2):
+            _load(pool, r, lfam3.initial_state(o, km, seed=5 + r))
+            pool.set_rotation(r, OMEGA)
+        torch.cuda.synchronize()
+        pool.step(2)
+        torch.cuda.synchronize()
+        got.append([_read(pool, r) for r in range(2)])
+    for r in range(2):
+        for f in ("U", "V", "T", "S", "P"):
+            assert rel_l2(got[0][r][f], got[1][r][f]) < TOL, (r, f)
