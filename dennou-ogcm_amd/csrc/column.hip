@@ -244,7 +244,10 @@ __global__ __launch_bounds__(256) void k_col_quick(const double* __restrict__ om
 // SRC/dgtsv.f, the NRHS = 1 path), in its order of operations.  Each finished row of the
 // forward sweep (d, du and its right-hand side) waits for the backward sweep in one of three
 // places: the last RR rows in registers (slots fixed by unrolled loops), the LR rows before
-// them in LDS (row-major over the block's threads), the rest in `work` (d, du; pitch npts;
+// them in LDS (row-major over the block's threads).  Of the rest, up to 64 layers (REC) the
+// elimination is done a second time, into the registers that the backward sweep has left by
+// then: three loads a row, against three stores and three loads of a workspace (at most 20 rows;
+// T170L60: 16, 81 us before, 72 after); above that they wait in `work` (d, du; pitch npts;
 // 3 km values per point reserved) and qa (the right-hand side).  The grid has one thread per
 // point and few waves per SIMD, so the registers cost no occupancy.  The second superdiagonal
 // is nonzero only after a row interchange, so up to 64 layers a bit mask in a register
@@ -267,6 +270,19 @@ __global__ __launch_bounds__(256) void k_col_vdiff(const double* __restrict__ q0
                                                    const double* __restrict__ bfric, double* __restrict__ qa,
                                                    long ldo, double* __restrict__ work, int npts) {
 #pragma clang fp contract(off)
+  // REC: up to 64 layers with register rows
+  constexpr bool REC = MASK && RR > 0;
+  constexpr int RC = REC ? 64 - 2 - RR - LR : 1;  // most rows to compute again
+  static_assert(!REC || RC > 0, "rows left over");
+  __shared__ double sm1[MASK ? 65 : 1], sm2[MASK ? 65 : 1];
+  if constexpr (MASK) {  // the half levels' weights, the same for every column
+    for (int h = 1 + threadIdx.x; h < km; h += 256) {
+      const double s = cdk[h - 1] + cdk[h];
+      sm1[h] = cdk[h] / s;
+      sm2[h] = cdk[h - 1] / s;
+    }
+    __syncthreads();
+  }
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= npts) return;
   const double bf = (MOM && btm_dirichlet) ? ntl(bfric + i) : 0.0;
@@ -279,8 +295,13 @@ __global__ __launch_bounds__(256) void k_col_vdiff(const double* __restrict__ q0
   unsigned long long piv = 0ull;
   // half-level coefficient r[h] from the layers above (h-1) and below (h)
   auto rhalf = [&](int h, double kva, double e3a, double kvb, double e3b) {
-    const double s = cdk[h - 1] + cdk[h];
-    const double m1 = cdk[h] / s, m2 = cdk[h - 1] / s;
+    double m1, m2;
+    if constexpr (MASK) {
+      m1 = sm1[h], m2 = sm2[h];
+    } else {
+      const double s = cdk[h - 1] + cdk[h];
+      m1 = cdk[h] / s, m2 = cdk[h - 1] / s;
+    }
     const double num = m1 * kva + m2 * kvb;
     const double den = fdk[h] * (m1 * e3a + m2 * e3b);
     return num / den;
@@ -345,9 +366,8 @@ __global__ __launch_bounds__(256) void k_col_vdiff(const double* __restrict__ q0
   double rd[RR > 0 ? RR : 1], ru[RR > 0 ? RR : 1], rb[RR > 0 ? RR : 1];
   __shared__ double sd[LR > 0 ? LR : 1][256], su[LR > 0 ? LR : 1][256], sb[LR > 0 ? LR : 1][256];
   const int tx = threadIdx.x;
-  // step j with row j+2 = r2; the finished row j goes to register slot reg (reg >= 0), to
-  // LDS (J0 <= j < J1) or to the workspace
-  auto eliminate = [&](int j, const VdiffRow& r2, int reg) {
+  // step j with row j+2 = r2: the finished row j in od, ou, ob
+  auto elim = [&](int j, const VdiffRow& r2, double& od, double& ou, double& ob) {
     double du2;
     const bool keep = fabs(d) >= fabs(dl);  // no interchange
     if (keep) {
@@ -367,25 +387,49 @@ __global__ __launch_bounds__(256) void k_col_vdiff(const double* __restrict__ q0
       b = bn;
       bn = tb - fact * bn;
     }
-    if (RR > 0 && reg >= 0) {
-      rd[reg] = d;
-      ru[reg] = du;
-      rb[reg] = b;
-    } else if (LR > 0 && j >= J0) {
-      sd[j - J0][tx] = d;
-      su[j - J0][tx] = du;
-      sb[j - J0][tx] = b;
-    } else {
-      wd[(long)j * nw] = d;
-      wu[(long)j * nw] = du;
-      qa[(long)j * ldo + i] = b;
-    }
+    od = d, ou = du, ob = b;
     if (!MASK || !keep) w2[(long)j * nw] = du2;
     if (MASK && !keep) piv |= 1ull << j;
     d = dn, du = dun, b = bn;
     dl = r2.al, dn = r2.ad, dun = r2.au, bn = r2.b;
   };
+  // the finished row goes to register slot reg (reg >= 0), to LDS (J0 <= j < J1), or, of the rows
+  // above, to the workspace or nowhere (REC)
+  auto eliminate = [&](int j, const VdiffRow& r2, int reg) {
+    double od, ou, ob;
+    elim(j, r2, od, ou, ob);
+    if (RR > 0 && reg >= 0) {
+      rd[reg] = od;
+      ru[reg] = ou;
+      rb[reg] = ob;
+    } else if (LR > 0 && j >= J0) {
+      sd[j - J0][tx] = od;
+      su[j - J0][tx] = ou;
+      sb[j - J0][tx] = ob;
+    } else if (!REC) {
+      wd[(long)j * nw] = od;
+      wu[(long)j * nw] = ou;
+      qa[(long)j * ldo + i] = ob;
+    }
+  };
   int j = 0;
+  if constexpr (REC) {  // rows above J0: read again later, so without the streaming hint
+    for (; j < J0; j += CU) {
+      double pr[CU], pk[CU], pe[CU];
+#pragma unroll
+      for (int u = 0; u < CU; u++) {
+        const int k = j + u + 2;  // < km - 1: these rows end RR + LR rows and more above it
+        pr[u] = rhs[(long)k * ldg + i];
+        pk[u] = kv[(long)(k + 1) * ldg + i];
+        pe[u] = e3[(long)(k + 1) * ldg + i];
+      }
+#pragma unroll
+      for (int u = 0; u < CU; u++) {
+        if (j + u < J0) eliminate(j + u, build_row(j + u + 2, pr[u], pk[u], pe[u]), -1);
+      }
+    }
+    j = J0;
+  }
   for (; j + CU - 1 <= J1 - 1; j += CU) {  // rows j+2 .. j+CU+1 loaded together
     double pr[CU], pk[CU], pe[CU];
 #pragma unroll
@@ -482,6 +526,48 @@ __global__ __launch_bounds__(256) void k_col_vdiff(const double* __restrict__ q0
     for (; jl >= J0; jl--)
       back(jl, sd[jl - J0][tx], su[jl - J0][tx], (!MASK || ((piv >> jl) & 1ull)) ? w2[(long)jl * nw] : 0.0,
            sb[jl - J0][tx], ntl(q0 + (long)jl * ldg + i));
+  }
+  if constexpr (REC) {  // the first rows again, into the registers that the last ones have left
+    if (J0 == 0) return;
+    kv_c = kv[i];
+    e3_c = e3[i];
+    r_up = kv_c / (fdk[0] * e3_c);
+    const VdiffRow q0r = build_row(0, rhs[i], kv[ldg + i], e3[ldg + i]);
+    const VdiffRow q1r = build_row(1, rhs[ldg + i], kv[2 * ldg + i], e3[2 * ldg + i]);
+    d = q0r.ad, du = q0r.au, b = q0r.b;
+    dl = q1r.al, dn = q1r.ad, dun = q1r.au, bn = q1r.b;
+    double qd[RC], qu[RC], qb[RC];
+#pragma unroll
+    for (int u0 = 0; u0 < RC; u0 += CU) {
+      if (u0 >= J0) break;
+      double pr[CU], pk[CU], pe[CU];
+#pragma unroll
+      for (int v = 0; v < CU; v++) {
+        const int k = u0 + v + 2;
+        pr[v] = rhs[(long)k * ldg + i];
+        pk[v] = kv[(long)(k + 1) * ldg + i];
+        pe[v] = e3[(long)(k + 1) * ldg + i];
+      }
+#pragma unroll
+      for (int v = 0; v < CU; v++)
+        if (u0 + v < RC && u0 + v < J0) elim(u0 + v, build_row(u0 + v + 2, pr[v], pk[v], pe[v]), qd[u0 + v], qu[u0 + v], qb[u0 + v]);
+    }
+    constexpr int G = (RC + CU - 1) / CU * CU;
+#pragma unroll
+    for (int u0 = G - CU; u0 >= 0; u0 -= CU) {
+      if (u0 >= J0) continue;
+      double pv[CU], pq[CU];
+#pragma unroll
+      for (int v = 0; v < CU; v++) {
+        const long r = u0 + v < J0 ? u0 + v : J0 - 1;
+        pv[v] = ((piv >> r) & 1ull) ? w2[r * nw] : 0.0;
+        pq[v] = ntl(q0 + r * ldg + i);
+      }
+#pragma unroll
+      for (int v = CU - 1; v >= 0; v--)
+        if (u0 + v < RC && u0 + v < J0) back(u0 + v, qd[u0 + v], qu[u0 + v], pv[v], qb[u0 + v], pq[v]);
+    }
+    return;
   }
   int jb = (LR > 0 ? J0 : J1) - 1;
   for (; jb - (CU - 1) >= 0; jb -= CU) {  // rows jb .. jb-CU+1 loaded together
