@@ -115,6 +115,21 @@ struct FftPlan {
 
 constexpr int FFT_FIELDS_MAX = 3;
 
+// What the FP64 inverse FFT does with a grid value x as it stores it, instead of a pass over the
+// grid afterwards (columns of pitch ld, as the grid's columns):
+//   E_RHS   y = (y + x) + in0, for columns from split on with y2 in the output's place (its column 0)
+//   E_PRED  y = (h (2 in0 + in1) / 3 + c x) / h
+//   E_TRC   t = h x / h: y = t, o2 = o1, o1 = t
+enum InvEpiKind { E_NONE = 0, E_RHS, E_PRED, E_TRC };
+struct InvEpi {
+  int kind = E_NONE, split = 0;
+  double* y2 = nullptr;
+  const double *in0 = nullptr, *in1 = nullptr;
+  double *o1 = nullptr, *o2 = nullptr;
+  long ld = 0;
+  double h = 1.0, c = 0.0;
+};
+
 struct FftArgs {
   int I, M, N, J;
   int ncols;
@@ -137,6 +152,7 @@ struct FftArgs {
   int nf;                  // fields in one launch (FP64 register kernels; grid y), each of ncols columns
   const void* more_in[FFT_FIELDS_MAX - 1];  // inputs and outputs of fields 1 .. nf-1
   void* more_out[FFT_FIELDS_MAX - 1];
+  InvEpi epi;              // inverse, one FP64 field of a register kernel
 };
 
 // ---------------------------------------------------------------- workspace
@@ -247,6 +263,9 @@ int fwd_add(dsht_plan* p, const double* xy, long ldg, double* w, long sl, long s
             hipStream_t s);
 int uv2vordiv_scaled(dsht_plan* p, const double* u, const double* v, const double* rowscale, long ldg, double* vor,
                      double* div, long sl, long sc, int ncols, const double* diag, hipStream_t s);
+// xy = w_xy's inverse with an epilogue in its FFT; FP64 form with a register FFT only (uv_scaled_ok)
+int inv_epi(dsht_plan* p, const double* w, long sl, long sc, double* xy, long ldg, int ncols, const InvEpi& e,
+            hipStream_t s);
 // its divergence alone
 int div_scaled(dsht_plan* p, const double* u, const double* v, const double* rowscale, long ldg, double* div, long sl,
                long sc, int ncols, hipStream_t s);
@@ -269,7 +288,8 @@ int launch_fft_fwd(const dsht_plan* p, const double* const* xy, int nf, long ldg
 // for field i and rowscale applies to those fields alone
 bool fft_reg_ok(const dsht_plan* p);
 int launch_fft_inv(const dsht_plan* p, const double2* const* G, int nf, long gld, int ncols, double* const* xy, long ldg,
-                   hipStream_t s, const double* rowscale = nullptr, int deriv = 0);
+                   hipStream_t s, const double* rowscale = nullptr, int deriv = 0,
+                   const InvEpi* epi = nullptr);
 // FP32 Fourier intermediates of the split-precision forms; colmax (nullable) receives the
 // per-column max |G| as float bits
 bool reg_fft_supported(int M);

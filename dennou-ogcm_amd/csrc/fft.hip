@@ -538,13 +538,14 @@ static int fft_fwd_any(const dsht_plan* p, const XT* const* xys, int nf, long ld
 
 template <typename GT, typename XT>
 static int fft_inv_any(const dsht_plan* p, const GT* const* Gs, int nf, long gld, int ncols, XT* const* xys, long ldg,
-                       hipStream_t s, const double* rowscale, int deriv, XT* xy2) {
+                       hipStream_t s, const double* rowscale, int deriv, XT* xy2, const InvEpi* epi = nullptr) {
   FftArgs a = fft_args(p, ldg, ncols, gld);
+  if (epi) a.epi = *epi;
   a.rowscale = rowscale;
   a.deriv = deriv;
   a.xy2 = xy2;
-  if ((deriv || xy2) && !fft_reg_ok(p))
-    return fail(DSHT_EUNSUPPORTED, "derivative inverse FFT needs a register kernel");
+  if ((deriv || xy2 || epi) && !fft_reg_ok(p))
+    return fail(DSHT_EUNSUPPORTED, "derivative and epilogue inverse FFTs need a register kernel");
   // inverse: FP32 arithmetic on the split forms' FP32 Fourier coefficients (each output point
   // is a sum of already-FP32 terms; the error stays at FP32 rounding of the output scale)
   a.fp32 = (sizeof(GT) == 8 && p->fft_kind == 0) ? 1 : 0;
@@ -588,8 +589,8 @@ int launch_fft_fwd(const dsht_plan* p, const double* const* xy, int nf, long ldg
 }
 
 int launch_fft_inv(const dsht_plan* p, const double2* const* G, int nf, long gld, int ncols, double* const* xy, long ldg,
-                   hipStream_t s, const double* rowscale, int deriv) {
-  return fft_inv_any<double2, double>(p, G, nf, gld, ncols, xy, ldg, s, rowscale, deriv, nullptr);
+                   hipStream_t s, const double* rowscale, int deriv, const InvEpi* epi) {
+  return fft_inv_any<double2, double>(p, G, nf, gld, ncols, xy, ldg, s, rowscale, deriv, nullptr, epi);
 }
 
 int launch_fft_fwd32(const dsht_plan* p, const double* xy, long ldg, int ncols, float2* G, long gld,

@@ -448,8 +448,9 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_fwd_r(const XT* __restrict__
 // 2 (dual): both from one read of the coefficients -- the field into xy, then the
 // derivative, times a.rowscale, into a.xy2 -- the coefficients stay in registers between the
 // two passes; 3: fields of one launch (grid y) of either kind, bit y of a.deriv set for the
-// derivative of field y.  Separate instantiations keep each form's register allocation.  XT:
-// grid element type.
+// derivative of field y; 4, 5, 6 (FP64): the field with the epilogue E_RHS, E_PRED, E_TRC, whose
+// operands are loaded before the last pass.  Separate instantiations keep each form's register
+// allocation.  XT: grid element type.
 template <int R1, int R2, int NT, typename GT, typename V, int MODE, typename XT>
 __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__ G, XT* __restrict__ xy,
                                                   FftArgs a) {
@@ -570,12 +571,69 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__
     __syncthreads();
     if (rr2 < ROWS) {
       V u[R1];
+      int j, c;
+      const bool ok = map_row(a, g0, rr2, ROWS, j, c);
+      constexpr int NE = MODE == 4 || MODE == 5 ? 2 : MODE == 6 ? 1 : 0;  // operand arrays of the epilogue
+      // operands in chunks of CE values, one chunk ahead, the first before the last pass: all at once
+      // spilled registers
+      constexpr int CE = 4;
+      dvec2 e[2][NE ? NE : 1][NE ? CE : 1];
+      XT *x = nullptr, *o1 = nullptr, *o2 = nullptr;
+      const double *e0 = nullptr, *e1 = nullptr;
+      auto operands = [&](auto Q) {
+        constexpr int q = decltype(Q)::value;
+#pragma unroll
+        for (int i = 0; i < CE; i++) {
+          const int k1 = q * CE + i;
+          if (k1 >= R1) break;
+          e[q & 1][0][i] = __builtin_nontemporal_load(reinterpret_cast<const dvec2*>(e0 + 2 * R2 * k1));
+          if constexpr (NE == 2)
+            e[q & 1][1][i] = __builtin_nontemporal_load(reinterpret_cast<const dvec2*>(e1 + 2 * R2 * k1));
+        }
+      };
+      if constexpr (NE > 0) {
+        if (ok) {
+          const long jo = (long)j * (2 * M) + 2 * k2, eo = c * a.epi.ld + jo;
+          x = (MODE == 4 && c >= a.epi.split ? a.epi.y2 + (c - a.epi.split) * a.ldg : xy + c * a.ldg) + jo;
+          o1 = a.epi.o1 + eo, o2 = a.epi.o2 + eo;
+          e0 = MODE == 4 ? x : MODE == 5 ? a.epi.in0 + eo : o1;
+          e1 = MODE == 4 ? a.epi.in0 + eo : a.epi.in1 + eo;
+        }
+      }
       const V* Y = buf + rr2 * SR + k2;
 #pragma unroll
       for (int p = 0; p < R1; p++) u[p] = Y[p * PY];
       dft<R1, +1>(u);
-      int j, c;
-      if (map_row(a, g0, rr2, ROWS, j, c)) {
+      if constexpr (NE > 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (ok) {
+          operands(std::integral_constant<int, 0>{});
+          sfor<(R1 + CE - 1) / CE>([&](auto Q) {
+            constexpr int q = decltype(Q)::value;
+            if constexpr ((q + 1) * CE < R1) operands(std::integral_constant<int, q + 1>{});
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < CE; i++) {
+              const int k1 = q * CE + i;
+              if (k1 >= R1) break;
+              const dvec2 v = {u[k1].x, u[k1].y}, a0 = e[q & 1][0][i];
+              const int o = 2 * R2 * k1;
+              dvec2 t;
+              if constexpr (MODE == 4) {
+                t = (a0 + v) + e[q & 1][1][i];
+              } else if constexpr (MODE == 5) {
+                t = (a.epi.h * (2.0 * a0 + e[q & 1][1][i]) / 3.0 + a.epi.c * v) / a.epi.h;
+              } else {
+                t = a.epi.h * v / a.epi.h;
+                store_pair(o1 + o, t.x, t.y);
+                store_pair(o2 + o, a0.x, a0.y);
+              }
+              store_pair(x + o, t.x, t.y);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          });
+        }
+      } else if (ok) {
         // dual: the field unscaled into xy, the derivative times the row scale into xy2
         const double s = (a.rowscale && (MODE < 2 || deriv)) ? a.rowscale[j] : 1.0;
         XT* out = (MODE == 2 && pass == 1) ? reinterpret_cast<XT*>(a.xy2) : xy;
@@ -655,6 +713,13 @@ static int reg_inv_nt(const GT* G, const FftArgs& a, XT* xy, hipStream_t s) {
   if (a.xy2) return reg_inv_mode<R1, R2, NT, GT, V, 2, XT>(G, a, xy, s);
   if constexpr (sizeof(GT) == 16) {
     if (a.deriv && a.nf > 1) return reg_inv_mode<R1, R2, NT, GT, V, 3, XT>(G, a, xy, s);
+    if constexpr (sizeof(XT) == 8) {
+      switch (a.epi.kind) {
+        case E_RHS: return reg_inv_mode<R1, R2, NT, GT, V, 4, XT>(G, a, xy, s);
+        case E_PRED: return reg_inv_mode<R1, R2, NT, GT, V, 5, XT>(G, a, xy, s);
+        case E_TRC: return reg_inv_mode<R1, R2, NT, GT, V, 6, XT>(G, a, xy, s);
+      }
+    }
   }
   if (a.deriv) return reg_inv_mode<R1, R2, NT, GT, V, 1, XT>(G, a, xy, s);
   return reg_inv_mode<R1, R2, NT, GT, V, 0, XT>(G, a, xy, s);

@@ -1273,8 +1273,24 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
              s->d_two_omega, s->d_mu, c.depth, s->d_cdk, np, I, K, 0.5 * (2.0 * dt), c56dt, c.alpha > 0.0 ? 1 : 0,
              s->Upr, s->Vpr);
   if ((rc = lf_htrc(s, TN, UN, VN, c.depth, nr, st))) return rc;
-  if ((rc = lf_htrc_grid(s, nt, st))) return rc;
-  LF_LAUNCH(k_lf_pred_trc, ntr, st, TN, TB, s->HT, c.depth + 0.0, c56dt, ntr, s->TSpr);
+  // the tracers' updates as the FFT stores their grids, or in a pass after it: T170L60 133 -> 85 (this)
+  // and 134 -> 100 us.  Not where a latitude row is no whole number of 128-byte lines, whose store
+  // runs share lines with their neighbours': the step at 540 x 270 x 30 2.54 -> 2.55 ms, at
+  // 270 x 136 x 30 816 -> 833 us, while 384 x 192 x 30 gains 2 %
+  const bool epi = uv_scaled_ok(p) && I % 16 == 0;
+  if (epi) {
+    InvEpi e;
+    e.kind = E_PRED;
+    e.in0 = TN;
+    e.in1 = TB;
+    e.ld = np;
+    e.h = c.depth;
+    e.c = c56dt;
+    if ((rc = inv_epi(p, s->w1, nt, 1, s->TSpr, np, nt, e, st))) return rc;
+  } else {
+    if ((rc = lf_htrc_grid(s, nt, st))) return rc;
+    LF_LAUNCH(k_lf_pred_trc, ntr, st, TN, TB, s->HT, c.depth + 0.0, c56dt, ntr, s->TSpr);
+  }
   // ---- corrector
   if ((rc = lf_vordiv(s, s->Upr, s->Vpr, s->wVD, nc, st))) return rc;
   LF_LAUNCHC(k_lf_eos_hyd, np, nr, 1, st, s->TSpr, np, K, s->d_zck, s->d_cdk, ea, s->Dens, s->Hyd);
@@ -1323,6 +1339,15 @@ int dsht_lfam3_step(dsht_lfam3* s, int nr, void* stream) {
     if ((rc = lf_htrc_grid(s, nt, st))) return rc;
     if ((rc = lf_vsolve(s, false, VSolve{{TN, nullptr}, {s->HT, nullptr}, {TA, nullptr}}, 2 * nr, 1, st))) return rc;
     if ((rc = dsht_fwd_d(p, DSHT_VAL, TA, np, s->w1, nt, 1, nt, s->d_dtrc, st))) return rc;
+  }
+  if (epi) {
+    InvEpi e;
+    e.kind = E_TRC;
+    e.o1 = TN;
+    e.o2 = TB;
+    e.ld = np;
+    e.h = c.depth;
+    return inv_epi(p, s->w1, nt, 1, TA, np, nt, e, st);
   }
   if ((rc = dsht_inv_d(p, DSHT_VAL, s->w1, nt, 1, TA, np, nt, nullptr, st))) return rc;
   LF_LAUNCH(k_lf_trc_final, ntr, st, TA, TN, TB, c.depth, ntr);
