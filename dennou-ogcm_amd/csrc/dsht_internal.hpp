@@ -152,7 +152,7 @@ struct FftArgs {
   int nf;                  // fields in one launch (FP64 register kernels; grid y), each of ncols columns
   const void* more_in[FFT_FIELDS_MAX - 1];  // inputs and outputs of fields 1 .. nf-1
   void* more_out[FFT_FIELDS_MAX - 1];
-  InvEpi epi;              // inverse, one FP64 field of a register kernel
+  const InvEpi* epi;       // inverse, one FP64 field of a register kernel (host memory, nullable)
 };
 
 // ---------------------------------------------------------------- workspace
@@ -213,8 +213,9 @@ struct dsht_plan {
                        // split forms' inverse FFT), 1 = LDS Stockham, 2 = register FFT in
                        // 128-thread blocks, 3 = register FFT with FP64 arithmetic in every form
   int fft_order = 1;   // register FFT row-group order: 0 packed, 1 latitude-major (default)
-  int leg_kind = 0;    // contractions.  FP64: 0 = LDS-staged inverse, fragment-stream forward;
-                       // 1/3 = LDS-staged; 2 = per-wave fragment streams.
+  int leg_kind = 0;    // contractions.  FP64: 0 = whole-K LDS staging where it fits, else K-chunked
+                       // inverse and fragment-stream forward; 1/3 = K-chunked LDS staging; 2 =
+                       // per-wave fragment streams.
                        // Split-form inverse: 0 = per form (whole-K LDS staging for BF16X6 and
                        // FP16X3, packed data panels otherwise), 2 = packed panels, 3 = whole-K
 };

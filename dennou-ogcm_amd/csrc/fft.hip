@@ -540,7 +540,7 @@ template <typename GT, typename XT>
 static int fft_inv_any(const dsht_plan* p, const GT* const* Gs, int nf, long gld, int ncols, XT* const* xys, long ldg,
                        hipStream_t s, const double* rowscale, int deriv, XT* xy2, const InvEpi* epi = nullptr) {
   FftArgs a = fft_args(p, ldg, ncols, gld);
-  if (epi) a.epi = *epi;
+  a.epi = epi;
   a.rowscale = rowscale;
   a.deriv = deriv;
   a.xy2 = xy2;

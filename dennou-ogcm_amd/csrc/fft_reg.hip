@@ -444,16 +444,72 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_fwd_r(const XT* __restrict__
   }
 }
 
+// the stores of a thread's R1 values of row (j, c) with an epilogue (InvEpi).  Its operands come in
+// chunks of CE values, one chunk ahead, the first after the last pass: any earlier or more of them
+// spilled registers (512 x 256 x 120, E_PRED: 85 us; 97 with the first chunk before the pass)
+template <int MODE, int R1, int R2>
+__device__ __forceinline__ void store_epi(const FftArgs& a, const InvEpi& epi, double* __restrict__ xy,
+                                          const double2 (&u)[R1], int j, int c, int k2) {
+  constexpr int NE = MODE == 6 ? 1 : 2, CE = 4;
+  __builtin_amdgcn_sched_barrier(0);
+  const long jo = (long)j * (2 * R1 * R2) + 2 * k2, eo = c * epi.ld + jo;
+  double* x = (MODE == 4 && c >= epi.split ? epi.y2 + (c - epi.split) * a.ldg : xy + c * a.ldg) + jo;
+  double *o1 = epi.o1 + eo, *o2 = epi.o2 + eo;
+  const double* e0 = MODE == 4 ? x : MODE == 5 ? epi.in0 + eo : o1;
+  const double* e1 = MODE == 4 ? epi.in0 + eo : epi.in1 + eo;
+  dvec2 e[2][NE][CE];
+  auto operands = [&](auto Q) {
+    constexpr int q = decltype(Q)::value;
+#pragma unroll
+    for (int i = 0; i < CE; i++) {
+      const int k1 = q * CE + i;
+      if (k1 >= R1) break;
+      e[q & 1][0][i] = __builtin_nontemporal_load(reinterpret_cast<const dvec2*>(e0 + 2 * R2 * k1));
+      if constexpr (NE == 2)
+        e[q & 1][1][i] = __builtin_nontemporal_load(reinterpret_cast<const dvec2*>(e1 + 2 * R2 * k1));
+    }
+  };
+  operands(std::integral_constant<int, 0>{});
+  sfor<(R1 + CE - 1) / CE>([&](auto Q) {
+    constexpr int q = decltype(Q)::value;
+    if constexpr ((q + 1) * CE < R1) operands(std::integral_constant<int, q + 1>{});
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < CE; i++) {
+      const int k1 = q * CE + i;
+      if (k1 >= R1) break;
+      const dvec2 v = {u[k1].x, u[k1].y}, a0 = e[q & 1][0][i];
+      const int o = 2 * R2 * k1;
+      dvec2 t;
+      if constexpr (MODE == 4) {
+        t = (a0 + v) + e[q & 1][1][i];
+      } else if constexpr (MODE == 5) {
+        t = (epi.h * (2.0 * a0 + e[q & 1][1][i]) / 3.0 + epi.c * v) / epi.h;
+      } else {
+        t = epi.h * v / epi.h;
+        store_pair(o1 + o, t.x, t.y);
+        store_pair(o2 + o, a0.x, a0.y);
+      }
+      store_pair(x + o, t.x, t.y);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  });
+}
+
+struct NoEpi {};
+template <int MODE>
+using EpiArg = std::conditional_t<(MODE >= 4), InvEpi, NoEpi>;
+
 // MODE 0: the field; 1: its longitude derivative (transform i m X_m, times a.rowscale);
 // 2 (dual): both from one read of the coefficients -- the field into xy, then the
 // derivative, times a.rowscale, into a.xy2 -- the coefficients stay in registers between the
 // two passes; 3: fields of one launch (grid y) of either kind, bit y of a.deriv set for the
 // derivative of field y; 4, 5, 6 (FP64): the field with the epilogue E_RHS, E_PRED, E_TRC, whose
-// operands are loaded before the last pass.  Separate instantiations keep each form's register
+// stores are store_epi's.  Separate instantiations keep each form's register
 // allocation.  XT: grid element type.
 template <int R1, int R2, int NT, typename GT, typename V, int MODE, typename XT>
 __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__ G, XT* __restrict__ xy,
-                                                  FftArgs a) {
+                                                  FftArgs a, EpiArg<MODE> epi) {
   if constexpr (sizeof(GT) == 16) {  // fields of one launch
     if (blockIdx.y) {
       G = static_cast<const GT*>(a.more_in[blockIdx.y - 1]);
@@ -571,75 +627,22 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__
     __syncthreads();
     if (rr2 < ROWS) {
       V u[R1];
-      int j, c;
-      const bool ok = map_row(a, g0, rr2, ROWS, j, c);
-      constexpr int NE = MODE == 4 || MODE == 5 ? 2 : MODE == 6 ? 1 : 0;  // operand arrays of the epilogue
-      // operands in chunks of CE values, one chunk ahead, the first before the last pass: all at once
-      // spilled registers
-      constexpr int CE = 4;
-      dvec2 e[2][NE ? NE : 1][NE ? CE : 1];
-      XT *x = nullptr, *o1 = nullptr, *o2 = nullptr;
-      const double *e0 = nullptr, *e1 = nullptr;
-      auto operands = [&](auto Q) {
-        constexpr int q = decltype(Q)::value;
-#pragma unroll
-        for (int i = 0; i < CE; i++) {
-          const int k1 = q * CE + i;
-          if (k1 >= R1) break;
-          e[q & 1][0][i] = __builtin_nontemporal_load(reinterpret_cast<const dvec2*>(e0 + 2 * R2 * k1));
-          if constexpr (NE == 2)
-            e[q & 1][1][i] = __builtin_nontemporal_load(reinterpret_cast<const dvec2*>(e1 + 2 * R2 * k1));
-        }
-      };
-      if constexpr (NE > 0) {
-        if (ok) {
-          const long jo = (long)j * (2 * M) + 2 * k2, eo = c * a.epi.ld + jo;
-          x = (MODE == 4 && c >= a.epi.split ? a.epi.y2 + (c - a.epi.split) * a.ldg : xy + c * a.ldg) + jo;
-          o1 = a.epi.o1 + eo, o2 = a.epi.o2 + eo;
-          e0 = MODE == 4 ? x : MODE == 5 ? a.epi.in0 + eo : o1;
-          e1 = MODE == 4 ? a.epi.in0 + eo : a.epi.in1 + eo;
-        }
-      }
       const V* Y = buf + rr2 * SR + k2;
 #pragma unroll
       for (int p = 0; p < R1; p++) u[p] = Y[p * PY];
       dft<R1, +1>(u);
-      if constexpr (NE > 0) {
-        __builtin_amdgcn_sched_barrier(0);
-        if (ok) {
-          operands(std::integral_constant<int, 0>{});
-          sfor<(R1 + CE - 1) / CE>([&](auto Q) {
-            constexpr int q = decltype(Q)::value;
-            if constexpr ((q + 1) * CE < R1) operands(std::integral_constant<int, q + 1>{});
-            __builtin_amdgcn_sched_barrier(0);
+      int j, c;
+      if (map_row(a, g0, rr2, ROWS, j, c)) {
+        if constexpr (MODE >= 4) {
+          store_epi<MODE, R1, R2>(a, epi, xy, u, j, c, k2);
+        } else {
+          // dual: the field unscaled into xy, the derivative times the row scale into xy2
+          const double s = (a.rowscale && (MODE < 2 || deriv)) ? a.rowscale[j] : 1.0;
+          XT* out = (MODE == 2 && pass == 1) ? reinterpret_cast<XT*>(a.xy2) : xy;
+          XT* x = out + c * a.ldg + (long)j * (2 * M);
 #pragma unroll
-            for (int i = 0; i < CE; i++) {
-              const int k1 = q * CE + i;
-              if (k1 >= R1) break;
-              const dvec2 v = {u[k1].x, u[k1].y}, a0 = e[q & 1][0][i];
-              const int o = 2 * R2 * k1;
-              dvec2 t;
-              if constexpr (MODE == 4) {
-                t = (a0 + v) + e[q & 1][1][i];
-              } else if constexpr (MODE == 5) {
-                t = (a.epi.h * (2.0 * a0 + e[q & 1][1][i]) / 3.0 + a.epi.c * v) / a.epi.h;
-              } else {
-                t = a.epi.h * v / a.epi.h;
-                store_pair(o1 + o, t.x, t.y);
-                store_pair(o2 + o, a0.x, a0.y);
-              }
-              store_pair(x + o, t.x, t.y);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-          });
+          for (int k1 = 0; k1 < R1; k1++) store_pair(x + 2 * (k2 + R2 * k1), (double)u[k1].x * s, (double)u[k1].y * s);
         }
-      } else if (ok) {
-        // dual: the field unscaled into xy, the derivative times the row scale into xy2
-        const double s = (a.rowscale && (MODE < 2 || deriv)) ? a.rowscale[j] : 1.0;
-        XT* out = (MODE == 2 && pass == 1) ? reinterpret_cast<XT*>(a.xy2) : xy;
-        XT* x = out + c * a.ldg + (long)j * (2 * M);
-#pragma unroll
-        for (int k1 = 0; k1 < R1; k1++) store_pair(x + 2 * (k2 + R2 * k1), (double)u[k1].x * s, (double)u[k1].y * s);
       }
     }
   }  // pass
@@ -702,8 +705,10 @@ static int reg_inv_mode(const GT* G, const FftArgs& a, XT* xy, hipStream_t s) {
   using C = RegFft<R1, R2, NT, V>;
   static const long cap = resident_grid(k_fft_inv_r<R1, R2, NT, GT, V, MODE, XT>, C::THREADS, C::LDS);
   const long nb = field_grid(row_groups(a, C::ROWS), cap, a.nf);
+  EpiArg<MODE> epi;
+  if constexpr (MODE >= 4) epi = *a.epi;
   hipLaunchKernelGGL((k_fft_inv_r<R1, R2, NT, GT, V, MODE, XT>), dim3((unsigned)nb, a.nf), dim3(C::THREADS), C::LDS, s,
-                     G, xy, a);
+                     G, xy, a, epi);
   DSHT_HIP(hipGetLastError());
   return 0;
 }
@@ -714,7 +719,8 @@ static int reg_inv_nt(const GT* G, const FftArgs& a, XT* xy, hipStream_t s) {
   if constexpr (sizeof(GT) == 16) {
     if (a.deriv && a.nf > 1) return reg_inv_mode<R1, R2, NT, GT, V, 3, XT>(G, a, xy, s);
     if constexpr (sizeof(XT) == 8) {
-      switch (a.epi.kind) {
+      switch (a.epi ? a.epi->kind : E_NONE) {
+        case E_NONE: break;
         case E_RHS: return reg_inv_mode<R1, R2, NT, GT, V, 4, XT>(G, a, xy, s);
         case E_PRED: return reg_inv_mode<R1, R2, NT, GT, V, 5, XT>(G, a, xy, s);
         case E_TRC: return reg_inv_mode<R1, R2, NT, GT, V, 6, XT>(G, a, xy, s);

@@ -577,8 +577,9 @@ int launch_leg_fwd(const dsht_plan* p, int op, const LegFwdArgs& a, hipStream_t 
                    ntab[] = {1, 1, 1, 2, 2, 2};
   leg_work(p, nin[op], nout[op], nt[op], ntab[op], true, a.ncols, &by, &fl);
   ProfScope ps("leg_fwd", s, by, fl);
-  // forward: the per-wave fragment-stream kernel by default (measured 165 against 174 us at
-  // T170 x 360); DSHT_TUNE_LEG = 1 or 3 selects the LDS-staged kernel
+  // The whole-K staged kernel where one block's latitudes fit its LDS (F_VAL T170 x 360: 137-144 us;
+  // the fragment streams 178, the K-chunked kernel below 187), else the fragment streams.
+  // DSHT_TUNE_LEG = 1 or 3 selects the K-chunked kernel, 2 the fragment streams
   if (p->leg_kind == 0 && leg_fwd_staged_ok(p, op)) return launch_leg_fwd_staged(p, op, a, s);
   if (op == F_VALSUBALPHA || a.add) return fail(DSHT_EUNSUPPORTED, "launch_leg_fwd: op %d needs the staged kernel", op);
   if (p->leg_kind == 0 || p->leg_kind == 2) return launch_leg_fwd_direct(p, op, a, s);
@@ -593,8 +594,8 @@ int launch_leg_fwd(const dsht_plan* p, int op, const LegFwdArgs& a, hipStream_t 
 }
 
 int launch_leg_inv(const dsht_plan* p, int op, const LegInvArgs& a, hipStream_t s) {
-  // the fused value/gradient form defaults to 16-column blocks (its 32-column form needs the
-  // shorter K chunk to fit its registers; measured 185 against 191 us at T170 x 240)
+  // K-chunked kernel: the fused value/gradient form defaults to 16-column blocks (its 32-column
+  // form needs the shorter K chunk to fit its registers)
   const bool wide = p->leg_cb ? p->leg_cb == 32 : (op != I_VGRAD && a.ncols > 16);
   double by, fl;
   static const int nin[] = {1, 1, 1, 2, 2, 1}, nout[] = {1, 1, 1, 1, 2, 3}, nt[] = {1, 1, 1, 2, 4, 2},
@@ -605,6 +606,8 @@ int launch_leg_inv(const dsht_plan* p, int op, const LegInvArgs& a, hipStream_t 
   const int nw = op == I_VGRAD ? (a.G0 ? 1 : 0) + (a.G1 ? 1 : 0) + (a.G2 ? 1 : 0) : nout[op];
   leg_work(p, nin[op], nw, nt[op], ntab[op], false, a.ncols, &by, &fl);
   ProfScope ps("leg_inv", s, by, fl);
+  // the whole-K staged kernel where a block's spectra fit its LDS (fused T170 x 240: 149 us, the
+  // K-chunked kernel 187), else the K-chunked one; DSHT_TUNE_LEG as for the forward
   if (p->leg_kind == 2) return launch_leg_inv_direct(p, op, a, s);
   if (p->leg_kind == 0 && leg_inv_staged_ok(p, op)) return launch_leg_inv_staged(p, op, a, s);
   switch (op) {

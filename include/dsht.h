@@ -287,9 +287,9 @@ int dsht_coef_d(dsht_plan* plan, int which, const double* params, int nparams, d
                                   blocks; FP32 arithmetic in the inverse FFT of the split forms,
                                   whose Fourier coefficients are FP32), 1 = LDS Stockham, 2 = register kernel, 128-thread blocks,
                                   3 = register kernel, FP64 arithmetic in every form */
-#define DSHT_TUNE_LEG 3        /* Legendre contractions.  FP64: 0 = LDS-staged inverse with the
-                                  fragment-stream forward (default), 1 or 3 = LDS-staged, 2 = per-wave
-                                  fragment streams.  Split-form inverse: 0 = per form (default:
+#define DSHT_TUNE_LEG 3        /* Legendre contractions.  FP64: 0 = whole-K LDS staging where it
+                                  fits (default; else 3's inverse and 2's forward), 1 or 3 = K-chunked
+                                  LDS staging, 2 = per-wave fragment streams.  Split-form inverse: 0 = per form (default:
                                   whole-K LDS staging for BF16X6 and FP16X3, packed data panels otherwise),
                                   2 = packed data panels, 3 = whole-K LDS staging; 1 (a retired
                                   design) returns DSHT_EUNSUPPORTED.  (Key 4 is retired.) */
