@@ -529,7 +529,8 @@ def column_bench(torch, dsht, reps=21, nsets=3):
 def lfam3_bench(torch, dsht, steps=20, N=NMAX, km=KM):
     """The device LF-AM3 dynamics step at T170L60 (I=512, J=256): one run, and four runs of
     the same truncation in one pool (each transform over all their layers in one call).
-    One step = (42 KM + 9) forward + (28 KM + 9) inverse units per run."""
+    One step = (42 KM + 9) forward + (28 KM + 9) inverse units per run, the reference's count: the
+    library leaves out those whose results the step has or does not read."""
     from dsht import serve
 
     out = {"workload": f"LF-AM3 dynamics step (rigid lid, linear EOS), T{N}L{km} (I={IM}, J={JM}), FP64, "
