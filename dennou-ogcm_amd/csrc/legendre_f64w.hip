@@ -378,9 +378,11 @@ __global__ __launch_bounds__(WAVES * 64, 2) void k_f64_fwd_wk(LegFwdArgs a, int 
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           const int n = m + par + 2 * ((par ? t - tE : t) * TILE + krow + 4 * i);
-          const int l = n <= N ? n * (n + 1) + (part ? -m : m) : 0;
+          const bool mine = n <= N && !(m == 0 && part);  // a coefficient that this lane stores
+          const int l = mine ? n * (n + 1) + (part ? -m : m) : 0;
           dv[o][i] = dg ? dg[l] : 1.0;
-          if constexpr (OP == F_VAL) old[o][i] = a.add ? a.W0[l * a.sl + (long)c * a.sc] : 0.0;
+          // other coefficients are being stored by other lanes
+          if constexpr (OP == F_VAL) old[o][i] = a.add && mine ? a.W0[l * a.sl + (long)c * a.sc] : 0.0;
         }
       }
 #pragma unroll
