@@ -61,8 +61,9 @@ struct RediArgs {
 
 // Quotients by one divisor d from its reciprocal: two Newton steps on the hardware estimate, and a
 // quotient corrected by its exact remainder (Markstein, IBM J. Res. Dev. 34, 1990), which rounds as
-// the division does where no intermediate leaves the normal range.  A divisor outside
-// (2^-900, 2^900), 0, an infinity or NaN is divided by as such.
+// the division does where no intermediate leaves the normal range.  Where the quotient overflows the
+// correction is NaN, and v_div_fixup_f64 makes the infinity of it that the division gives.  A divisor
+// outside (2^-900, 2^900), 0, an infinity or NaN is divided by as such.
 __device__ inline bool recip_ok(double d) {
   const double m = fabs(d);
   return m > 0x1p-900 && m < 0x1p900;
