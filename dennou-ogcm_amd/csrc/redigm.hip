@@ -7,7 +7,8 @@
 // it evaluates the slopes of the top layers down to the first layer deeper than the eddy
 // displacement and of the bottom layers up to the first one higher than it above the bottom, and
 // stops there, as the reference's scans exit.  k_redigm_col then walks the layers, one thread a
-// column and segment of layers, with a one-layer window: vertical differences on the half levels
+// column and segment of layers (with few layers a thread scans and walks its whole column in one
+// launch), with a one-layer window: vertical differences on the half levels
 // (calc_GradTRC :412-424), the JM95 expansion coefficients and the slopes (calc_IsoNeutralSlope_new
 // :745-775), the taper (DM95 or GKW91 times LDD95), the Redi and skew fluxes of both tracers
 // on the layer and on the half level above it (calc_IsopycDiffFlux :497-553, calc_SkewFlux
@@ -188,78 +189,84 @@ __device__ inline void slopes_of(const RediArgs& a, const double* rfdk, int k, c
   layer_slopes(a, rfdk, k, tm, tc, tp, sm, sc, sp, f.z, L);
 }
 
-// The LDD95 scans (TaperingFunc_LDD95 :392-428), each stopping at its first hit: blockIdx.y = 0
-// from the surface (depth tmps, layer ks), 1 from the bottom (tmpb, kb).  The pair (depth, layer)
-// goes to the first layer of each segment of the walk, where the segment's own thread reads it
-// before it stores its fluxes there: temperature and salinity planes of flon (surface) or flat
-// (bottom).
+// One LDD95 scan of a column (TaperingFunc_LDD95 :392-428), stopping at its first hit: from the
+// surface (DIR > 0) or from the bottom up.  depth, hit: the depth and layer found (0 and none).
+template <int DIR>
+__device__ __forceinline__ void redigm_scan(const RediArgs& a, const double* wfd, long q, unsigned qb, double& depth,
+                                            int& hit) {
+  const int km = a.km;
+  const double asn = a.lat_cs[a.J + q / a.I];
+  double disph = 2.0 / (a.two_omega * asn);
+  disph = fmin(fmax(15e3, disph), 100e3);
+  const double dzmax = a.smax * disph;
+  const int k0 = DIR > 0 ? 0 : km - 1;
+  const double topo = DIR > 0 ? 0.0 : a.topo[q];
+  depth = 0.0;
+  hit = DIR > 0 ? -1 : km;
+  Pre ring[SRING];
+#pragma unroll
+  for (int u = 0; u < SRING; u++)
+    if (u < km) fetch_layer(a, qb, k0 + DIR * u, DIR, ring[u]);
+  double xc = ld(a.pt + (long)k0 * a.ldg, qb), yc = ld(a.sa + (long)k0 * a.ldg, qb);
+  double xb = xc, yb = yc;  // the layer behind in the walk (k0 itself at the start)
+  double mx = 0.0;
+  bool done = false;
+  for (int i0 = 0; i0 < km && !done; i0 += SRING) {
+#pragma unroll
+    for (int u = 0; u < SRING; u++) {
+      const int i = i0 + u;
+      if (done || i >= km) continue;
+      const int k = k0 + DIR * i;
+      const Pre c = ring[u];
+      if (i + SRING < km) fetch_layer(a, qb, k + DIR * SRING, DIR, ring[u]);
+      const bool end = i + 1 == km;
+      const double xn = end ? xc : c.tn, yn = end ? yc : c.sn;
+      Lay L;
+      if (DIR > 0)
+        slopes_of(a, wfd, k, c, xb, xc, xn, yb, yc, yn, L);
+      else
+        slopes_of(a, wfd, k, c, xn, xc, xb, yn, yc, yb, L);
+      const double sab = sqrt(L.slon * L.slon + L.slat * L.slat);
+      if (sab > mx) mx = sab;
+      if (DIR > 0 ? (0.0 - c.z) > dzmax : (c.z - (-topo)) > dzmax) {
+        hit = k;
+        depth = fmin(mx, a.smax) * disph;
+        done = true;
+      }
+      xb = xc, yb = yc, xc = xn, yc = yn;
+    }
+  }
+}
+
+// Both scans, blockIdx.y = 0 from the surface, 1 from the bottom.  The pair (depth, layer) goes to
+// the first layer of each segment of the walk, where the segment's own thread reads it before it
+// stores its fluxes there: temperature and salinity planes of flon (surface) or flat (bottom).
 __global__ __launch_bounds__(256) void k_redigm_scan(RediArgs a) {
   __shared__ double wfd[REDI_LDS_LAYERS];
   for (int k = threadIdx.x; k < a.km; k += 256) wfd[k] = a.rfdk[k];
   __syncthreads();
   const long q = (long)blockIdx.x * 256 + threadIdx.x;
   if (q >= a.npts) return;
-  const int km = a.km;
   const unsigned qb = (unsigned)q * 8u;
-  const double asn = a.lat_cs[a.J + q / a.I];
-  double disph = 2.0 / (a.two_omega * asn);
-  disph = fmin(fmax(15e3, disph), 100e3);
-  const double dzmax = a.smax * disph;
-  auto scan = [&](auto DIR) {
-    constexpr int dir = decltype(DIR)::value;
-    const int k0 = dir > 0 ? 0 : km - 1;
-    const double topo = dir > 0 ? 0.0 : a.topo[q];
-    double depth = 0.0;
-    int hit = dir > 0 ? -1 : km;
-    Pre ring[SRING];
-#pragma unroll
-    for (int u = 0; u < SRING; u++)
-      if (u < km) fetch_layer(a, qb, k0 + dir * u, dir, ring[u]);
-    double xc = ld(a.pt + (long)k0 * a.ldg, qb), yc = ld(a.sa + (long)k0 * a.ldg, qb);
-    double xb = xc, yb = yc;  // the layer behind in the walk (k0 itself at the start)
-    double mx = 0.0;
-    bool done = false;
-    for (int i0 = 0; i0 < km && !done; i0 += SRING) {
-#pragma unroll
-      for (int u = 0; u < SRING; u++) {
-        const int i = i0 + u;
-        if (done || i >= km) continue;
-        const int k = k0 + dir * i;
-        const Pre c = ring[u];
-        if (i + SRING < km) fetch_layer(a, qb, k + dir * SRING, dir, ring[u]);
-        const bool end = i + 1 == km;
-        const double xn = end ? xc : c.tn, yn = end ? yc : c.sn;
-        Lay L;
-        if (dir > 0)
-          slopes_of(a, wfd, k, c, xb, xc, xn, yb, yc, yn, L);
-        else
-          slopes_of(a, wfd, k, c, xn, xc, xb, yn, yc, yb, L);
-        const double sab = sqrt(L.slon * L.slon + L.slat * L.slat);
-        if (sab > mx) mx = sab;
-        if (dir > 0 ? (0.0 - c.z) > dzmax : (c.z - (-topo)) > dzmax) {
-          hit = k;
-          depth = fmin(mx, a.smax) * disph;
-          done = true;
-        }
-        xb = xc, yb = yc, xc = xn, yc = yn;
-      }
-    }
-    double* o = dir > 0 ? a.flon : a.flat;
-    const long oS = (long)km * a.ldo;
-    for (int k = 0; k < km; k += a.seg) {
-      st(o + (long)k * a.ldo, qb, depth);
-      st(o + oS + (long)k * a.ldo, qb, (double)hit);
-    }
-  };
+  double depth;
+  int hit;
   if (blockIdx.y == 0)
-    scan(std::integral_constant<int, 1>{});
+    redigm_scan<1>(a, wfd, q, qb, depth, hit);
   else
-    scan(std::integral_constant<int, -1>{});
+    redigm_scan<-1>(a, wfd, q, qb, depth, hit);
+  double* o = blockIdx.y == 0 ? a.flon : a.flat;
+  const long oS = (long)a.km * a.ldo;
+  for (int k = 0; k < a.km; k += a.seg) {
+    st(o + (long)k * a.ldo, qb, depth);
+    st(o + oS + (long)k * a.ldo, qb, (double)hit);
+  }
 }
 
 // Segment blockIdx.y of the walk: layers k0 .. k1-1, with the layer above (its half-level terms)
-// and the layer below (the flux into the segment's last layer) computed again.
-__global__ __launch_bounds__(256, 3) void k_redigm_col(RediArgs a) {
+// and the layer below (the flux into the segment's last layer) computed again.  SCAN: the whole
+// column, after its own scans.
+template <bool SCAN>
+__global__ __launch_bounds__(256, SCAN ? 2 : 3) void k_redigm_col(RediArgs a) {
   // per layer k: m1 = cdk[k]/(cdk[k-1]+cdk[k]), m2 = cdk[k-1]/(cdk[k-1]+cdk[k]) (r_m1, r_m2 of
   // the half level on top of layer k, calc_IsopycDiffFlux :491-494) and z_RCDK = 1/cdk[k]
   // (DOGCM_Admin_Grid_mod.f90:315), each the same IEEE division as in the loop
@@ -285,8 +292,15 @@ __global__ __launch_bounds__(256, 3) void k_redigm_col(RediArgs a) {
   const double cs = a.lat_cs[q / a.I];
   const double topo = a.topo[q];
   const long oS = (long)km * a.ldo, o0 = (long)k0 * a.ldo;
-  const double tmps = ld(a.flon + o0, qb), tmpb = ld(a.flat + o0, qb);
-  const int ks = (int)ld(a.flon + oS + o0, qb), kb = (int)ld(a.flat + oS + o0, qb);
+  double tmps, tmpb;
+  int ks, kb;
+  if constexpr (SCAN) {
+    redigm_scan<1>(a, wfd, q, qb, tmps, ks);
+    redigm_scan<-1>(a, wfd, q, qb, tmpb, kb);
+  } else {
+    tmps = ld(a.flon + o0, qb), tmpb = ld(a.flat + o0, qb);
+    ks = (int)ld(a.flon + oS + o0, qb), kb = (int)ld(a.flat + oS + o0, qb);
+  }
   const double kr = a.kr, kg = a.kg;
   Lay P;                         // layer k-1
   double rPh = 0.0;              // 1 / P.h
@@ -397,14 +411,25 @@ int launch_redigm_col(const dsht_plan* p, const RediParams& c, const double* pt,
   a.two_omega = 2.0 * c.omega;
   const double bytes = (14.0 * km + 1.0) * (double)a.npts * 8.0;
   ProfScope prof("redigm_col", s, bytes, 0.0);
-  // Segments: at least 5120 waves (3 a SIMD on 1024 SIMDs run at once) of 3 layers or
-  // more.  Whole column (one segment) against this rule: 512 x 256 x 60 (3 segments) 229 and
+  const unsigned nb = (unsigned)((a.npts + 255) / 256);
+  // One launch, a thread a whole column, where segments give little or nothing: few layers (a second
+  // launch and the halo layers cost more: 64 x 32 x 2 8.4 and 9.2 us, 512 x 256 x 5 26 and 34), more
+  // of them on grids that give every SIMD one wave (400 x 200 x 12 43 and 45 us, x 24 69 and 64;
+  // 384 x 192 x 14 45 and 45) or one and a half (512 x 256 x 10 41 and 51 us, x 20 73 and 83;
+  // 540 x 270 x 24 109 and 106)
+  if (km <= (a.npts < 65536 ? 9 : a.npts < 98304 ? 14 : 20)) {
+    a.seg = km;
+    hipLaunchKernelGGL(k_redigm_col<true>, dim3(nb), dim3(256), 0, s, a);
+    DSHT_HIP(hipGetLastError());
+    return 0;
+  }
+  // Segments: at least 5120 waves (3 a SIMD on 1024 SIMDs run at once), of at least 2 layers but for
+  // the last.  Whole column (one segment) against this rule: 512 x 256 x 60 (3 segments) 229 and
   // 227 us, 256 x 128 x 60 (10) 133 and 76 us, 128 x 64 x 20 (7) 49 and 25 us
   const long nseg = std::max(1l, std::min((5120l * 64 + a.npts - 1) / a.npts, (km + 2l) / 3));
   a.seg = (int)((km + nseg - 1) / nseg);
-  const unsigned nb = (unsigned)((a.npts + 255) / 256);
   hipLaunchKernelGGL(k_redigm_scan, dim3(nb, 2), dim3(256), 0, s, a);
-  hipLaunchKernelGGL(k_redigm_col, dim3(nb, (unsigned)((km + a.seg - 1) / a.seg)), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(k_redigm_col<false>, dim3(nb, (unsigned)((km + a.seg - 1) / a.seg)), dim3(256), 0, s, a);
   DSHT_HIP(hipGetLastError());
   return 0;
 }
