@@ -19,6 +19,8 @@
 // CPU evaluation of the reference loops bit for bit.  The kernels are bound by HBM: each
 // input and output value is touched once, through non-temporal loads and stores (with
 // cached access they ran at 5.2 TB/s on T170L60 grids, non-temporal at 5.8-6.0 TB/s).
+#include <type_traits>
+
 #include "dsht_internal.hpp"
 
 namespace dsht {
@@ -257,11 +259,14 @@ __global__ __launch_bounds__(256) void k_col_quick(const double* __restrict__ om
 // MOM selects calc_VDiffMOMEq (:865-975): right-hand side dt rhs[k] (no division by e3) and,
 // for a Dirichlet bottom, Ad = 1 + alpha coef (bfric + r[km-1]) with the bottom friction
 // coefficient bfric of the grid point (:963).
+// WL: the half levels' weights, the same for every column, in LDS (from 10 layers on: 256 x 128 x
+// 20 22.4 us without, 21.3 with; below, the barrier before the first row costs more than the
+// divisions: 64 x 32 x 2 2.85 and 3.05 us, x 5 5.3 and 5.5, x 10 9.0 both).
 struct VdiffRow {
   double al, ad, au, b;
 };
 
-template <bool MOM, bool MASK, int RR, int LR>
+template <bool MOM, bool MASK, int RR, int LR, bool WL = MASK>
 __global__ __launch_bounds__(256) void k_col_vdiff(const double* __restrict__ q0, const double* __restrict__ rhs,
                                                    const double* __restrict__ kv, const double* __restrict__ e3,
                                                    long ldg, int km, const double* __restrict__ cdk,
@@ -274,8 +279,8 @@ __global__ __launch_bounds__(256) void k_col_vdiff(const double* __restrict__ q0
   constexpr bool REC = MASK && RR > 0;
   constexpr int RC = REC ? 64 - 2 - RR - LR : 1;  // most rows to compute again
   static_assert(!REC || RC > 0, "rows left over");
-  __shared__ double sm1[MASK ? 65 : 1], sm2[MASK ? 65 : 1];
-  if constexpr (MASK) {  // the half levels' weights, the same for every column
+  __shared__ double sm1[WL ? 65 : 1], sm2[WL ? 65 : 1];
+  if constexpr (WL) {
     for (int h = 1 + threadIdx.x; h < km; h += 256) {
       const double s = cdk[h - 1] + cdk[h];
       sm1[h] = cdk[h] / s;
@@ -296,7 +301,7 @@ __global__ __launch_bounds__(256) void k_col_vdiff(const double* __restrict__ q0
   // half-level coefficient r[h] from the layers above (h-1) and below (h)
   auto rhalf = [&](int h, double kva, double e3a, double kvb, double e3b) {
     double m1, m2;
-    if constexpr (MASK) {
+    if constexpr (WL) {
       m1 = sm1[h], m2 = sm2[h];
     } else {
       const double s = cdk[h - 1] + cdk[h];
@@ -632,10 +637,13 @@ int launch_col_vdiff(const double* q0, const double* rhs, const double* kv, cons
   // the last finished rows stay in registers (32 with the interchange mask, 24 without) and
   // the VDIFF_LR before them in LDS when the column is long enough for the register rows
   constexpr int RM = 32, RN = 24;
-  auto k = bfric ? (km <= 64 ? (km >= RM + 2 ? k_col_vdiff<true, true, RM, VDIFF_LR> : k_col_vdiff<true, true, 0, 0>)
-                             : k_col_vdiff<true, false, RN, VDIFF_LR>)
-                 : (km <= 64 ? (km >= RM + 2 ? k_col_vdiff<false, true, RM, VDIFF_LR> : k_col_vdiff<false, true, 0, 0>)
-                             : k_col_vdiff<false, false, RN, VDIFF_LR>);
+  auto pick = [km](auto MOM) {
+    constexpr bool mom = decltype(MOM)::value;
+    if (km < 10) return k_col_vdiff<mom, true, 0, 0, false>;
+    if (km < RM + 2) return k_col_vdiff<mom, true, 0, 0>;
+    return km <= 64 ? k_col_vdiff<mom, true, RM, VDIFF_LR> : k_col_vdiff<mom, false, RN, VDIFF_LR>;
+  };
+  auto k = bfric ? pick(std::true_type{}) : pick(std::false_type{});
   hipLaunchKernelGGL(k, dim3(col_grid(npts)), dim3(256), 0, s, q0, rhs, kv, e3, ldg, km, cdk, fdk, dt, alpha,
                      sfc_dirichlet, btm_dirichlet, bfric, qa, ldo, work, npts);
   DSHT_HIP(hipGetLastError());
