@@ -344,7 +344,10 @@ int dsht_prof_query(const char* name, double* total_ms, long* count, double* byt
  * State in device memory (dsht_lfam3_state): U, V (km grids per run, run r layer k at grid
  * column r*km + k), tracers (potential temperature [K] then salinity per run: column
  * (2r + t)*km + k), surface pressure (one grid per run), at time levels B and N; a step
- * advances runs [0, nruns) and rotates the levels (B <- N, N <- A).  The vertical grid is
+ * advances runs [0, nruns) and rotates the levels (B <- N, N <- A).  A step checks its
+ * arguments and takes its scratch before it writes level B or N; one that then returns an error
+ * of the device leaves them undefined (those of momentum and pressure move before the tracers
+ * are computed).  The vertical grid is
  * the Chebyshev-Lobatto one of dsht_sig_grid(km, km, -1, 0) (km even).  A step allocates
  * nothing itself; the plan's transform workspaces are sized by the first step on a stream.
  * Runs are independent: a run's result does not depend on the other runs in the pool.      */
