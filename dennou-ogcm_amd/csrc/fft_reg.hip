@@ -501,7 +501,7 @@ template <int MODE>
 using EpiArg = std::conditional_t<(MODE >= 4), InvEpi, NoEpi>;
 
 // MODE 0: the field; 1: its longitude derivative (transform i m X_m, times a.rowscale);
-// 2 (dual): both from one read of the coefficients -- the field into xy, then the
+// 2 (dual, FP32 coefficients): both from one read of the coefficients -- the field into xy, then the
 // derivative, times a.rowscale, into a.xy2 -- the coefficients stay in registers between the
 // two passes; 3: fields of one launch (grid y) of either kind, bit y of a.deriv set for the
 // derivative of field y; 4, 5, 6 (FP64): the field with the epilogue E_RHS, E_PRED, E_TRC, whose
@@ -715,8 +715,10 @@ static int reg_inv_mode(const GT* G, const FftArgs& a, XT* xy, hipStream_t s) {
 
 template <int R1, int R2, int NT, typename GT, typename V, typename XT>
 static int reg_inv_nt(const GT* G, const FftArgs& a, XT* xy, hipStream_t s) {
-  if (a.xy2) return reg_inv_mode<R1, R2, NT, GT, V, 2, XT>(G, a, xy, s);
-  if constexpr (sizeof(GT) == 16) {
+  if constexpr (sizeof(GT) == 8) {
+    if (a.xy2) return reg_inv_mode<R1, R2, NT, GT, V, 2, XT>(G, a, xy, s);
+  } else {
+    if (a.xy2) return fail(DSHT_EUNSUPPORTED, "dual inverse FFT: FP32 coefficients only");
     if (a.deriv && a.nf > 1) return reg_inv_mode<R1, R2, NT, GT, V, 3, XT>(G, a, xy, s);
     if constexpr (sizeof(XT) == 8) {
       switch (a.epi ? a.epi->kind : E_NONE) {
