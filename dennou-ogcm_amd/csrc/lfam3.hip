@@ -705,7 +705,7 @@ struct dsht_lfam3 {
   std::vector<double> cdk, fdk, rcdk, rfdk, zck;
   std::vector<double*> allocs;
   // constants
-  double *d_cdk = nullptr, *d_fdk = nullptr, *d_rcdk = nullptr, *d_rfdk = nullptr, *d_zck = nullptr;
+  double *d_cdk = nullptr, *d_rcdk = nullptr, *d_rfdk = nullptr, *d_zck = nullptr;
   double *d_mu = nullptr, *d_cs = nullptr, *d_two_omega = nullptr;
   double *d_m1 = nullptr, *d_m2 = nullptr, *d_dfac = nullptr;  // QUICK weights per half level
   double *d_dmom = nullptr, *d_dtrc = nullptr, *d_advf = nullptr, *d_nn1 = nullptr, *d_nn1p = nullptr, *d_hcoef = nullptr,
@@ -713,10 +713,13 @@ struct dsht_lfam3 {
   // state: levels B (0), N (1), A (2)
   double *U[3] = {}, *V[3] = {}, *TS[3] = {}, *SP[3] = {};
   // work
-  double *ucos = nullptr, *vcos = nullptr, *VD = nullptr, *Dens = nullptr, *Hyd = nullptr;
+  double *VD = nullptr, *Dens = nullptr, *Hyd = nullptr;
   double *Geo = nullptr, *GLon = nullptr, *GLat = nullptr, *Am = nullptr, *Bg = nullptr, *Cg = nullptr;
   double *URHS = nullptr, *VRHS = nullptr, *Upr = nullptr, *Vpr = nullptr;
-  double *TSpr = nullptr, *HT = nullptr, *FU = nullptr, *FV = nullptr, *VF = nullptr;
+  // FU, FV: the tracers' horizontal fluxes, dead once transformed; the tracers' tendency grids (HT)
+  // and the winds times cos(lat) (ucos, vcos) of the forms that need those share their memory
+  double *TSpr = nullptr, *FU = nullptr, *FV = nullptr, *VF = nullptr;
+  double *HT = nullptr, *ucos = nullptr, *vcos = nullptr;
   double* b2[16] = {};  // 2-D barotropic work, one grid per run each
   double *wVD = nullptr, *wGeo = nullptr, *wC = nullptr, *w1 = nullptr, *w2 = nullptr;
   double *wB = nullptr, *wC2 = nullptr, *wDSP = nullptr, *wDDiv = nullptr, *wZero = nullptr;
@@ -1063,7 +1066,6 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
     if (!rc) rc = lf_upload(s, d, v);
   };
   U(&s->d_cdk, s->cdk);
-  U(&s->d_fdk, s->fdk);
   U(&s->d_rcdk, s->rcdk);
   U(&s->d_rfdk, s->rfdk);
   U(&s->d_zck, s->zck);
@@ -1086,8 +1088,6 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
     A(&s->TS[lv], 2 * NC * np);
     A(&s->SP[lv], R * np);
   }
-  A(&s->ucos, NC * np);
-  A(&s->vcos, NC * np);
   A(&s->VD, 2 * NC * np);
   A(&s->Dens, NC * np);
   A(&s->Hyd, NC * np);
@@ -1102,10 +1102,11 @@ int dsht_lfam3_create(dsht_plan* p, const dsht_lfam3_config* cfg, dsht_lfam3** o
   A(&s->Upr, NC * np);
   A(&s->Vpr, NC * np);
   A(&s->TSpr, 2 * NC * np);
-  A(&s->HT, 2 * NC * np);
   A(&s->FU, 2 * NC * np);
   A(&s->FV, 2 * NC * np);
   A(&s->VF, 2 * NC * np);
+  s->HT = s->ucos = s->FU;
+  s->vcos = s->FV;
   for (auto& b : s->b2) A(&b, R * np);
   A(&s->wVD, (size_t)L * 2 * NC);
   A(&s->wGeo, (size_t)L * NC);
