@@ -20,8 +20,9 @@ the seeded initial state) and may leave one when it finishes (`save_to`), in dog
 layout (dsht/restart.py; DOGCM_IO_Restart_mod.f90), so a served run can be stopped and resumed
 later, in another pool or process.
 
-A step makes (42 KM + 9) forward and (28 KM + 9) inverse transform units per run
-(dsht_lfam3_units); pairs/s = units / 2 / s.
+The reference's step makes (42 KM + 9) forward and (28 KM + 9) inverse transform units per run
+(dsht_lfam3_units); pairs/s = units / 2 / s counts those, though the device step leaves out the
+ones whose results it has or does not read.
 """
 import time
 
@@ -119,7 +120,7 @@ class Pool:
         self.plan, self.nmax, self.km, self.cap = plan, plan.nmax, km, capacity
         self.max_runs = capacity  # latency cap on the active runs (set by calibrate)
         self.lf = LfAm3(plan, lfam3_config(km=km, max_runs=capacity, dt=dt, **(cfg_kw or {})))
-        # state, constants and work of one slot: about 41 grids per layer plus spectra
+        # state, work and transform scratch of one slot: at most 41 grids per layer plus spectra
         self.bytes_per_run = 8 * (41 * km * plan.im * plan.jm + 12 * km * plan.lm)
         self.runs = []
         self.t_ref = None
