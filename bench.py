@@ -327,11 +327,11 @@ def roofline_probe(torch, plan, dsht, form, scope, bufs, reps=10):
     else:
         roof = {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS}
     roof["traffic"] = traffic_table().get((form, scope))
-    # FFT launches per call of the fused inverse: three in FP64 (one per output grid), two in
-    # the split forms (the field with its longitude derivative from one read, the latitude
-    # derivative); launch-average bytes and times cover both kinds
-    per_call = (3 if form == "fp64" else 2) if scope == "fft_inv" else 1
-    roof.update({"kernel": scope, "columns_per_launch": nc * reps * per_call / cnt, "avg_launch_us": 1e6 * t,
+    # FFT passes over the columns per call of the fused inverse: three in FP64 (one per output grid,
+    # in one launch), two in the split forms (a launch for the field with its longitude derivative
+    # from one read, one for the latitude derivative); launch-average bytes and times cover all
+    passes = (3 if form == "fp64" else 2) if scope == "fft_inv" else 1
+    roof.update({"kernel": scope, "columns_per_launch": nc * reps * passes / cnt, "avg_launch_us": 1e6 * t,
                  "algorithmic_bytes_per_launch": by / cnt, "algorithmic_flops_per_launch": fl / cnt,
                  "traffic_source": "profiles/hbm_traffic_T170L60.md" if roof["traffic"] else None})
     return roof
@@ -529,8 +529,9 @@ def column_bench(torch, dsht, reps=21, nsets=3):
 def lfam3_bench(torch, dsht, steps=20, N=NMAX, km=KM):
     """The device LF-AM3 dynamics step at T170L60 (I=512, J=256): one run, and four runs of
     the same truncation in one pool (each transform over all their layers in one call).
-    One step = (42 KM + 9) forward + (28 KM + 9) inverse units per run, the reference's count: the
-    library leaves out those whose results the step has or does not read."""
+    pairs_per_s counts the reference's (42 KM + 9) forward + (28 KM + 9) inverse units per run and
+    step; made_pairs_per_s the 27 KM + 5 grids that the FP64 form transforms forward and the
+    15 KM + 5 inverse (it leaves out those whose results the step has or does not read)."""
     from dsht import serve
 
     out = {"workload": f"LF-AM3 dynamics step (rigid lid, linear EOS), T{N}L{km} (I={IM}, J={JM}), FP64, "
@@ -556,8 +557,9 @@ def lfam3_bench(torch, dsht, steps=20, N=NMAX, km=KM):
         ms = e0.elapsed_time(e1) / steps
         f, i = pool.lf.units(nr)
         ok = bool(torch.isfinite(pool.lf.state(dsht.LF_U, dsht.LF_N)[:nr * km]).all())
+        made = (42 * km + 10) * nr / 2
         out[f"runs_{nr}"] = {"ms_per_step": ms, "pairs_per_s": (f + i) / 2 / (ms * 1e-3), "pairs_per_step": (f + i) / 2,
-                             "finite": ok}
+                             "made_pairs_per_s": made / (ms * 1e-3), "made_pairs_per_step": made, "finite": ok}
         pool = None
     return out
 
@@ -742,8 +744,9 @@ def serving_bench(torch, dsht, n_req=32, rate=20.0, nsteps=200, seed=0x5E4E, fac
     b, u = res["batched"], res["one_at_a_time"]
     return {
         "workload": f"{n_req} LF-AM3 runs, Poisson arrivals at {rate:g}/s, {nsteps} steps each, truncation from "
-                    f"{list(serve.GRIDS)}, KM from [20, 30, 60], rotation 0.25-4x Earth; FP64; one step = "
-                    f"(42 KM + 9) forward + (28 KM + 9) inverse units per run",
+                    f"{list(serve.GRIDS)}, KM from [20, 30, 60], rotation 0.25-4x Earth; FP64; pairs/s count the "
+                    f"reference's (42 KM + 9) forward + (28 KM + 9) inverse units per run and step, of which the "
+                    f"device step makes 27 KM + 5 and 15 KM + 5",
         "batched": b,
         "batched_concurrent": res["batched_concurrent"],
         "batched_uncapped": res["batched_uncapped"],

@@ -364,8 +364,8 @@ __global__ __launch_bounds__(256) void k_col_vdiff(const double* __restrict__ q0
   double dl = r1.al, dn = r1.ad, dun = r1.au, bn = r1.b;
   // RR > 0: the finished rows of the last RR steps before the final one (j = J1 .. km-3) stay
   // in registers (d, du, b); the LR rows before them (j = J0 .. J1-1) in LDS, row-major over
-  // the block's threads; only the rows above J0 make the workspace round trip.  The rare
-  // second superdiagonal of an interchange goes to the workspace in every tier.
+  // the block's threads; the rows above J0 are eliminated again (REC) or make the workspace round
+  // trip.  The rare second superdiagonal of an interchange goes to the workspace in every tier.
   const int J1 = km - 2 - RR;
   const int J0 = J1 - LR > 0 ? J1 - LR : 0;
   double rd[RR > 0 ? RR : 1], ru[RR > 0 ? RR : 1], rb[RR > 0 ? RR : 1];

@@ -560,7 +560,8 @@ __global__ __launch_bounds__(NT, WPE<V>) void k_fft_inv_r(const GT* __restrict__
   // below two thirds of M, all that an alias-free grid's truncation has, where the kernel runs
   // two waves per SIMD either way and the registers are free (M = 192 and 256; 120 fields of
   // 512 x 256: 45.6 -> 42.4 us).  Not at M = 128 (50 -> 56 us: a wave per SIMD less) and not with
-  // the per-field derivative, whose several fields a launch already overlap (258 -> 256..260 us)
+  // the per-field derivative, whose several fields a launch already overlap (258 -> 256..260 us);
+  // M = 135 and 270 were not measured
   constexpr int PF = sizeof(GT) == 8 && M <= 256 ? NL
                      : sizeof(GT) == 16 && (M == 192 || M == 256) && MODE < 2
                          ? ((2 * M / 3 + 2) * ROWS + C::THREADS - 1) / C::THREADS

@@ -21,8 +21,8 @@
 // Bound: HBM and, close to it, the vector issue (about 410 instructions a layer, 285 of them FP64).
 // Algorithmic bytes per call: the 8 input layer fields (ptemp, salt, h, z, the four gradients)
 // and the 6 output layer fields once: (14 km + 1) I J 8 bytes; the scans reread a few layers.
-// 512 x 256 x 60: scan 46 us, walk 189 us (4.9 TB/s); both in one kernel of one thread a column
-// took 284 us.  What the difference was: the layer thicknesses' reciprocals were loaded from memory
+// 512 x 256 x 60: scan 46 us, walk 189 us (4.9 TB/s); an earlier kernel of one thread a column took
+// 284 us.  What the difference was: the layer thicknesses' reciprocals were loaded from memory
 // behind the next layer's loads, and so waited for them (rfdk is in LDS now); 13 full divisions a
 // layer (now 4 reciprocals and corrected quotients); tanh (now one exp); 208 registers.
 
@@ -423,7 +423,7 @@ int launch_redigm_col(const dsht_plan* p, const RediParams& c, const double* pt,
     DSHT_HIP(hipGetLastError());
     return 0;
   }
-  // Segments: at least 5120 waves (3 a SIMD on 1024 SIMDs run at once), of at least 2 layers but for
+  // Segments: at least 5120 waves (3 a SIMD on 1024 SIMDs run at once) of 3 layers or more but for
   // the last.  Whole column (one segment) against this rule: 512 x 256 x 60 (3 segments) 229 and
   // 227 us, 256 x 128 x 60 (10) 133 and 76 us, 128 x 64 x 20 (7) 49 and 25 us
   const long nseg = std::max(1l, std::min((5120l * 64 + a.npts - 1) / a.npts, (km + 2l) / 3));
