@@ -7,11 +7,13 @@ pytestmark = pytest.mark.gpu
 
 
 def test_pool_memory(gpu):
+    import gc
     import torch
     import dsht
     N, I, J, km, runs = 42, 128, 64, 60, 8
     grid, spec = 8 * I * J, 8 * (N + 1) ** 2
     p = dsht.Plan(N, I, J, radius=6.371e6)
+    gc.collect()  # nothing of earlier tests is freed between the readings
     torch.cuda.synchronize()
     free = torch.cuda.mem_get_info(gpu)[0]
     pool = dsht.LfAm3(p, dsht.lfam3_config(km=km, max_runs=runs))

@@ -26,3 +26,25 @@ def test_columns_match_oracle(gpu, N, I, J, km, interior, tilt, shallow):
     ocfg, cfg = _cfg_pair(interior=interior)
     for name, g, ref in zip(("flx_lon", "flx_lat", "vdiv"), _device(p, x, gpu, cfg), _oracle(p, x, ocfg)):
         assert np.max(np.abs(g - ref)) < 1e-13 * np.max(np.abs(ref)), name
+
+
+@pytest.mark.parametrize("km", [2, 9, 10])
+def test_padded_layers(gpu, km):
+    """Layers of a larger pitch (and 8 bytes off a 16-byte boundary) give the same bits."""
+    import torch
+    import dsht
+    p = dsht.Plan(10, 32, 16, radius=R_EARTH)
+    x = {k: torch.tensor(np.ascontiguousarray(v), device=gpu) for k, v in _inputs(p, km, 5.0, True).items()}
+    pitch = p.im * p.jm + 7
+
+    def padded(t):
+        buf = torch.full((1 + t.shape[0] * pitch,), float("nan"), dtype=torch.float64, device=gpu)
+        v = torch.as_strided(buf, t.shape, (pitch, p.im, 1), 1)
+        v.copy_(t)
+        return v
+
+    def call(f):
+        return p.col_redigm_d(f(x["pt"]), f(x["sa"]), f(x["h"]), f(x["z"]), x["topo"], x["cdk"], x["rfdk"], f(x["gl"]),
+                              f(x["ga"]))
+    for a, b in zip(call(padded), call(lambda t: t)):
+        assert torch.equal(a, b)
