@@ -1401,7 +1401,7 @@ int dsht_col_redigm_d(dsht_plan* p, const dsht_redigm_config* cfg, const double*
       if (overlaps(outs[i], outs[k])) return fail(DSHT_EARG, "the outputs %s and %s overlap", onames[i], onames[k]);
   }
   return launch_redigm_col(p, r, ptemp, salt, h, z, ldg, km, topo, cdk, rfdk, grad_lon, grad_lat, ldg, flx_lon,
-                           flx_lat, vdiv, ldo, (hipStream_t)stream);
+                           flx_lat, vdiv, ldo, true, (hipStream_t)stream);
 }
 
 long dsht_redigm_work_size(const dsht_plan* p, int km) {
@@ -1454,7 +1454,7 @@ int dsht_redigm_d(dsht_plan* p, const dsht_redigm_config* cfg, const double* pte
   }
   if ((rc = dsht_inv_vgrad_d(p, w, n2, 1, nullptr, glon, glat, IJ, (int)n2, nullptr, s))) return rc;
   if ((rc = launch_redigm_col(p, r, ptemp, salt, h, z, ldg, km, topo, cdk, rfdk, glon, glat, IJ, flon, flat, vdv,
-                              IJ, s)))
+                              IJ, false, s)))
     return rc;
   // append_Redi_GM_RHS (:340-346): xy_w(w_AlphaOptr_xy(FLon cos, FLat cos)) into glon
   if ((rc = dsht_alpha_fwd_d(p, flon, flat, IJ, w, n2, 1, (int)n2, nullptr, s))) return rc;

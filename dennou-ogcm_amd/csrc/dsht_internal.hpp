@@ -343,7 +343,7 @@ struct RediParams {
 int launch_redigm_col(const dsht_plan* p, const RediParams& c, const double* pt, const double* sa, const double* h,
                       const double* z, long ldg, int km, const double* topo, const double* cdk, const double* rfdk,
                       const double* glon, const double* glat, long ldgr, double* flon, double* flat, double* vdiv,
-                      long ldo, hipStream_t s);
+                      long ldo, bool alone, hipStream_t s);  // alone: the call's only work
 int launch_redigm_rhs(const dsht_plan* p, double* rt, double* rs, long ldo, const double* hdiv, const double* vdiv,
                       long ldw, int km, hipStream_t s);
 int launch_spec_energy(const dsht_plan* p, int ens, const double* w, long sl, long sc, int ncols, double* nma,

@@ -190,19 +190,16 @@ __device__ inline void slopes_of(const RediArgs& a, const double* rfdk, int k, c
 }
 
 // One LDD95 scan of a column (TaperingFunc_LDD95 :392-428), stopping at its first hit: from the
-// surface (DIR > 0) or from the bottom up.  depth, hit: the depth and layer found (0 and none).
-template <int DIR>
-__device__ __forceinline__ void redigm_scan(const RediArgs& a, const double* wfd, long q, unsigned qb, double& depth,
-                                            int& hit) {
+// surface (DIR > 0) or from the bottom up.  found(depth, hit): the depth and layer (0 and none).
+template <int DIR, typename F>
+__device__ __forceinline__ void redigm_scan(const RediArgs& a, const double* wfd, long q, unsigned qb, double disph,
+                                            F found) {
   const int km = a.km;
-  const double asn = a.lat_cs[a.J + q / a.I];
-  double disph = 2.0 / (a.two_omega * asn);
-  disph = fmin(fmax(15e3, disph), 100e3);
   const double dzmax = a.smax * disph;
   const int k0 = DIR > 0 ? 0 : km - 1;
   const double topo = DIR > 0 ? 0.0 : a.topo[q];
-  depth = 0.0;
-  hit = DIR > 0 ? -1 : km;
+  double depth = 0.0;
+  int hit = DIR > 0 ? -1 : km;
   Pre ring[SRING];
 #pragma unroll
   for (int u = 0; u < SRING; u++)
@@ -236,6 +233,13 @@ __device__ __forceinline__ void redigm_scan(const RediArgs& a, const double* wfd
       xb = xc, yb = yc, xc = xn, yc = yn;
     }
   }
+  found(depth, hit);
+}
+
+// the eddy displacement at a point's latitude (TaperingFunc_LDD95 :392-396)
+__device__ __forceinline__ double eddy_displacement(const RediArgs& a, long q) {
+  const double asn = a.lat_cs[a.J + q / a.I];
+  return fmin(fmax(15e3, 2.0 / (a.two_omega * asn)), 100e3);
 }
 
 // Both scans, blockIdx.y = 0 from the surface, 1 from the bottom.  The pair (depth, layer) goes to
@@ -248,18 +252,20 @@ __global__ __launch_bounds__(256) void k_redigm_scan(RediArgs a) {
   const long q = (long)blockIdx.x * 256 + threadIdx.x;
   if (q >= a.npts) return;
   const unsigned qb = (unsigned)q * 8u;
-  double depth;
-  int hit;
+  const double disph = eddy_displacement(a, q);
+  auto keep = [&](double* o) {
+    return [=](double depth, int hit) {
+      const long oS = (long)a.km * a.ldo;
+      for (int k = 0; k < a.km; k += a.seg) {
+        st(o + (long)k * a.ldo, qb, depth);
+        st(o + oS + (long)k * a.ldo, qb, (double)hit);
+      }
+    };
+  };
   if (blockIdx.y == 0)
-    redigm_scan<1>(a, wfd, q, qb, depth, hit);
+    redigm_scan<1>(a, wfd, q, qb, disph, keep(a.flon));
   else
-    redigm_scan<-1>(a, wfd, q, qb, depth, hit);
-  double* o = blockIdx.y == 0 ? a.flon : a.flat;
-  const long oS = (long)a.km * a.ldo;
-  for (int k = 0; k < a.km; k += a.seg) {
-    st(o + (long)k * a.ldo, qb, depth);
-    st(o + oS + (long)k * a.ldo, qb, (double)hit);
-  }
+    redigm_scan<-1>(a, wfd, q, qb, disph, keep(a.flat));
 }
 
 // Segment blockIdx.y of the walk: layers k0 .. k1-1, with the layer above (its half-level terms)
@@ -295,8 +301,9 @@ __global__ __launch_bounds__(256, SCAN ? 2 : 3) void k_redigm_col(RediArgs a) {
   double tmps, tmpb;
   int ks, kb;
   if constexpr (SCAN) {
-    redigm_scan<1>(a, wfd, q, qb, tmps, ks);
-    redigm_scan<-1>(a, wfd, q, qb, tmpb, kb);
+    const double disph = eddy_displacement(a, q);
+    redigm_scan<1>(a, wfd, q, qb, disph, [&](double depth, int hit) { tmps = depth, ks = hit; });
+    redigm_scan<-1>(a, wfd, q, qb, disph, [&](double depth, int hit) { tmpb = depth, kb = hit; });
   } else {
     tmps = ld(a.flon + o0, qb), tmpb = ld(a.flat + o0, qb);
     ks = (int)ld(a.flon + oS + o0, qb), kb = (int)ld(a.flat + oS + o0, qb);
@@ -399,7 +406,7 @@ __global__ __launch_bounds__(256) void k_redigm_rhs(double* __restrict__ rt, dou
 int launch_redigm_col(const dsht_plan* p, const RediParams& c, const double* pt, const double* sa, const double* h,
                       const double* z, long ldg, int km, const double* topo, const double* cdk, const double* rfdk,
                       const double* glon, const double* glat, long ldgr, double* flon, double* flat, double* vdiv,
-                      long ldo, hipStream_t s) {
+                      long ldo, bool alone, hipStream_t s) {
   RediArgs a;
   a.pt = pt, a.sa = sa, a.h = h, a.z = z, a.topo = topo, a.cdk = cdk, a.rfdk = rfdk, a.glon = glon, a.glat = glat;
   a.lat_cs = p->d_lat_cs;
@@ -412,19 +419,20 @@ int launch_redigm_col(const dsht_plan* p, const RediParams& c, const double* pt,
   const double bytes = (14.0 * km + 1.0) * (double)a.npts * 8.0;
   ProfScope prof("redigm_col", s, bytes, 0.0);
   const unsigned nb = (unsigned)((a.npts + 255) / 256);
-  // One launch, a thread a whole column, where segments give little or nothing: few layers (a second
-  // launch and the halo layers cost more: 64 x 32 x 2 8.4 and 9.2 us, 512 x 256 x 5 26 and 34), more
-  // of them on grids that give every SIMD one wave (400 x 200 x 12 43 and 45 us, x 24 69 and 64;
-  // 384 x 192 x 14 45 and 45) or one and a half (512 x 256 x 10 41 and 51 us, x 20 73 and 83;
-  // 540 x 270 x 24 109 and 106)
-  if (km <= (a.npts < 65536 ? 9 : a.npts < 98304 ? 14 : 20)) {
+  // One launch, a thread a whole column, where segments give little or nothing: 2 and 3 layers (a
+  // second launch and the halo layers cost more: 64 x 32 x 2 8.4 and 9.2 us), more on grids that give
+  // every SIMD one wave (400 x 200 x 12 43 and 45 us, x 24 69 and 64; 384 x 192 x 14 45 and 45) or
+  // one and a half (512 x 256 x 10 41 and 51 us, x 20 73 and 83; 540 x 270 x 24 109 and 106).  A call
+  // of its own up to 9 layers on any grid, which waits for the host's launches (64 x 32 x 5 20.8 and
+  // 23.4 us a call, though 15.2 and 13.2 on the device; x 10 23.4 and 23.4)
+  if (km <= (a.npts < 65536 ? (alone ? 9 : 3) : a.npts < 98304 ? 14 : 20)) {
     a.seg = km;
     hipLaunchKernelGGL(k_redigm_col<true>, dim3(nb), dim3(256), 0, s, a);
     DSHT_HIP(hipGetLastError());
     return 0;
   }
-  // Segments: at least 5120 waves (3 a SIMD on 1024 SIMDs run at once) of 3 layers or more but for
-  // the last.  Whole column (one segment) against this rule: 512 x 256 x 60 (3 segments) 229 and
+  // Segments: at least 5120 waves (3 a SIMD on 1024 SIMDs run at once) of 3 layers or more (of 4
+  // layers 2) but for the last.  Whole column (one segment) against this rule: 512 x 256 x 60 (3 segments) 229 and
   // 227 us, 256 x 128 x 60 (10) 133 and 76 us, 128 x 64 x 20 (7) 49 and 25 us
   const long nseg = std::max(1l, std::min((5120l * 64 + a.npts - 1) / a.npts, (km + 2l) / 3));
   a.seg = (int)((km + nseg - 1) / nseg);

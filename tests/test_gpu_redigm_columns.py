@@ -1,6 +1,6 @@
 """The Redi/GM column part (csrc/redigm.hip) on both sides of the rule that gives a thread its whole
-column, scans and walk in one launch (up to 9 layers; up to 14 from 65536 points on, up to 20 from
-98304), or a segment of layers after a launch of the scans: layer counts and grids around each line,
+column, scans and walk in one launch (up to 9 layers, 3 within the whole tendency; up to 14 from
+65536 points on, up to 20 from 98304), or a segment of layers after a launch of the scans: layer counts and grids around each line,
 against the oracle, with tapers that reach over most layers and with scans that find nothing.
 
 Tolerance as the column part's elsewhere: 1e-13 of each output's largest value.
