@@ -432,8 +432,8 @@ int launch_redigm_col(const dsht_plan* p, const RediParams& c, const double* pt,
     return 0;
   }
   // Segments: at least 5120 waves (3 a SIMD on 1024 SIMDs run at once) of 3 layers or more (of 4
-  // layers 2) but for the last.  Whole column (one segment) against this rule: 512 x 256 x 60 (3 segments) 229 and
-  // 227 us, 256 x 128 x 60 (10) 133 and 76 us, 128 x 64 x 20 (7) 49 and 25 us
+  // layers 2) but for the last.  Whole column (one segment) against this rule: 512 x 256 x 60 (3
+  // segments) 229 and 227 us, 256 x 128 x 60 (10) 133 and 76 us, 128 x 64 x 20 (7) 49 and 25 us
   const long nseg = std::max(1l, std::min((5120l * 64 + a.npts - 1) / a.npts, (km + 2l) / 3));
   a.seg = (int)((km + nseg - 1) / nseg);
   hipLaunchKernelGGL(k_redigm_scan, dim3(nb, 2), dim3(256), 0, s, a);
